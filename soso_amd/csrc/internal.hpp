@@ -151,7 +151,7 @@ struct soso_hip {
     // the scratch pointers it was captured with, so a slot outgrown while any
     // graph exists is retired, not freed: retired buffers are freed once no
     // graph is left (graph_destroy) or with the handle.
-    static constexpr int N_SCRATCH = 17;
+    static constexpr int N_SCRATCH = 18;
     void *scratch[N_SCRATCH] = {};
     size_t scratch_cap[N_SCRATCH] = {};
     std::vector<void *> retired;
@@ -309,6 +309,10 @@ bool mfma_moe_scan_ok(size_t n, size_t top_k, size_t n_groups, uint8_t dt_gu, ui
 bool tiled_q4k_ok(uint8_t dtype, size_t rows, size_t cols);
 int launch_tile_q4k(soso_hip *h, const void *src_dev, void *dst_dev, size_t rows, size_t cols);
 int launch_mfma_matmul(soso_hip *h, const Weight &w, const float *x, size_t n, float *y);
+// (k_gemm.hip) -- several tokens per row on the f16 matrix cores: whether they
+// are the faster ones for a shape, and their launch (DECLINED: no scratch)
+bool gemm_wins(uint8_t dtype, size_t rows, size_t cols, size_t n);
+int launch_gemm(soso_hip *h, const Weight &w, const float *x, size_t n, float *y);
 size_t moe_max_items(const soso_hip *h, size_t slots, size_t n_groups);
 int launch_router_topk(soso_hip *h, const float *w_dev, const float *x_dev, size_t n, size_t hdim,
                        size_t n_exp, size_t top_k, int32_t *idx_dev, float *wgt_dev, float *logits_dev);

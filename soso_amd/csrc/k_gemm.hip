@@ -1,0 +1,1008 @@
+// k_gemm.hip -- products of several tokens per weight row (GpuDispatch::matmul,
+// crates/soso-llm-core/src/gpu.rs:443-455): Q4_K, Q6_K and Q8_0 rows against x
+// split into two f16 parts, on the f16 matrix cores.
+//
+// Arithmetic.  x is scaled by a power of two 2^s per token and 256-column
+// super-block (its largest element into [2^14, 2^15)) and written as hi + lo,
+// two f16 numbers whose sum is within 2^-23 of every element above 2^-17 of
+// the block's largest, and within 2^-40 of the largest below that (the integer
+// kernels' digits: within 2^-23 of the largest).  An element above 2^14 times
+// the third largest of its 128-column block's 8-column maxima (at most 16 can
+// be) is taken out, marked by a negative 2^-s, and its products are added at
+// the end with the weights dequantized exactly, so that it cannot push the rest
+// of its block below that floor.  Weights times the block scales are whole
+// numbers: Q4_K's sc q (up to 945) exact in f16, Q6_K's sc (q - 32) (up to
+// 4096) exact as two f16, Q8_0's codes exact (its f32 scales are applied to the
+// block's sums).  Every product is exact in the f32 accumulators; a
+// super-block's sum S is one chain, and per super-block out += 2^-s d S in f32,
+// for Q4_K 2^-s (d S - dmin M) with M = sum m_j xsum_j over the eight
+// sub-blocks' f32 sums of x, split in two as x is.  Against 64 bits (normal x,
+// 4096 x 4096): 4.0e-7 (Q4_K), 1.8e-7 (Q6_K), 1.4e-7 (Q8_0) where the integer
+// digits gave 1.3e-6, 9.0e-7 and 5.4e-7.  A block that holds an Inf or a NaN
+// gets 2^-s = NaN: NaN products, as the CPU's dot gives Inf or NaN.
+//
+// v_mfma_f32_32x32x16_f16 operands (lane l: n = l % 32, f = l / 32):
+//   A (32 x 16): token n, k = 8 f .. 8 f + 7      <- LDS, x as staged below
+//   B (16 x 32): weight row n, the same k          <- registers, dequantized
+//   D (32 x 32): column n = weight row, register i = token 8 (i / 4) + 4 f + i % 4
+// A and B only have to agree on which element a (f, byte) slot of a step
+// holds, so the order is the weights'.  Q4_K and Q8_0: step t = 0..3 of a
+// 64-element unit takes its 32-element block t / 2, elements 16 f + 8 (t % 2) +
+// {0, 2, 1, 3, 4, 6, 5, 7} (the order in which masking a dword with 0x000F000F
+// yields byte pairs); Q6_K: quarter t of the unit's half, elements 16 k + 8 f +
+// the same eight (k: the unit's parity).
+#include "mv_core.hpp"
+
+#include <algorithm>
+
+typedef _Float16 gm_h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 gm_h8 __attribute__((ext_vector_type(8)));
+typedef float gm_f4 __attribute__((ext_vector_type(4)));
+typedef float gm_f16v __attribute__((ext_vector_type(16)));
+typedef uint32_t gm_u4 __attribute__((ext_vector_type(4))); // (a HIP uint4 array here ends up in scratch memory)
+
+// Staged x, for tiles of 32 tokens (rows past n are zeros):
+//   F [tile][unit][step 4][hi, lo][lane 64][16 B]   8 KiB per unit
+//   M [tile][super-block][lane 64][16 B]            eight sub-block sums, hi (f = 0) and lo (f = 1)
+//   P [tile][super-block][32] f32                   2^-s per token
+struct GmX {
+    const uint8_t *f, *m;
+    const float *p;
+};
+constexpr int GM_UNIT = 8192, GM_SUMS = 1024;
+
+__device__ __forceinline__ uint32_t gm_pack(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, gm_h2{(_Float16)a, (_Float16)b});
+}
+
+// Maximum over the 32 lanes of this lane's half wavefront.
+__device__ __forceinline__ float gm_half_max(float v)
+{
+    auto st = [](float a, uint32_t b) { return fmaxf(a, __uint_as_float(b)); };
+    v = st(v, dpp_keep<0xB1>(__float_as_uint(v)));
+    v = st(v, dpp_keep<0x4E>(__float_as_uint(v)));
+    v = st(v, dpp_keep<0x141>(__float_as_uint(v)));
+    v = st(v, dpp_keep<0x140>(__float_as_uint(v)));
+    v = st(v, dpp_keep<0x142, 0xA>(__float_as_uint(v)));
+    const int lo = __builtin_amdgcn_readlane(__float_as_int(v), 31), hi = __builtin_amdgcn_readlane(__float_as_int(v), 63);
+    return __int_as_float((threadIdx.x & 32) ? hi : lo);
+}
+__device__ __forceinline__ float gm_abs_max(gm_f4 v)
+{
+    return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+}
+// Above this an element of a 128-column block (32 lanes, four finite columns
+// each) is taken out: 2^14 times the third largest of the block's 16 maxima of
+// 8 columns.  Where that is zero no element needs the room.
+__device__ __forceinline__ float gm_outlier_thr(gm_f4 v)
+{
+    const int lane = threadIdx.x & 63;
+    float cm = gm_abs_max(v);
+    cm = fmaxf(cm, dpp_f<0xB1>(cm));
+    for (int r = 0; r < 2; r++) {
+        const uint64_t top = __ballot(cm == gm_half_max(cm));
+        const uint32_t mine = lane < 32 ? (uint32_t)top : (uint32_t)(top >> 32);
+        if (__builtin_ctz(mine) >> 1 == (lane & 31) >> 1) cm = -1.0f;
+    }
+    const float third = gm_half_max(cm);
+    return third > 0.0f ? 16384.0f * third : INFINITY;
+}
+
+// One token's 256 columns (four per lane) as a tile's row m: the fragments of
+// its four units at xf, the sub-blocks' sums at xm (Q4_K) and 2^-s.  c8, this
+// lane's group of eight columns, sits in unit u, step st, half f.
+template <int FMT>
+__device__ __forceinline__ void gm_stage_row(gm_f4 v, int lane, int m, uint8_t *xf, uint8_t *xm, float *xp)
+{
+    const int c8 = lane >> 1;
+    int u, st, f;
+    if constexpr (FMT == FMT_Q6K) {
+        u = 2 * (c8 >> 4) + ((c8 >> 1) & 1);
+        st = (c8 >> 2) & 3;
+        f = c8 & 1;
+    } else {
+        u = c8 >> 3;
+        st = 2 * ((c8 >> 2) & 1) + (c8 & 1);
+        f = (c8 >> 1) & 1;
+    }
+    uint8_t *dst = xf + u * GM_UNIT + st * 2048 + f * 512 + 8 * (lane & 1) + 16 * m;
+    float mx = gm_abs_max(v);
+    float sm = (v[0] + v[1]) + (v[2] + v[3]);
+    if (sm != sm) mx = INFINITY; // a NaN element (or Inf - Inf): the block is non-finite
+    // the maximum over the wavefront and the smallest maximum of its 32-column
+    // groups: within 2^14 of each other, no element is an outlier (the two
+    // largest 8-column maxima sit in at most two groups of each 128)
+    auto st_max = [](float a, uint32_t b) { return fmaxf(a, __uint_as_float(b)); };
+    auto st_min = [](float a, uint32_t b) { return fminf(a, __uint_as_float(b)); };
+    mx = st_max(mx, dpp_keep<0xB1>(__float_as_uint(mx)));
+    mx = st_max(mx, dpp_keep<0x4E>(__float_as_uint(mx)));
+    mx = st_max(mx, dpp_keep<0x141>(__float_as_uint(mx)));
+    float mn = st_min(mx, dpp_keep<0x140>(__float_as_uint(mx)));
+    mx = st_max(mx, dpp_keep<0x140>(__float_as_uint(mx)));
+    mn = st_min(mn, dpp_keep<0x142, 0xA>(__float_as_uint(mn)));
+    mx = st_max(mx, dpp_keep<0x142, 0xA>(__float_as_uint(mx)));
+    mn = st_min(mn, dpp_keep<0x143, 0xC>(__float_as_uint(mn)));
+    mx = st_max(mx, dpp_keep<0x143, 0xC>(__float_as_uint(mx)));
+    mn = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mn), 63));
+    mx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx), 63));
+    const bool finite = mx < INFINITY;
+    bool out = false;
+    if (__builtin_expect(finite && mx > 16384.0f * mn, 0)) { // uniform
+        const float thr = gm_outlier_thr(v);
+        bool mine = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (fabsf(v[i]) > thr) {
+                v[i] = 0.0f;
+                mine = true;
+            }
+        out = __ballot(mine) != 0;
+        mx = wave_max_dpp(gm_abs_max(v));
+        sm = (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    const int s = mx > 0.0f && finite ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
+    float e[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        e[i] = finite ? ldexpf(v[i], s) : 0.0f;
+        lo[i] = e[i] - (float)(_Float16)e[i];
+    }
+    *(uint2 *)dst = make_uint2(gm_pack(e[0], e[2]), gm_pack(e[1], e[3]));
+    *(uint2 *)(dst + 1024) = make_uint2(gm_pack(lo[0], lo[2]), gm_pack(lo[1], lo[3]));
+    if constexpr (FMT == FMT_Q4K) {
+        // the sub-block's sum (8 lanes), scaled by 2^(s - 5): at most 2^15
+        sm = seg_sum_dpp<8>(sm);
+        if ((lane & 7) == 0) {
+            const float q = finite ? ldexpf(sm, s - 5) : 0.0f;
+            const _Float16 hi = (_Float16)q;
+            _Float16 *d = (_Float16 *)xm + 8 * m + (lane >> 3);
+            d[0] = hi;
+            d[256] = (_Float16)(q - (float)hi);
+        }
+    }
+    if (lane == 0) *xp = !finite ? __builtin_nanf("") : out ? -ldexpf(1.0f, -s) : ldexpf(1.0f, -s);
+}
+
+// One workgroup per (32-token tile, super-block): eight wavefronts of four
+// tokens each; the fragments meet in LDS and leave as one contiguous 32 KiB.
+template <int FMT>
+__global__ void __launch_bounds__(512) k_gm_stage(const float *__restrict__ x, int n, int cols,
+                                                  uint8_t *__restrict__ xf, uint8_t *__restrict__ xm,
+                                                  float *__restrict__ xp)
+{
+    __shared__ uint4 frag[4 * GM_UNIT / 16];
+    __shared__ uint4 sums[GM_SUMS / 16];
+    const int nb = (cols + 255) >> 8, tile = (int)blockIdx.x / nb, sb = (int)blockIdx.x % nb;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool in = 256 * sb + 4 * lane < cols; // (a last super-block may be partial: zeros)
+    gm_f4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int t = 32 * tile + 4 * wave + k;
+        v[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
+        if (in && t < n) v[k] = *(const gm_f4 *)(x + (size_t)t * cols + 256 * sb + 4 * lane);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        gm_stage_row<FMT>(v[k], lane, 4 * wave + k, (uint8_t *)frag, (uint8_t *)sums,
+                          xp + (size_t)blockIdx.x * 32 + 4 * wave + k);
+    __syncthreads();
+    uint4 *of = (uint4 *)(xf + (size_t)blockIdx.x * (4 * GM_UNIT));
+#pragma unroll
+    for (int i = 0; i < 4; i++) of[i * 512 + threadIdx.x] = frag[i * 512 + threadIdx.x];
+    if (FMT == FMT_Q4K && threadIdx.x < 64)
+        ((uint4 *)(xm + (size_t)blockIdx.x * GM_SUMS))[threadIdx.x] = sums[threadIdx.x];
+}
+
+// (typedefs of the compiler's own vectors: a HIP uint4 array that a lambda
+// fills ends up in scratch memory)
+__device__ __forceinline__ gm_u4 gm_ld(rsrc_t r, uint32_t off)
+{
+    return __builtin_bit_cast(gm_u4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
+}
+__device__ __forceinline__ gm_h2 gm_h2_of(uint32_t v) { return __builtin_bit_cast(gm_h2, v); }
+__device__ __forceinline__ gm_h2 gm_dup(float v) { return gm_h2{(_Float16)v, (_Float16)v}; }
+
+// Bytes a and b of w as the f16 pair 1024 + byte (0x6400 | byte).
+template <int a, int b>
+__device__ __forceinline__ gm_h2 gm_bytes(uint32_t w)
+{
+    return gm_h2_of(__builtin_amdgcn_perm(0x64646464u, w, 0x04000400u | (uint32_t)a | ((uint32_t)b << 16)));
+}
+// The same byte b (0 .. 3, a constant after unrolling) twice.
+__device__ __forceinline__ gm_h2 gm_byte_dup(uint32_t w, int b)
+{
+    return gm_h2_of(__builtin_amdgcn_perm(0x64646464u, w, 0x04000400u | (uint32_t)b | ((uint32_t)b << 16)));
+}
+
+__device__ __forceinline__ gm_h8 gm_join(gm_h2 a, gm_h2 b, gm_h2 c, gm_h2 d)
+{
+    return gm_h8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+// gfx950's swap of a in lanes 32 .. 63 with b in lanes 0 .. 31.
+__device__ __forceinline__ void gm_swap32(uint32_t &a, uint32_t &b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void gm_swap32(gm_u4 &a, gm_u4 &b)
+{
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t x = a[i], y = b[i];
+        gm_swap32(x, y);
+        a[i] = x;
+        b[i] = y;
+    }
+}
+
+// The weights of a wavefront's 64 rows for half a super-block (units 2 i and 2
+// i + 1), format by format.  load: lane (n, k = lane / 32) requests, of rows n
+// and 32 + n, the 16 bytes of unit k in every plane, so that a row's bytes are
+// read 32 at a time; split: lane swaps (a plane or half index against the
+// lane's k) hand lane (n, f) what its operand takes of each unit; frag<>: the
+// operand of step t of unit v (0 or 1).  head_*: what a row holds once per
+// super-block, lane l requesting row l's.  SETS: halves in flight.
+template <int FMT, int SETS>
+struct GmW;
+
+template <int SETS>
+struct GmW<FMT_Q4K, SETS> {
+    static constexpr int PARTS = 1; // operands per step (hi, and lo where a weight needs two f16)
+    gm_u4 L[SETS][2][2], hn;
+    gm_u4 q[2][2]; // [rows 32 j][unit]: the 16 code bytes of plane f
+    uint32_t sc4[2][2], m4[2][2], dd[2];
+    uint32_t off_h, off_q, row32, plane;
+    __device__ __forceinline__ void init(int row, int lane, size_t stride, int U)
+    {
+        const int nb = U >> 2;
+        off_h = (uint32_t)((row + lane) * stride);
+        off_q = (uint32_t)((row + (lane & 31)) * stride) + 16u * (uint32_t)(nb + (lane >> 5));
+        row32 = (uint32_t)(32 * stride);
+        plane = 64u * (uint32_t)nb;
+    }
+    __device__ __forceinline__ void head_load(rsrc_t rs, int sb) { hn = gm_ld(rs, off_h + 16u * (uint32_t)sb); }
+    __device__ __forceinline__ void load(rsrc_t rs, int half, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                L[set][j][k] = gm_ld(rs, off_q + (uint32_t)j * row32 + (uint32_t)k * plane + 32u * (uint32_t)half);
+    }
+    // the scales of a super-block's eight sub-blocks (get_scale_min_k4,
+    // dequant.rs:150-159), four per dword
+    __device__ __forceinline__ void head()
+    {
+        gm_u4 h[2] = {hn, hn};
+        gm_swap32(h[0], h[1]);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            dd[j] = h[j][0];
+            sc4[j][0] = h[j][1] & 0x3F3F3F3Fu;
+            m4[j][0] = h[j][2] & 0x3F3F3F3Fu;
+            sc4[j][1] = (h[j][3] & 0x0F0F0F0Fu) | ((h[j][1] >> 2) & 0x30303030u);
+            m4[j][1] = ((h[j][3] >> 4) & 0x0F0F0F0Fu) | ((h[j][2] >> 2) & 0x30303030u);
+        }
+    }
+    __device__ __forceinline__ void split(int, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            q[j][0] = L[set][j][0];
+            q[j][1] = L[set][j][1];
+            gm_swap32(q[j][0], q[j][1]);
+        }
+    }
+    // Step t of unit v of half i.  A masked nibble q is the subnormal f16 q
+    // 2^-24 (16 q 2^-24 where the high nibbles stay in place) and its product
+    // with sc 2^10 (sc 2^6) is q sc 2^-14, exact: a dword costs one shift, four
+    // ands and four packed multiplies.
+    __device__ __forceinline__ void frag(int i, int v, int t, int j, gm_h8 (&b)[PARTS]) const
+    {
+        const int sub = 4 * i + 2 * v + (t >> 1);
+        const gm_h2 sc = (gm_byte_dup(sc4[j][sub >> 2], sub & 3) - gm_dup(1024.0f)) * gm_dup(t < 2 ? 1024.0f : 64.0f);
+        const uint32_t mask = t < 2 ? 0x000F000Fu : 0x00F000F0u;
+        const uint32_t w0 = q[j][v][2 * (t & 1)], w1 = q[j][v][2 * (t & 1) + 1];
+        b[0] = gm_join(gm_h2_of(w0 & mask) * sc, gm_h2_of((w0 >> 8) & mask) * sc, gm_h2_of(w1 & mask) * sc,
+                       gm_h2_of((w1 >> 8) & mask) * sc);
+    }
+    __device__ __forceinline__ float scale(int j) const { return 16384.0f * half_bits_to_f32(dd[j] & 0xffffu); }
+    __device__ __forceinline__ float min_scale(int j) const { return -32.0f * half_bits_to_f32(dd[j] >> 16); }
+    __device__ __forceinline__ gm_h8 mins(int j) const
+    {
+        const gm_h2 k = gm_dup(1024.0f);
+        return gm_join(gm_bytes<0, 1>(m4[j][0]) - k, gm_bytes<2, 3>(m4[j][0]) - k, gm_bytes<0, 1>(m4[j][1]) - k,
+                       gm_bytes<2, 3>(m4[j][1]) - k);
+    }
+};
+
+template <int SETS>
+struct GmW<FMT_Q6K, SETS> {
+    static constexpr int PARTS = 2;
+    gm_u4 L[SETS][2][3], hn;
+    uint32_t dn;
+    uint32_t q[2][3][2][2]; // [rows][QH, QLa, QLb][unit][dword]: bytes 8 f .. 8 f + 7
+    uint32_t sc4[2][4], dd[2]; // scales + 128
+    uint32_t off_h, off_d, off_q, row32, plane;
+    __device__ __forceinline__ void init(int row, int lane, size_t stride, int U)
+    {
+        const int nb = U >> 2;
+        off_h = (uint32_t)((row + lane) * stride);
+        off_d = off_h + 208u * (uint32_t)nb;
+        off_q = (uint32_t)((row + (lane & 31)) * stride) + 16u * (uint32_t)(nb + (lane >> 5));
+        row32 = (uint32_t)(32 * stride);
+        plane = 64u * (uint32_t)nb;
+    }
+    __device__ __forceinline__ void head_load(rsrc_t rs, int sb)
+    {
+        hn = gm_ld(rs, off_h + 16u * (uint32_t)sb);
+        dn = bld2(rs, off_d + 2u * (uint32_t)sb);
+    }
+    __device__ __forceinline__ void load(rsrc_t rs, int half, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                L[set][j][k] = gm_ld(rs, off_q + (uint32_t)j * row32 + (uint32_t)k * plane + 32u * (uint32_t)half);
+    }
+    __device__ __forceinline__ void head()
+    {
+        gm_u4 h[2] = {hn, hn};
+        gm_swap32(h[0], h[1]);
+        dd[0] = dd[1] = dn;
+        gm_swap32(dd[0], dd[1]);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) sc4[j][k] = h[j][k] ^ 0x80808080u;
+    }
+    __device__ __forceinline__ void split(int, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+#pragma unroll
+                for (int w = 0; w < 2; w++) {
+                    q[j][k][0][w] = L[set][j][k][w];
+                    q[j][k][1][w] = L[set][j][k][2 + w];
+                    gm_swap32(q[j][k][0][w], q[j][k][1][w]);
+                }
+    }
+    // Step t: quarter t of the half.  sc (q - 32) is a whole number up to
+    // 4096: its f16 rounding and the remainder (at most 1) are both exact.
+    __device__ __forceinline__ void frag(int i, int v, int t, int j, gm_h8 (&b)[PARTS]) const
+    {
+        const int s = 8 * i + v + 2 * t;
+        const gm_h2 sc = gm_byte_dup(sc4[j][s >> 2], s & 3) - gm_dup(1152.0f);
+        gm_h2 hi[4], lo[4];
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            const uint32_t l = q[j][1 + (t & 1)][v][w], hq = q[j][0][v][w];
+            const uint32_t c = ((t < 2 ? l : l >> 4) & 0x0F0F0F0Fu) |
+                               (t == 0 ? (hq << 4) & 0x30303030u
+                                : t == 1 ? (hq << 2) & 0x30303030u
+                                : t == 2 ? hq & 0x30303030u
+                                         : (hq >> 2) & 0x30303030u);
+            const gm_h2 a = gm_bytes<0, 2>(c) - gm_dup(1056.0f), d = gm_bytes<1, 3>(c) - gm_dup(1056.0f);
+            hi[2 * w] = a * sc;
+            hi[2 * w + 1] = d * sc;
+            lo[2 * w] = __builtin_elementwise_fma(a, sc, -hi[2 * w]);
+            lo[2 * w + 1] = __builtin_elementwise_fma(d, sc, -hi[2 * w + 1]);
+        }
+        b[0] = gm_join(hi[0], hi[1], hi[2], hi[3]);
+        b[1] = gm_join(lo[0], lo[1], lo[2], lo[3]);
+    }
+    __device__ __forceinline__ float scale(int j) const { return half_bits_to_f32(dd[j] & 0xffffu); }
+};
+
+template <int SETS>
+struct GmW<FMT_Q80, SETS> {
+    static constexpr int PARTS = 1;
+    gm_u4 L[SETS][2][4], hs[SETS];
+    gm_u4 q[2][2][2]; // [rows][block][unit]: the block's code bytes 16 f .. 16 f + 15
+    gm_u4 sc[2];      // the half's four block scales (f32 bits)
+    uint32_t off_h, off_q, row32, plane;
+    int U;
+    __device__ __forceinline__ void init(int row, int lane, size_t stride, int U_)
+    {
+        U = U_;
+        off_h = (uint32_t)((row + lane) * stride);
+        off_q = (uint32_t)((row + (lane & 31)) * stride) + ((8u * (uint32_t)U + 15u) & ~15u) + 16u * (uint32_t)(lane >> 5);
+        row32 = (uint32_t)(32 * stride);
+        plane = 16u * (uint32_t)U;
+    }
+    __device__ __forceinline__ void head_load(rsrc_t, int) {}
+    __device__ __forceinline__ void head() {}
+    __device__ __forceinline__ void load(rsrc_t rs, int half, int set)
+    {
+        hs[set] = gm_ld(rs, off_h + 16u * (uint32_t)half);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                L[set][j][k] = gm_ld(rs, off_q + (uint32_t)j * row32 + (uint32_t)k * plane + 32u * (uint32_t)half);
+    }
+    __device__ __forceinline__ void split(int half, int set)
+    {
+        // Units past the row's end (a partial last super-block) hold whatever
+        // follows in memory: zero scales, and x is staged as zeros there.
+        gm_u4 h = hs[set];
+        if (2 * half + 1 >= U) { // uniform
+            h[2] = h[3] = 0u;
+            if (2 * half >= U) h[0] = h[1] = 0u;
+        }
+        sc[0] = sc[1] = h;
+        gm_swap32(sc[0], sc[1]);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                q[j][b][0] = L[set][j][2 * b];
+                q[j][b][1] = L[set][j][2 * b + 1];
+                gm_swap32(q[j][b][0], q[j][b][1]);
+            }
+    }
+    __device__ __forceinline__ void frag(int, int v, int t, int j, gm_h8 (&b)[PARTS]) const
+    {
+        const gm_h2 k = gm_dup(1152.0f);
+        const uint32_t w0 = q[j][t >> 1][v][2 * (t & 1)] ^ 0x80808080u;
+        const uint32_t w1 = q[j][t >> 1][v][2 * (t & 1) + 1] ^ 0x80808080u;
+        b[0] = gm_join(gm_bytes<0, 2>(w0) - k, gm_bytes<1, 3>(w0) - k, gm_bytes<0, 2>(w1) - k, gm_bytes<1, 3>(w1) - k);
+    }
+    __device__ __forceinline__ float block_scale(int v, int b, int j) const
+    {
+        return __builtin_bit_cast(float, (uint32_t)sc[j][2 * v + b]);
+    }
+};
+
+// Weight (row, column c) as the reference dequantizes it (dq_* in
+// k_matvec.hip); U units per packed row.
+template <int FMT>
+__device__ float gm_weight(const uint8_t *__restrict__ row, int c, int U)
+{
+    const int nb = U >> 2, sb = c >> 8, e = c & 255;
+    if constexpr (FMT == FMT_Q4K) {
+        const uint8_t *H = row + 16 * sb, *s = H + 4;
+        const float d = f16_to_f32_ref(H[0] | (H[1] << 8)), dmin = f16_to_f32_ref(H[2] | (H[3] << 8));
+        const int u = 4 * sb + (e >> 6), j = e >> 5, b = e & 31;
+        const int q = row[16 * nb + (b < 16 ? 0 : 16 * U) + 16 * u + (b & 15)];
+        const int sc = j < 4 ? s[j] & 63 : (s[j + 4] & 15) | ((s[j - 4] >> 6) << 4);
+        const int m = j < 4 ? s[j + 4] & 63 : (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
+        return __fsub_rn(__fmul_rn(__fmul_rn(d, (float)sc), (float)((e & 32) ? q >> 4 : q & 15)),
+                         __fmul_rn(dmin, (float)m));
+    } else if constexpr (FMT == FMT_Q80) {
+        const int u = c >> 6, b = c & 63;
+        const int8_t q = (int8_t)row[((8 * U + 15) & ~15) + 16 * U * (b >> 4) + 16 * u + (b & 15)];
+        return __fmul_rn((float)q, ((const float *)row)[c >> 5]);
+    } else {
+        const int h = e >> 7, t = (e >> 5) & 3, k = (e >> 4) & 1, i = e & 15, u = 4 * sb + 2 * h + k;
+        const int l = row[16 * nb + 16 * U * (1 + (t & 1)) + 16 * u + i], hi = row[16 * nb + 16 * u + i];
+        const int q = (int)((t < 2 ? l & 15 : l >> 4) | (((hi >> (2 * t)) & 3) << 4)) - 32;
+        const uint8_t *D = row + 16 * nb + 48 * U + 2 * sb;
+        const int sc = (int8_t)row[16 * sb + 8 * h + k + 2 * t];
+        return __fmul_rn(__fmul_rn(f16_to_f32_ref(D[0] | (D[1] << 8)), (float)sc), (float)q);
+    }
+}
+
+// The products of the elements that the staging took out of tokens t0 .. t0 +
+// nt - 1 in super-blocks sb0 .. sb1 - 1, found again by the same rule, into the
+// sums of this lane's rows r and r + 32 (the tile's token t is register 4 (t /
+// 8) + t % 4 of half t / 4 % 2).  Rare: kept out of the streaming loop.
+template <int FMT>
+__device__ __forceinline__ void gm_add_outliers(gm_f16v (&acc)[2], const uint8_t *__restrict__ W, size_t stride,
+                                                int rows, int cols, int r, const float *__restrict__ x, int nt, int sb0,
+                                                int sb1)
+{
+    const int lane = threadIdx.x & 63;
+    for (int sb = sb0; sb < sb1; sb++)
+        for (int t = 0; t < nt; t++) {
+            gm_f4 v = {0.f, 0.f, 0.f, 0.f};
+            if (256 * sb + 4 * lane < cols) v = *(const gm_f4 *)(x + (size_t)t * cols + 256 * sb + 4 * lane);
+            if (__ballot(!(gm_abs_max(v) < INFINITY) || v[0] + v[1] + v[2] + v[3] != v[0] + v[1] + v[2] + v[3]))
+                continue; // a non-finite block: every output is NaN already
+            const float thr = gm_outlier_thr(v);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint64_t todo = __ballot(fabsf(v[i]) > thr);
+                while (todo) { // uniform
+                    const int src = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    const float xv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[i]), src));
+                    const int c = 256 * sb + 4 * src + i;
+                    const bool mine = ((t >> 2) & 1) == lane >> 5;
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const int row = r + 32 * j;
+                        const float p = mine && row < rows ? gm_weight<FMT>(W + (size_t)row * stride, c, cols >> 6) * xv : 0.0f;
+#pragma unroll
+                        for (int k = 0; k < 16; k++)
+                            if (k == 4 * (t >> 3) + (t & 3)) acc[j][k] += p;
+                    }
+                }
+            }
+        }
+}
+
+// A workgroup of four wavefronts owns 256 rows (64 per wavefront, two 32-row
+// tiles) and MT tiles of 32 tokens, over the super-blocks of its split.  A
+// wavefront dequantizes its own rows' operands in registers, once for all its
+// tokens; x comes through LDS, a unit ahead, and each 1 KiB fragment read there
+// feeds two products.  Bound by the matrix cores (two products per weight and
+// token, three for Q6_K) and the dequantization beside them.  Measured on
+// MI355X (us, before -> here; TFLOP/s of the product): Q4_K 14336 x 4096 at 512
+// tokens 319 -> 138 (436), 4096 x 14336 at 199 228 -> 80 (292); Q6_K 4096 x
+// 14336 at 256 3271 -> 106 (284, vector by vector before); Q8_0 4096 x 4096 at
+// 512 187 -> 78 (220).  With the weight loads' 32-byte pieces read from one
+// place instead 124 us at 14336 x 4096 x 512; codes loaded by one lane each (16
+// bytes per row and load) took 213, x's next unit requested where the scheduler
+// put it 204.  A whole super-block's codes in flight measured the same.
+template <int FMT, int MT>
+__global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, size_t stride, int rows, int cols,
+                                                 GmX x, const float *__restrict__ xs32, int n, int ntt, int nsplit,
+                                                 int items, float *__restrict__ out)
+{
+    // consecutive items share their rows (the token tiles of a row block) and
+    // stay on one XCD (workgroups go round the eight in turn), so a row
+    // block's weights come out of HBM once per XCD that holds it
+    const int per = (items + 7) / 8, w = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (w >= items || ((int)blockIdx.x >> 3) >= per) return;
+    const int tt = w % ntt, sp = w / ntt % nsplit, rb = w / (ntt * nsplit);
+    const int lane = threadIdx.x & 63, f = lane >> 5, nl = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nb = (cols + 255) >> 8, U = 4 * nb; // staged super-blocks and units
+    const int sb0 = (int)((long)nb * sp / nsplit), sb1 = (int)((long)nb * (sp + 1) / nsplit);
+    const int r0 = 256 * rb, rend = min(rows, r0 + 256);
+    const rsrc_t rs = make_rsrc(W + (size_t)r0 * stride, (uint32_t)((size_t)(rend - r0) * stride));
+    constexpr int XW = 2 * MT; // 16-byte words of a unit's x per thread
+    __shared__ gm_u4 xs[2][MT * GM_UNIT / 16];
+    __shared__ float ps[2][MT * 32];
+    // this workgroup's token tiles, MT * U units
+    const rsrc_t rx = make_rsrc(x.f + (size_t)tt * MT * U * GM_UNIT, (uint32_t)((size_t)MT * U * GM_UNIT));
+    const float *xp = x.p + ((size_t)(tt * MT + (int)(threadIdx.x >> 5)) * nb) * 32 + (threadIdx.x & 31);
+    GmW<FMT, 1> wt;
+    wt.init(64 * wave, lane, stride, cols >> 6);
+    constexpr int PARTS = GmW<FMT, 1>::PARTS;
+
+    gm_f16v acc[MT][2], S[MT][2];
+    const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[m][j] = zero;
+    gm_u4 xr[XW];
+    auto load_x = [&](int u) {
+#pragma unroll
+        for (int k = 0; k < XW; k++)
+            xr[k] = __builtin_bit_cast(gm_u4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rx, 16 * (int)threadIdx.x,
+                                                  ((k >> 1) * U + u) * GM_UNIT + 4096 * (k & 1), 0));
+    };
+    auto store_x = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < XW; k++) xs[b][(k >> 1) * (GM_UNIT / 16) + 256 * (k & 1) + threadIdx.x] = xr[k];
+    };
+    // Q8_0: the super-block's sums, each block's scale applied
+    gm_f16v T[FMT == FMT_Q80 ? MT : 1][2];
+    uint64_t taken = 0; // whether a token of the tiles had outliers
+    load_x(4 * sb0);
+    wt.head_load(rs, sb0);
+    wt.load(rs, 2 * sb0, 0);
+    store_x(0);
+    __syncthreads();
+    for (int sb = sb0; sb < sb1; sb++) {
+        wt.head();
+        gm_h8 am[MT];
+        float pv = 0.0f;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int u = 4 * sb + p;
+            if (!(p & 1)) wt.split(2 * sb + (p >> 1), 0);
+            // in flight during this unit's products: the next unit's x (the
+            // last unit's once more at the end) and, every other unit, the next
+            // half super-block's weights
+            load_x(min(u + 1, 4 * sb1 - 1));
+            if (p == 1) wt.load(rs, 2 * sb + 1, 0);
+            if (p == 3) {
+                const int sn = min(sb + 1, sb1 - 1);
+                wt.load(rs, 2 * sn, 0);
+                wt.head_load(rs, sn);
+                if (FMT == FMT_Q4K) {
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+                        am[m] = *(const gm_h8 *)(x.m + ((size_t)(tt * MT + m) * nb + sb) * GM_SUMS + 16 * lane);
+                }
+                if ((int)threadIdx.x < MT * 32) pv = xp[(size_t)sb * 32];
+            }
+            __builtin_amdgcn_sched_barrier(0); // (the scheduler would sink the loads to their use)
+            const uint8_t *xb = (const uint8_t *)xs[p & 1] + 16 * lane;
+            // step i = t * MT + m: the next step's x (and codes) are fetched
+            // while this one's products run
+            gm_h8 ah[2], al[2], b[2][2][PARTS];
+            ah[0] = *(const gm_h8 *)xb;
+            al[0] = *(const gm_h8 *)(xb + 1024);
+#pragma unroll
+            for (int j = 0; j < 2; j++) wt.frag(p >> 1, p & 1, 0, j, b[0][j]);
+#pragma unroll
+            for (int i = 0; i < 4 * MT; i++) {
+                const int t = i / MT, m = i % MT, t1 = (i + 1) / MT, m1 = (i + 1) % MT;
+                if (i + 1 < 4 * MT) {
+                    ah[(i + 1) & 1] = *(const gm_h8 *)(xb + m1 * GM_UNIT + t1 * 2048);
+                    al[(i + 1) & 1] = *(const gm_h8 *)(xb + m1 * GM_UNIT + t1 * 2048 + 1024);
+                    if (m == MT - 1) {
+#pragma unroll
+                        for (int j = 0; j < 2; j++) wt.frag(p >> 1, p & 1, t1, j, b[t1 & 1][j]);
+                    }
+                }
+                const gm_h8 hi = ah[i & 1], lo = al[i & 1];
+                // the sums start at the super-block's (Q8_0: the block's) first step
+                const bool first = FMT == FMT_Q80 ? !(t & 1) : p == 0 && t == 0;
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    S[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b[t & 1][j][0], first ? zero : S[m][j], 0, 0, 0);
+                if constexpr (PARTS == 2) {
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        S[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[t & 1][j][PARTS - 1], S[m][j], 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    S[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[t & 1][j][0], S[m][j], 0, 0, 0);
+                if constexpr (FMT == FMT_Q80) {
+                    if (t & 1) {
+#pragma unroll
+                        for (int j = 0; j < 2; j++) {
+                            const float s = wt.block_scale(p & 1, t >> 1, j);
+#pragma unroll
+                            for (int e = 0; e < 16; e++)
+                                T[m][j][e] = p == 0 && t == 1 ? s * S[m][j][e] : fmaf(s, S[m][j][e], T[m][j][e]);
+                            // (keeps the scaling here: sunk to the super-block's
+                            // end, it would hold every block's sums until then)
+                            asm volatile("" : "+v"(T[m][j]));
+                        }
+                    }
+                }
+            }
+            store_x((p + 1) & 1);
+            if (p == 3 && (int)threadIdx.x < MT * 32) ps[sb & 1][threadIdx.x] = pv;
+            __syncthreads();
+        }
+        // out += 2^-s (d S - 32 dmin M), Q6_K without M, Q8_0 2^-s T
+        taken |= __ballot(ps[sb & 1][lane & (32 * MT - 1)] < 0.0f);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            float pt[16]; // 2^-s of this lane's tokens
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 v = *(const float4 *)(ps[sb & 1] + 32 * m + 8 * k + 4 * f);
+                pt[4 * k] = v.x;
+                pt[4 * k + 1] = v.y;
+                pt[4 * k + 2] = v.z;
+                pt[4 * k + 3] = v.w;
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if constexpr (FMT == FMT_Q4K) {
+                    const float d = wt.scale(j), dm = wt.min_scale(j);
+                    const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[m], wt.mins(j), zero, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        acc[m][j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[m][j][i], dm * M[i]), acc[m][j][i]);
+                } else if constexpr (FMT == FMT_Q6K) {
+                    const float d = wt.scale(j);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[m][j][i] = fmaf(fabsf(pt[i]), d * S[m][j][i], acc[m][j][i]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[m][j][i] = fmaf(fabsf(pt[i]), T[m][j][i], acc[m][j][i]);
+                }
+            }
+        }
+    }
+    if (__builtin_expect(taken != 0, 0)) {
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            const int t0 = 32 * (tt * MT + m);
+            gm_add_outliers<FMT>(acc[m], W, stride, rows, cols, r0 + 64 * wave + nl, xs32 + (size_t)t0 * cols,
+                                 min(32, n - t0), sb0, sb1);
+        }
+    }
+    float *o = out + (size_t)sp * n * rows;
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int row = r0 + 64 * wave + 32 * j + nl;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int t = 32 * (tt * MT + m) + 8 * (i >> 2) + 4 * f + (i & 3);
+                if (t < n && row < rows) o[(size_t)t * rows + row] = acc[m][j][i];
+            }
+        }
+}
+
+// The same for few tokens: one tile of 32, x converted by every workgroup
+// itself (a conversion launch took longer than it saved: 14336 x 4096 at 2 / 8 /
+// 16 tokens 24.8 / 24.9 / 25.5 us with one, 18.6 / 20.2 / 22.9 without) a
+// super-block ahead of its products, one barrier per super-block and a whole
+// super-block of weights in flight.
+template <int FMT>
+__global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__ W, size_t stride, int rows, int cols,
+                                                     const float *__restrict__ x, int n_all, int ntt, int nsplit, int items,
+                                                     float *__restrict__ out)
+{
+    const int per = (items + 7) / 8, w = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (w >= items) return;
+    const int tt = w % ntt, sp = w / ntt % nsplit, rb = w / (ntt * nsplit);
+    const int n = min(32, n_all - 32 * tt); // this tile's tokens
+    x += (size_t)32 * tt * cols;
+    const int lane = threadIdx.x & 63, f = lane >> 5, nl = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nb = (cols + 255) >> 8;
+    const int sb0 = (int)((long)nb * sp / nsplit), sb1 = (int)((long)nb * (sp + 1) / nsplit);
+    const int r0 = 256 * rb, rend = min(rows, r0 + 256);
+    const rsrc_t rs = make_rsrc(W + (size_t)r0 * stride, (uint32_t)((size_t)(rend - r0) * stride));
+    GmW<FMT, 2> wt;
+    wt.init(64 * wave, lane, stride, cols >> 6);
+    constexpr int PARTS = GmW<FMT, 2>::PARTS;
+    wt.head_load(rs, sb0);
+    wt.load(rs, 2 * sb0, 0);
+    wt.load(rs, 2 * sb0 + 1, 1);
+    // the staged tile's four units, sums and 2^-s, double-buffered
+    constexpr int SUMS = FMT == FMT_Q4K ? GM_SUMS : 16;
+    __shared__ gm_u4 xs[2][4 * GM_UNIT / 16];
+    __shared__ gm_u4 ms[2][SUMS / 16];
+    __shared__ float ps[2][32];
+    // tokens wave + 4 k: a lane's four columns of each
+    gm_f4 xv[8];
+    const int tmax = (n - wave + 3) >> 2; // this wavefront's tokens
+    auto load_x = [&](int sb) {
+        const bool in = 256 * sb + 4 * lane < cols;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            xv[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
+            if (k < tmax && in) xv[k] = *(const gm_f4 *)(x + (size_t)(wave + 4 * k) * cols + 256 * sb + 4 * lane);
+        }
+    };
+    auto store_x = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (k < tmax)
+                gm_stage_row<FMT>(xv[k], lane, wave + 4 * k, (uint8_t *)xs[b], (uint8_t *)ms[b], &ps[b][wave + 4 * k]);
+    };
+    load_x(sb0);
+    __builtin_amdgcn_sched_barrier(0);
+    // tokens past n stay zero in both buffers
+    for (int i = threadIdx.x; i < 2 * 4 * GM_UNIT / 16; i += 256)
+        if ((i & 31) >= n) (&xs[0][0])[i] = gm_u4{0u, 0u, 0u, 0u};
+    if (FMT == FMT_Q4K && threadIdx.x < 2 * SUMS / 16 && ((int)threadIdx.x & 31) >= n)
+        (&ms[0][0])[threadIdx.x] = gm_u4{0u, 0u, 0u, 0u};
+    if (threadIdx.x < 64) (&ps[0][0])[threadIdx.x] = 0.0f;
+    __syncthreads();
+    store_x(0);
+    load_x(min(sb0 + 1, sb1 - 1));
+    __syncthreads();
+    gm_f16v acc[2], S[2];
+    const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    acc[0] = acc[1] = zero;
+    uint64_t taken = 0;
+    for (int sb = sb0; sb < sb1; sb++) {
+        const int cur = (sb - sb0) & 1, sn = min(sb + 1, sb1 - 1);
+        wt.head();
+        wt.head_load(rs, sn);
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            if (!(p & 1)) {
+                wt.split(2 * sb + (p >> 1), p >> 1);
+                wt.load(rs, 2 * sn + (p >> 1), p >> 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const uint8_t *xb = (const uint8_t *)xs[cur] + p * GM_UNIT + 16 * lane;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                gm_h8 b[2][PARTS];
+#pragma unroll
+                for (int j = 0; j < 2; j++) wt.frag(p >> 1, p & 1, t, j, b[j]);
+                const gm_h8 hi = *(const gm_h8 *)(xb + t * 2048), lo = *(const gm_h8 *)(xb + t * 2048 + 1024);
+                const bool first = p == 0 && t == 0;
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b[j][0], first ? zero : S[j], 0, 0, 0);
+                if constexpr (PARTS == 2) {
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[j][PARTS - 1], S[j], 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[j][0], S[j], 0, 0, 0);
+            }
+        }
+        taken |= __ballot(ps[cur][lane & 31] < 0.0f);
+        float pt[16];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const gm_f4 v = *(const gm_f4 *)(ps[cur] + 8 * k + 4 * f);
+#pragma unroll
+            for (int i = 0; i < 4; i++) pt[4 * k + i] = v[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (FMT == FMT_Q4K) {
+                const float d = wt.scale(j), dm = wt.min_scale(j);
+                const gm_h8 am = *(const gm_h8 *)((const uint8_t *)ms[cur] + 16 * lane);
+                const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wt.mins(j), zero, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[j][i], dm * M[i]), acc[j][i]);
+            } else {
+                const float d = wt.scale(j);
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), d * S[j][i], acc[j][i]);
+            }
+        }
+        if (sb + 1 < sb1) { // uniform
+            store_x(cur ^ 1);
+            load_x(min(sb + 2, sb1 - 1));
+            __syncthreads();
+        }
+    }
+    if (__builtin_expect(taken != 0, 0))
+        gm_add_outliers<FMT>(acc, W, stride, rows, cols, r0 + 64 * wave + nl, x, n, sb0, sb1);
+    float *o = out + ((size_t)sp * n_all + 32 * tt) * rows;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int row = r0 + 64 * wave + 32 * j + nl;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = 8 * (i >> 2) + 4 * f + (i & 3);
+            if (t < n && row < rows) o[(size_t)t * rows + row] = acc[j][i];
+        }
+    }
+}
+
+// y = the splits' partial sums, added in split order; eight splits' values are
+// requested at a time (one after another, a thread's chain of round trips was
+// longer than the products: 1117 x 6912 at 49 tokens, 27 splits).
+template <typename T> // float, or four (where the splits' starts are 16-byte aligned)
+__global__ void __launch_bounds__(256) k_gm_reduce(const float *__restrict__ part, long count, int nsplit,
+                                                   float *__restrict__ y)
+{
+    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * (long)(sizeof(T) / 4);
+    if (i >= count) return;
+    T s = *(const T *)(part + i);
+    for (int k0 = 1; k0 < nsplit; k0 += 8) {
+        T v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = *(const T *)(part + min(k0 + k, nsplit - 1) * count + i);
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (k0 + k < nsplit) s += v[k]; // uniform
+    }
+    *(T *)(y + i) = s;
+}
+
+static bool gemm_shape_ok(uint8_t dtype, size_t rows, size_t cols)
+{
+    return (dtype == SOSO_HIP_DTYPE_Q4_K || dtype == SOSO_HIP_DTYPE_Q8_0 || dtype == SOSO_HIP_DTYPE_Q6_K) &&
+           cols % (dtype == SOSO_HIP_DTYPE_Q8_0 ? 64 : 256) == 0 && cols >= 256 && cols <= (1u << 20) && rows > 0 &&
+           rows < ((size_t)1 << 31) - 256 && (size_t)256 * packed_row_stride(dtype, cols) < ((size_t)1 << 31);
+}
+
+// Where these kernels are the faster ones, from both sides measured on
+// MI355X over rows x cols from 300 x 512 to 14336 x 14336 (us, before -> here):
+//  * Rows of more than 4096 columns ran vector by vector below 16 tokens (and
+//    always for Q6_K): 4096 x 14336 at 4 tokens 40 -> 22 (Q4_K), 50 -> 32
+//    (Q6_K); at 3 small matrices lose (300 x 8192: 17 -> 20).  Q8_0 wins from
+//    6 (79 -> 58; at 4: 53 -> 59).
+//  * Q4_K up to 4096 columns: against the batched vector kernel (below 16
+//    tokens) from 8 tokens and 2^22 weights (14336 x 4096 36.5 -> 20.2, 2048 x
+//    2048 10.1 -> 9.5; 768 x 2048 8.8 -> 9.4).  Against the integer matrix-core
+//    kernels, whose time is one chain along the columns, everywhere from 4096
+//    columns and 2^22 weights on (1024 x 4096 at 16 / 64 / 128 tokens 15.9 /
+//    16.1 / 24.8 -> 11.1 / 13.8 / 16.6); with fewer columns past 64 tokens
+//    (11305 x 768 at 64 / 100: 16.0 / 30.2 -> 18.8 / 18.0; 1000 x 1024 at 128:
+//    7.0 -> 11.9) or past 2^24 weights at 17 to 32 (14336 x 2048 at 16 / 24 /
+//    32 / 48: 15.1 / 25.3 / 24.4 / 23.2 -> 16.5 / 18.7 / 20.7 / 27.2).  Their
+//    form with x staged once (whole rounds of 16 tokens, whole 1024-column
+//    chunks) holds out longer: 2048 x 2048 at 128 / 300 tokens 14.9 / 35.3 ->
+//    16.1 / 26.8, 14336 x 2048 at 128 47.6 -> 34.4.
+//  * Q6_K up to 4096 columns: past 2^24 weights from 8 tokens (14336 x 4096
+//    41.7 -> 27.6); smaller ones from 48 tokens (1000 x 1024 38.9 -> 15.4),
+//    below which they keep the batched vector kernel and with it the bits of
+//    single matvecs.
+//  * Q8_0, whose four code planes cost its lines four visits: past 2^24 weights
+//    from 33 tokens (14336 x 4096 at 64: 97 -> 51; at 32: 51 -> 53), from 2^22
+//    weights at 16 tokens where a row has 4096 columns (1024 x 4096 24.1 ->
+//    14.4) and at 64 where it has fewer (2048 x 2048 21.7 -> 16.5; at 32: 13.2
+//    -> 15.5).  Widths that are no multiple of 256 ran on the batched vector
+//    kernel: from 16 tokens (5000 x 1440 26.3 -> 17.2), if 2^22 weights or
+//    1024 columns (2014 x 768 at 149: 15.6 -> 16.3).
+bool gemm_wins(uint8_t dtype, size_t rows, size_t cols, size_t n)
+{
+    if (n < 4 || n > (1u << 20) || !gemm_shape_ok(dtype, rows, cols)) return false;
+    const size_t weights = rows * cols;
+    const bool large = weights > (1u << 24), small = weights < (1u << 22);
+    if (dtype == SOSO_HIP_DTYPE_Q8_0) {
+        if (cols > 4096) return n >= 6;
+        if (cols % 256) return n >= 16 && (!small || cols >= 1024);
+        if (large) return n >= 33;
+        return !small && n >= (cols >= 4096 ? 16 : 64);
+    }
+    if (cols > 4096) return true;
+    if (dtype == SOSO_HIP_DTYPE_Q6_K) return n >= (large ? 8 : 48);
+    if (!small && n < 16) return n >= 8;
+    if (!small && cols >= 4096) return true;
+    if (n <= 64) return large && n > 16 && n <= 32;
+    if (n % 16 == 0 && cols % 1024 == 0 && n <= 128) return weights * n >= 3000000000u;
+    return weights * n >= 200000000u;
+}
+
+static int gm_reduce(soso_hip *h, const float *part, size_t count, size_t nsplit, float *y)
+{
+    if (count % 4 == 0 && ((uintptr_t)y & 15) == 0)
+        k_gm_reduce<gm_f4><<<(unsigned)((count + 1023) / 1024), 256, 0, h->stream>>>(part, (long)count, (int)nsplit, y);
+    else
+        k_gm_reduce<float><<<(unsigned)((count + 255) / 256), 256, 0, h->stream>>>(part, (long)count, (int)nsplit, y);
+    return hip_check(h, hipGetLastError(), "gemm reduce launch");
+}
+
+template <int FMT>
+static int launch_gemm_fmt(soso_hip *h, const Weight &w, const float *x, size_t n, float *y)
+{
+    const size_t cols = weight_kcols(w), rows = w.rows, nb = (cols + 255) / 256, rb = (rows + 255) / 256;
+    const size_t stride = packed_row_stride(w.dtype, cols);
+    // Few tokens, or a small product: a chain of super-blocks per workgroup that
+    // is short on round trips beats more products per weight (4096 x 4096 at 64
+    // tokens 20.6 us against 25.4, 6905 x 1280 at 200 26.6 against 33.3; at 200
+    // tokens 4096 x 4096 42.3 against 35.2, 14336 x 4096 at 64 43.4 against
+    // 37.5).
+    const bool few = FMT != FMT_Q80 && (n <= 32 || rows * cols * n <= ((size_t)1 << 31));
+    // (Q8_0's per-block scales need a second set of sums: one token tile)
+    const size_t MT = FMT != FMT_Q80 && !few ? 2 : 1;
+    const size_t ntt = (n + 32 * MT - 1) / (32 * MT), tiles = ntt * MT;
+    // as many column splits as fill the GPU's workgroup slots: two per CU, one
+    // for few tokens (fewer partial sums; 14336 x 4096 at 2 / 8 / 32 tokens
+    // 18.6 / 20.2 / 27.9 us against 19.3 / 20.9 / 28.9 with two)
+    const size_t slots = (few ? 1 : 2) * (size_t)h->num_cu;
+    const size_t nsplit = std::max<size_t>(1, std::min(nb, slots / (ntt * rb)));
+    const size_t items = rb * nsplit * ntt;
+    const unsigned grid = (unsigned)((items + 7) / 8 * 8);
+    float *part = y;
+    if (nsplit > 1) {
+        part = (float *)scratch_get(h, 17, nsplit * n * rows * 4);
+        if (!part) return SOSO_HIP_DECLINED;
+    }
+    if (few) {
+        if constexpr (FMT != FMT_Q80)
+            k_gemm_few<FMT><<<grid, 256, 0, h->stream>>>((const uint8_t *)w.dev, stride, (int)rows, (int)cols, x,
+                                                         (int)n, (int)ntt, (int)nsplit, (int)items, part);
+    } else {
+        const size_t f_b = tiles * nb * (4 * GM_UNIT), m_b = tiles * nb * GM_SUMS, p_b = tiles * nb * 128;
+        uint8_t *xg = (uint8_t *)scratch_get(h, 16, f_b + m_b + p_b);
+        if (!xg) return SOSO_HIP_DECLINED;
+        float *xp = (float *)(xg + f_b + m_b);
+        const GmX gx{xg, xg + f_b, xp};
+        k_gm_stage<FMT><<<(unsigned)(tiles * nb), 512, 0, h->stream>>>(x, (int)n, (int)cols, xg, xg + f_b, xp);
+        k_gemm<FMT, FMT == FMT_Q80 ? 1 : 2><<<grid, 256, 0, h->stream>>>(
+            (const uint8_t *)w.dev, stride, (int)rows, (int)cols, gx, x, (int)n, (int)ntt, (int)nsplit, (int)items, part);
+    }
+    const int rc = hip_check(h, hipGetLastError(), "gemm launch");
+    return rc == SOSO_HIP_OK && nsplit > 1 ? gm_reduce(h, part, n * rows, nsplit, y) : rc;
+}
+
+// DECLINED when the scratch it needs cannot be had (memory, or a slot that
+// would have to grow inside a graph capture): the other kernels, which need
+// none, take the call.
+int launch_gemm(soso_hip *h, const Weight &w, const float *x, size_t n, float *y)
+{
+    switch (w.dtype) {
+    case SOSO_HIP_DTYPE_Q4_K: return launch_gemm_fmt<FMT_Q4K>(h, w, x, n, y);
+    case SOSO_HIP_DTYPE_Q8_0: return launch_gemm_fmt<FMT_Q80>(h, w, x, n, y);
+    default: return launch_gemm_fmt<FMT_Q6K>(h, w, x, n, y);
+    }
+}

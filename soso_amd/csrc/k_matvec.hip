@@ -864,13 +864,14 @@ int launch_matvec_ex(soso_hip *h, const Weight &w, const MvIn &in, float *y, con
     return hip_check(h, hipGetLastError(), "matvec_ex launch");
 }
 
-// n vectors: from MATMUL_MFMA_MIN tokens up, Q4_K and Q8_0 rows of whole
-// 256-column super-blocks go to the matrix cores (k_mfma.hip: within the same
-// 1e-5 of the exact product, not bit-identical to the single-vector kernel);
-// fewer vectors, Q6_K at any count and other Q8_0 widths run mv_tok (each row
-// read once per launch of up to 16 tokens, every output bit-identical to its
-// own matvec); rows wider than 4096 columns run the single-vector kernel once
-// per vector.
+// n vectors.  Where enough tokens meet enough weights (gemm_wins) the f16
+// matrix cores take them (k_gemm.hip: closer to the exact product than the
+// single-vector kernel, not bit-identical to it).  Of the rest, from
+// MATMUL_MFMA_MIN tokens up, Q4_K and Q8_0 rows of whole 256-column
+// super-blocks go to the integer matrix cores (k_mfma.hip); others run mv_tok
+// (each row read once per launch of up to 16 tokens, every output bit-identical
+// to its own matvec), and rows wider than 4096 columns the single-vector kernel
+// once per vector.
 constexpr size_t MATMUL_MFMA_MIN = 16;
 
 // Tokens per wavefront of mv_tok: each loaded unit meets two tokens' digits
@@ -943,6 +944,10 @@ int launch_matvec(soso_hip *h, const Weight &w, const float *x, float *y, size_t
         const int rc = hip_check(h, hipGetLastError(), "pad x launch");
         if (rc != SOSO_HIP_OK) return rc;
         x = xp;
+    }
+    if (gemm_wins(w.dtype, w.rows, kc, n)) {
+        const int rc = launch_gemm(h, w, x, n, y);
+        if (rc != SOSO_HIP_DECLINED) return rc;
     }
     if (n >= MATMUL_MFMA_MIN && mfma_shape_ok(w.dtype, w.rows, kc)) return launch_mfma_matmul(h, w, x, n, y);
     // several tokens, rows of at most 64 units: each row read once per launch

@@ -281,8 +281,9 @@ int launch_kv_scatter(soso_hip *h, const void *src, bool src_f32, void *cache, b
 int launch_shared_swiglu(soso_hip *h, const float *g, float *u, size_t n);
 int launch_shared_gate(soso_hip *h, const float *x, const float *pg_w, float *y, size_t n, size_t hdim);
 // (k_gdn.hip) Gated DeltaNet block (GpuDispatch::gdn_bloque): null when the
-// shape runs, else why not; the launch needs u, n x (2 n_k + n_v) d floats.
+// shape runs, else why not; the launch needs u, gdn_scratch_floats floats.
 const char *gdn_unsupported(size_t n, size_t n_k, size_t n_v, size_t d, size_t kernel);
+size_t gdn_scratch_floats(size_t n, size_t n_k, size_t n_v);
 int launch_gdn_block(soso_hip *h, const float *hist, const float *conv, const float *z, const float *decay,
                      const float *beta, const float *norm, float *state, float *out, float *u, int n, int n_k,
                      int n_v, int kernel, float eps);

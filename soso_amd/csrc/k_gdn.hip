@@ -3,152 +3,318 @@
 // soso's CPU path computes it (bloque35.rs:372-465; one token of the decode
 // layer, arch.rs:586-768, is the same with n = 1).
 //
-// Two launches per block of n tokens:
-//   k_gdn_conv  grid (2 n_k + n_v heads, n tokens), one thread per channel of
-//               a head (d = 128): the causal conv over the history window,
-//               SiLU, and for q / k heads the l2 normalisation (q also scaled
-//               by 1 / sqrt(d)) -> u [n][C], C = 2 n_k d + n_v d
-//   k_gdn_rec   one workgroup of 1024 threads per value head: the head's
-//               d x d state lives in registers (thread (r, j) holds column j,
-//               rows 16 r .. 16 r + 15) for the whole block, read once and
-//               written once; per token
-//                 delta_j = (v_j - g sum_i S_ij k_i) beta
-//                 S_ij   <- g S_ij + k_i delta_j
-//                 o_j     = sum_i S_ij q_i
-//               then rmsnorm(o) with the ssm_norm weights and o *= silu(z).
-// The column sums run as 16-row partial sums per thread, combined over the 8
-// row groups through LDS (the CPU sums i in order; the bar is relative L2).
-// The next token's q, k, v and z are requested while the current token's
-// recurrence runs.
-// State traffic per block: 2 * n_v d^2 * 4 bytes (2 MiB each way for 32 heads
-// of 128), independent of n.
+// With S the head's d x d state (d = 128), per token
+//     delta_j = (v_j - g sum_i S_ij k_i) beta
+//     S_ij   <- g S_ij + k_i delta_j
+//     o_j     = sum_i S_ij q_i = g (sum_i S_ij q_i before) + delta_j (k . q)
+// then rmsnorm(o) with the ssm_norm weights and o *= silu(z).  Nothing joins
+// two columns j before the norm, so the columns of a head run apart:
+//   k_gdn_conv  a wavefront per token and q/k head pair or value head: the
+//               causal conv over the history window, SiLU, and for q / k the
+//               l2 normalisation (q also scaled by 1 / sqrt(d)) -> u [n][C],
+//               C = 2 n_k d + n_v d, and k . q [n][n_k]
+//   k_gdn_rec   the recurrence in eight workgroups per value head, the state
+//               in registers for the whole block, read once and written once;
+//               both sums of a token in one pass over the rows, then DPP adds
+//               across a column's lanes: no barrier per token
+//   k_gdn_norm  the norm and the gate, a wavefront per token and head
+//   k_gdn_rec_few  up to GDN_FEW tokens: a workgroup per head, norm and gate
+//               included (one launch less)
+// Both recurrences add in the same order, so a block's bits do not depend on how
+// its tokens were split into calls.  One workgroup of 1024 threads per head,
+// four workgroup barriers per token, took 370 us for 256 tokens of 32 heads;
+// the state traffic per block is 2 * n_v d^2 * 4 bytes (2 MiB each way for 32
+// heads), independent of n.
 #include "internal.hpp"
 
-constexpr int GDN_D = 128;             // head dim handled (gdn_bloque: d == 128 only)
-constexpr int GDN_RG = 8;              // row groups of the state per workgroup
-constexpr int GDN_RPT = GDN_D / GDN_RG; // state rows per thread
+constexpr int GDN_D = 128;    // head dim handled (gdn_bloque: d == 128 only)
+// Tokens up to which one workgroup takes a whole head (us per call, 32 value
+// heads, one workgroup per head / eight and the norm's launch: 4 tokens 8.98,
+// 5 9.93 / 9.8, 8 12.6 / 9.8).
+constexpr int GDN_FEW = 4;
+constexpr int GDN_CHUNK = 32; // tokens staged in LDS at a time beyond
 
 __device__ __forceinline__ float gdn_silu(float x) { return x / (1.0f + expf(-x)); }
 
-// Workgroup barrier for LDS only: LDS operations complete, then s_barrier,
-// without waiting for outstanding global loads (__syncthreads' fence would
-// wait for the next token's q/k/v/z, requested ahead on purpose).  The memory
-// clobber keeps the compiler from moving memory operations across it.
-__device__ __forceinline__ void gdn_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// sum over the 128 threads of a two-wavefront workgroup, returned to all
-__device__ __forceinline__ float gdn_sum128(float v, float *red)
+// sum over the wavefront, returned to all lanes
+__device__ __forceinline__ float gdn_sum64(float v)
 {
     v = seg_sum_dpp<64>(v);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 63) red[wave] = v;
-    __syncthreads();
-    const float s = red[0] + red[1];
-    __syncthreads();
-    return s;
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-__global__ void __launch_bounds__(GDN_D) k_gdn_conv(const float *__restrict__ hist, const float *__restrict__ conv,
-                                                    int C, int n_k, int kernel, float eps, float *__restrict__ u)
+// silu(conv) of two channels (2 lane, 2 lane + 1 of head hh) for token t
+__device__ __forceinline__ float2 gdn_conv2(const float *__restrict__ hist, const float *__restrict__ conv, int C,
+                                            int kernel, int ch, int t)
 {
-    __shared__ float red[2];
-    const int hh = blockIdx.x, t = blockIdx.y, ch = hh * GDN_D + (int)threadIdx.x;
-    const int prev = kernel - 1;
-    float acc = 0.0f;
-    for (int k = 0; k < prev; k++) acc = __fadd_rn(acc, __fmul_rn(conv[(size_t)ch * kernel + k], hist[(size_t)(t + k) * C + ch]));
-    acc = __fadd_rn(acc, __fmul_rn(conv[(size_t)ch * kernel + prev], hist[(size_t)(t + prev) * C + ch]));
-    float x = gdn_silu(acc);
-    if (hh < 2 * n_k) { // block-uniform
-        const float ss = gdn_sum128(x * x, red);
-        x *= 1.0f / sqrtf(ss + eps);
-        if (hh < n_k) x *= 1.0f / sqrtf((float)GDN_D);
+    float a = 0.0f, b = 0.0f;
+    for (int k = 0; k < kernel; k++) {
+        const float2 h = *(const float2 *)(hist + (size_t)(t + k) * C + ch);
+        a = __fadd_rn(a, __fmul_rn(conv[(size_t)ch * kernel + k], h.x));
+        b = __fadd_rn(b, __fmul_rn(conv[(size_t)(ch + 1) * kernel + k], h.y));
     }
-    u[(size_t)t * C + ch] = x;
+    return make_float2(gdn_silu(a), gdn_silu(b));
 }
 
-__global__ void __launch_bounds__(GDN_D * GDN_RG) k_gdn_rec(const float *__restrict__ u, const float *__restrict__ z,
-                                                           const float *__restrict__ decay,
-                                                           const float *__restrict__ beta,
-                                                           const float *__restrict__ norm, float *__restrict__ state,
-                                                           float *__restrict__ out, int n, int n_k, int n_v, float eps)
+// Wavefront: unit (a q/k head pair, then the value heads) of one token; kernel
+// widths 1..4 unrolled (KW), others by the loop (KW = 0).  (2 / 4 / 8 tokens
+// per wavefront, sharing their window: 256 tokens 55.5 / 58.1 / 66.1 us per call
+// against 54.8.)
+template <int KW>
+__global__ void __launch_bounds__(256) k_gdn_conv(const float *__restrict__ hist, const float *__restrict__ conv, int n,
+                                                  int n_k, int n_v, int kernel_, float eps, float *__restrict__ u,
+                                                  float *__restrict__ kq)
+{
+    const int kernel = KW ? KW : kernel_;
+    const int lane = threadIdx.x & 63, units = n_k + n_v;
+    const long gw = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int unit = (int)(gw % units);
+    const long t = gw / units;
+    if (t >= n) return; // no barriers here
+    const int C = (2 * n_k + n_v) * GDN_D;
+    const bool qk = unit < n_k;
+    const int ch = (qk ? unit : n_k + unit) * GDN_D + 2 * lane; // q head, or value head
+    float *ut = u + (size_t)t * C;
+    float2 q = gdn_conv2(hist, conv, C, kernel, ch, (int)t);
+    if (qk) {
+        const int ck = ch + n_k * GDN_D;
+        float2 k = gdn_conv2(hist, conv, C, kernel, ck, (int)t);
+        const float qn = 1.0f / sqrtf(gdn_sum64(q.x * q.x + q.y * q.y) + eps);
+        const float kn = 1.0f / sqrtf(gdn_sum64(k.x * k.x + k.y * k.y) + eps);
+        const float sc = 1.0f / sqrtf((float)GDN_D);
+        q = make_float2(q.x * qn * sc, q.y * qn * sc);
+        k = make_float2(k.x * kn, k.y * kn);
+        *(float2 *)(ut + ck) = k;
+        const float d = gdn_sum64(fmaf(k.x, q.x, k.y * q.y));
+        if (lane == 0) kq[(size_t)t * n_k + unit] = d;
+    }
+    *(float2 *)(ut + ch) = q;
+}
+
+// rmsnorm(o) over the head (gemm.rs:93-100) with its weights, then the SiLU
+// gate, of columns 2 lane and 2 lane + 1
+__device__ __forceinline__ float2 gdn_norm2(float2 o, float2 z, const float *__restrict__ norm, int lane, float eps)
+{
+    const float scale = 1.0f / sqrtf(gdn_sum64(o.x * o.x + o.y * o.y) / (float)GDN_D + eps);
+    const float2 w = *(const float2 *)(norm + 2 * lane);
+    return make_float2(__fmul_rn(__fmul_rn(__fmul_rn(o.x, scale), w.x), gdn_silu(z.x)),
+                       __fmul_rn(__fmul_rn(__fmul_rn(o.y, scale), w.y), gdn_silu(z.y)));
+}
+
+// The sums over a row group's eight rows (rows 4 r .. 4 r + 3 and 64 + 4 r ..
+// 64 + 4 r + 3 of group r = 0 .. 15, so that LDS reads are contiguous), and a
+// token's step once both sums over the 16 groups are there: the pieces that
+// both recurrence kernels share, so that their bits agree.
+__device__ __forceinline__ void gdn_group(const float (&S)[8], const float4 (&k)[2], const float4 (&q)[2], float &p,
+                                          float &r)
+{
+    const float kk[8] = {k[0].x, k[0].y, k[0].z, k[0].w, k[1].x, k[1].y, k[1].z, k[1].w};
+    const float qq[8] = {q[0].x, q[0].y, q[0].z, q[0].w, q[1].x, q[1].y, q[1].z, q[1].w};
+    float p1 = S[4] * kk[4], r1 = S[4] * qq[4];
+    p = S[0] * kk[0];
+    r = S[0] * qq[0];
+#pragma unroll
+    for (int i = 1; i < 4; i++) {
+        p = fmaf(S[i], kk[i], p);
+        p1 = fmaf(S[4 + i], kk[4 + i], p1);
+        r = fmaf(S[i], qq[i], r);
+        r1 = fmaf(S[4 + i], qq[4 + i], r1);
+    }
+    p += p1;
+    r += r1;
+}
+__device__ __forceinline__ float gdn_delta(float v, float g, float beta, float p) { return fmaf(-g, p, v) * beta; }
+__device__ __forceinline__ float gdn_out(float delta, float kq, float g, float r) { return fmaf(delta, kq, g * r); }
+__device__ __forceinline__ void gdn_update(float (&S)[8], const float4 (&k)[2], float g, float delta)
+{
+    const float kk[8] = {k[0].x, k[0].y, k[0].z, k[0].w, k[1].x, k[1].y, k[1].z, k[1].w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) S[i] = fmaf(kk[i], delta, g * S[i]);
+}
+
+// Up to GDN_FEW tokens: a workgroup per head, thread (r, j): column j, row
+// groups 2 r and 2 r + 1 (whole rows of the state per load).  The groups' sums
+// meet in LDS, one barrier per token; every thread of a column adds them.
+__global__ void __launch_bounds__(1024) k_gdn_rec_few(const float *__restrict__ u, const float *__restrict__ kq,
+                                                      const float *__restrict__ z, const float *__restrict__ decay,
+                                                      const float *__restrict__ beta, const float *__restrict__ norm,
+                                                      float *__restrict__ state, float *__restrict__ out, int n, int n_k,
+                                                      int n_v, float eps)
 {
     constexpr int D = GDN_D;
-    __shared__ float qs[D], ks[D], vs[D], zs[D], dl[D];
-    __shared__ float part[GDN_RG][D];
-    __shared__ float red[2];
-    const int vh = blockIdx.x, kh = vh % n_k, tid = threadIdx.x;
-    const int j = tid & (D - 1), r = tid >> 7;
-    const int qk = n_k * D, C = 2 * qk + n_v * D, vd = n_v * D;
-    float *st = state + (size_t)vh * D * D;
-    float S[GDN_RPT];
+    __shared__ float qk[GDN_FEW][2 * D];
+    __shared__ float vs[GDN_FEW][D];
+    __shared__ float2 part[2][8][D];
+    __shared__ float os[GDN_FEW][D];
+    const int vh = blockIdx.x, kh = vh % n_k, tid = threadIdx.x, j = tid & (D - 1), r = tid >> 7;
+    const int qd = n_k * D, C = 2 * qd + n_v * D, vd = n_v * D;
+    float *st = state + (size_t)vh * D * D + j;
+    for (int w = tid; w < n * 3 * D; w += 1024) { // n q, k, v rows of the head
+        const int t = w / (3 * D), c = w % (3 * D);
+        const float x = u[(size_t)t * C + (c < D ? kh * D + c : c < 2 * D ? qd + kh * D + c - D : 2 * qd + vh * D + c - 2 * D)];
+        if (c < 2 * D) qk[t][c] = x;
+        else vs[t][c - 2 * D] = x;
+    }
+    float S[2][8];
 #pragma unroll
-    for (int ii = 0; ii < GDN_RPT; ii++) S[ii] = st[(size_t)(r * GDN_RPT + ii) * D + j];
-    // threads 0 .. 127 carry one token's q, k, v, z ahead of the recurrence
-    float nq = 0.0f, nk = 0.0f, nv = 0.0f, nz = 0.0f;
-    auto fetch = [&](int t) {
-        if (tid < D) {
-            const float *ut = u + (size_t)t * C;
-            nq = ut[kh * D + tid];
-            nk = ut[qk + kh * D + tid];
-            nv = ut[2 * qk + vh * D + tid];
-            nz = z[(size_t)t * vd + vh * D + tid];
-        }
-    };
-    fetch(0);
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) S[a][i] = st[(size_t)(64 * (i >> 2) + 4 * (2 * r + a) + (i & 3)) * D];
+    __syncthreads();
     for (int t = 0; t < n; t++) {
-        if (tid < D) {
-            qs[tid] = nq;
-            ks[tid] = nk;
-            vs[tid] = nv;
-            zs[tid] = nz;
-        }
-        const float g = decay[(size_t)t * n_v + vh], b = beta[(size_t)t * n_v + vh];
-        gdn_lds_barrier();
-        if (t + 1 < n) fetch(t + 1); // in flight during this token's recurrence
-        // delta_j = (v_j - g sum_i S_ij k_i) beta
-        float p = 0.0f;
+        const float g = decay[(size_t)t * n_v + vh], b = beta[(size_t)t * n_v + vh], d = kq[(size_t)t * n_k + kh];
+        float4 k4[2][2], q4[2][2];
 #pragma unroll
-        for (int ii = 0; ii < GDN_RPT; ii++) p = __fadd_rn(p, __fmul_rn(S[ii], ks[r * GDN_RPT + ii]));
-        part[r][j] = p;
-        gdn_lds_barrier();
-        if (tid < D) {
-            float s = part[0][j];
+        for (int a = 0; a < 2; a++)
 #pragma unroll
-            for (int q = 1; q < GDN_RG; q++) s = __fadd_rn(s, part[q][j]);
-            dl[j] = __fmul_rn(__fsub_rn(vs[j], __fmul_rn(g, s)), b);
-        }
-        gdn_lds_barrier();
-        // S_ij <- g S_ij + k_i delta_j;  o_j = sum_i S_ij q_i (updated state)
-        const float dj = dl[j];
-        p = 0.0f;
+            for (int h = 0; h < 2; h++) {
+                q4[a][h] = *(const float4 *)&qk[t][64 * h + 4 * (2 * r + a)];
+                k4[a][h] = *(const float4 *)&qk[t][D + 64 * h + 4 * (2 * r + a)];
+            }
+        float p0, r0, p1, r1;
+        gdn_group(S[0], k4[0], q4[0], p0, r0);
+        gdn_group(S[1], k4[1], q4[1], p1, r1);
+        part[t & 1][r][j] = make_float2(p0 + p1, r0 + r1);
+        __syncthreads();
+        float2 s[8];
 #pragma unroll
-        for (int ii = 0; ii < GDN_RPT; ii++) {
-            const int i = r * GDN_RPT + ii;
-            S[ii] = __fadd_rn(__fmul_rn(g, S[ii]), __fmul_rn(ks[i], dj));
-            p = __fadd_rn(p, __fmul_rn(S[ii], qs[i]));
-        }
-        part[r][j] = p;
-        gdn_lds_barrier();
-        // o_j in threads 0 .. 127 (wavefronts 0 and 1); rmsnorm over the head
-        // (gemm.rs:93-100), then the SiLU gate
-        float o = 0.0f;
-        if (tid < D) {
-            o = part[0][j];
-#pragma unroll
-            for (int q = 1; q < GDN_RG; q++) o = __fadd_rn(o, part[q][j]);
-        }
-        const float ws = seg_sum_dpp<64>(tid < D ? o * o : 0.0f);
-        if ((tid & 63) == 63 && tid < D) red[tid >> 6] = ws;
-        gdn_lds_barrier();
-        if (tid < D) {
-            const float scale = 1.0f / sqrtf((red[0] + red[1]) / (float)D + eps);
-            o = __fmul_rn(__fmul_rn(o, scale), norm[j]);
-            out[(size_t)t * vd + vh * D + j] = __fmul_rn(o, gdn_silu(zs[j]));
-        }
-        gdn_lds_barrier(); // qs / ks / vs / zs / part / red reused by the next token
+        for (int a = 0; a < 8; a++) s[a] = part[t & 1][a][j];
+        const float p = ((s[0].x + s[1].x) + (s[2].x + s[3].x)) + ((s[4].x + s[5].x) + (s[6].x + s[7].x));
+        const float ro = ((s[0].y + s[1].y) + (s[2].y + s[3].y)) + ((s[4].y + s[5].y) + (s[6].y + s[7].y));
+        const float dj = gdn_delta(vs[t][j], g, b, p);
+        gdn_update(S[0], k4[0], g, dj);
+        gdn_update(S[1], k4[1], g, dj);
+        if (r == 0) os[t][j] = gdn_out(dj, d, g, ro);
     }
 #pragma unroll
-    for (int ii = 0; ii < GDN_RPT; ii++) st[(size_t)(r * GDN_RPT + ii) * D + j] = S[ii];
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) st[(size_t)(64 * (i >> 2) + 4 * (2 * r + a) + (i & 3)) * D] = S[a][i];
+    __syncthreads();
+    const int lane = tid & 63, wave = tid >> 6;
+    if (wave < n) {
+        const size_t o = (size_t)wave * vd + vh * D + 2 * lane;
+        *(float2 *)(out + o) =
+            gdn_norm2(*(const float2 *)&os[wave][2 * lane], *(const float2 *)(z + o), norm, lane, eps);
+    }
+}
+
+// Longer blocks: 16 columns per workgroup, four per wavefront, a column's 16
+// row groups in 16 lanes: 256 workgroups, a wavefront per SIMD, for 32 heads.
+// Bound by the chain of one token's instructions (about 70, 0.15 us): 256 tokens
+// of 16 q/k and 32 value heads took 385 us per call on MI355X with a workgroup
+// and four barriers per token and head, 55 us now; 64 tokens 86.8 -> 19.8.
+__global__ void __launch_bounds__(256) k_gdn_rec(const float *__restrict__ u, const float *__restrict__ kq,
+                                                 const float *__restrict__ decay, const float *__restrict__ beta,
+                                                 float *__restrict__ state, float *__restrict__ out, int n, int n_k,
+                                                 int n_v)
+{
+    constexpr int D = GDN_D, COLS = 16, NT = 256, TC = GDN_CHUNK, KQ = TC * 2 * D / 4 / NT, VW = TC * COLS / NT;
+    __shared__ float qk[2][TC][2 * D];
+    __shared__ float vs[2][TC][COLS];
+    __shared__ float4 gs[2][TC]; // g, beta, k . q
+    __shared__ float os[TC][COLS];
+    const int vh = (int)blockIdx.x % n_v, c0 = (int)blockIdx.x / n_v * COLS, kh = vh % n_k;
+    const int tid = threadIdx.x, cl = tid >> 4, rg = tid & 15; // column of the workgroup, row group
+    const int qd = n_k * D, C = 2 * qd + n_v * D, vd = n_v * D;
+    float *st = state + (size_t)vh * D * D + c0 + cl;
+    float S[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) S[i] = st[(size_t)(64 * (i >> 2) + 4 * rg + (i & 3)) * D];
+    // a chunk on its way: tokens t .. t + m - 1
+    float4 nqk[KQ], ng;
+    float nv[VW];
+    auto fetch = [&](int t, int m) {
+#pragma unroll
+        for (int k = 0; k < KQ; k++) {
+            const int w = k * NT + tid, tt = w / (2 * D / 4), c = w % (2 * D / 4) * 4; // q, then k
+            nqk[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (tt < m) nqk[k] = *(const float4 *)(u + (size_t)(t + tt) * C + (c < D ? kh * D + c : qd + kh * D + c - D));
+        }
+#pragma unroll
+        for (int k = 0; k < VW; k++) {
+            const int w = k * NT + tid, tt = w / COLS;
+            nv[k] = tt < m ? u[(size_t)(t + tt) * C + 2 * qd + vh * D + c0 + w % COLS] : 0.0f;
+        }
+        ng = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (tid < m) {
+            const size_t g = (size_t)(t + tid) * n_v + vh;
+            ng = make_float4(decay[g], beta[g], kq[(size_t)(t + tid) * n_k + kh], 0.0f);
+        }
+    };
+    auto store = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < KQ; k++) *(float4 *)(&qk[b][0][0] + 4 * (k * NT + tid)) = nqk[k];
+#pragma unroll
+        for (int k = 0; k < VW; k++) (&vs[b][0][0])[k * NT + tid] = nv[k];
+        if (tid < TC) gs[b][tid] = ng;
+    };
+    struct Ops { // a token's operands
+        float4 q[2], k[2], g;
+        float v;
+    };
+    fetch(0, min(TC, n));
+    store(0);
+    __syncthreads();
+    int b = 0;
+    for (int t0 = 0; t0 < n; t0 += TC) {
+        const int m = min(TC, n - t0);
+        if (t0 + TC < n) {
+            fetch(t0 + TC, min(TC, n - t0 - TC)); // in flight during this chunk's recurrence
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto operands = [&](int t, Ops &o) {
+            t = min(t, m - 1);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                o.q[h] = *(const float4 *)&qk[b][t][64 * h + 4 * rg];
+                o.k[h] = *(const float4 *)&qk[b][t][D + 64 * h + 4 * rg];
+            }
+            o.g = gs[b][t];
+            o.v = vs[b][t][cl];
+        };
+        auto step = [&](const Ops &o, int t) {
+            float p, r;
+            gdn_group(S, o.k, o.q, p, r);
+            p = seg_sum_dpp<16>(p);
+            r = seg_sum_dpp<16>(r);
+            const float dj = gdn_delta(o.v, o.g.x, o.g.y, p);
+            gdn_update(S, o.k, o.g.x, dj);
+            os[t][cl] = gdn_out(dj, o.g.z, o.g.x, r); // (the column's 16 lanes write the same value)
+        };
+        // two sets of operands in turn, each read from LDS a token ahead
+        Ops oa, ob;
+        operands(0, oa);
+        int t = 0;
+        for (; t + 2 <= m; t += 2) {
+            operands(t + 1, ob);
+            step(oa, t);
+            operands(t + 2, oa);
+            step(ob, t + 1);
+        }
+        if (t < m) step(oa, t);
+        if (t0 + TC < n) store(b ^ 1);
+        __syncthreads(); // the chunk's outputs, and the next chunk, are in LDS
+        for (int w = tid; w < m * (COLS / 4); w += NT) {
+            const int tt = w / (COLS / 4), c = w % (COLS / 4) * 4;
+            *(float4 *)(out + (size_t)(t0 + tt) * vd + vh * D + c0 + c) = *(const float4 *)&os[tt][c];
+        }
+        __syncthreads(); // os is rewritten by the next chunk
+        b ^= 1;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) st[(size_t)(64 * (i >> 2) + 4 * rg + (i & 3)) * D] = S[i];
+}
+
+// Wavefront per (token, value head), in place.
+__global__ void __launch_bounds__(256) k_gdn_norm(float *__restrict__ out, const float *__restrict__ z,
+                                                  const float *__restrict__ norm, long heads, float eps)
+{
+    const int lane = threadIdx.x & 63;
+    const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (w >= heads) return;
+    const size_t o = (size_t)w * GDN_D + 2 * lane;
+    *(float2 *)(out + o) = gdn_norm2(*(const float2 *)(out + o), *(const float2 *)(z + o), norm, lane, eps);
 }
 
 const char *gdn_unsupported(size_t n, size_t n_k, size_t n_v, size_t d, size_t kernel)
@@ -159,15 +325,33 @@ const char *gdn_unsupported(size_t n, size_t n_k, size_t n_v, size_t d, size_t k
     return nullptr;
 }
 
+size_t gdn_scratch_floats(size_t n, size_t n_k, size_t n_v) { return n * ((2 * n_k + n_v) * GDN_D + n_k); }
+
 int launch_gdn_block(soso_hip *h, const float *hist, const float *conv, const float *z, const float *decay,
                      const float *beta, const float *norm, float *state, float *out, float *u, int n, int n_k,
                      int n_v, int kernel, float eps)
 {
-    const int C = 2 * n_k * GDN_D + n_v * GDN_D;
-    k_gdn_conv<<<dim3((unsigned)(2 * n_k + n_v), (unsigned)n), GDN_D, 0, h->stream>>>(hist, conv, C, n_k, kernel, eps,
-                                                                                      u);
+    float *kq = u + (size_t)n * (2 * n_k + n_v) * GDN_D;
+    const unsigned cg = (unsigned)(((long)(n_k + n_v) * n + 3) / 4);
+#define GDN_CONV(KW) k_gdn_conv<KW><<<cg, 256, 0, h->stream>>>(hist, conv, n, n_k, n_v, kernel, eps, u, kq)
+    switch (kernel) {
+    case 1: GDN_CONV(1); break;
+    case 2: GDN_CONV(2); break;
+    case 3: GDN_CONV(3); break;
+    case 4: GDN_CONV(4); break;
+    default: GDN_CONV(0); break;
+    }
+#undef GDN_CONV
     int rc = hip_check(h, hipGetLastError(), "gdn conv launch");
     if (rc != SOSO_HIP_OK) return rc;
-    k_gdn_rec<<<(unsigned)n_v, GDN_D * GDN_RG, 0, h->stream>>>(u, z, decay, beta, norm, state, out, n, n_k, n_v, eps);
-    return hip_check(h, hipGetLastError(), "gdn recurrence launch");
+    if (n <= GDN_FEW) {
+        k_gdn_rec_few<<<(unsigned)n_v, 1024, 0, h->stream>>>(u, kq, z, decay, beta, norm, state, out, n, n_k, n_v, eps);
+        return hip_check(h, hipGetLastError(), "gdn recurrence launch");
+    }
+    k_gdn_rec<<<(unsigned)n_v * (GDN_D / 16), 256, 0, h->stream>>>(u, kq, decay, beta, state, out, n, n_k, n_v);
+    rc = hip_check(h, hipGetLastError(), "gdn recurrence launch");
+    if (rc != SOSO_HIP_OK) return rc;
+    const long heads = (long)n * n_v;
+    k_gdn_norm<<<(unsigned)((heads + 3) / 4), 256, 0, h->stream>>>(out, z, norm, heads, eps);
+    return hip_check(h, hipGetLastError(), "gdn norm launch");
 }

@@ -495,8 +495,8 @@ int soso_hip_gdn_block(soso_hip *h, const float *hist, const float *conv, const 
     CallClock clk(h);
     const size_t C = (2 * n_k + n_v) * d, vd = n_v * d;
     // one device buffer, 256-byte aligned pieces: the inputs, the state, the
-    // output and the conv/normalisation result u
-    const size_t sz[] = {(kernel - 1 + n) * C, C * kernel, n * vd, n * n_v, n * n_v, d, n_v * d * d, n * vd, n * C};
+    // output and the launches' scratch
+    const size_t sz[] = {(kernel - 1 + n) * C, C * kernel, n * vd, n * n_v, n * n_v, d, n_v * d * d, n * vd, gdn_scratch_floats(n, n_k, n_v)};
     size_t off[9], total = 0;
     for (int i = 0; i < 9; i++) {
         off[i] = total;
@@ -536,7 +536,7 @@ int soso_hip_gdn_block_dev(soso_hip *h, const float *hist, const float *conv, co
     if (rc != SOSO_HIP_OK) return rc;
     rc = make_current(h);
     if (rc != SOSO_HIP_OK) return rc;
-    float *u = (float *)scratch_get(h, 4, n * (2 * n_k + n_v) * d * 4);
+    float *u = (float *)scratch_get(h, 4, gdn_scratch_floats(n, n_k, n_v) * 4);
     if (!u) return set_err(h, SOSO_HIP_ERR_NOMEM, "gdn_block_dev: scratch (or growing it during capture)");
     return launch_gdn_block(h, hist, conv, z, decay, beta, norm, state, out, u, (int)n, (int)n_k, (int)n_v,
                             (int)kernel, eps);

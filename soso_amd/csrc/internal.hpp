@@ -81,6 +81,7 @@ struct MoeScratch {
     int *recs = nullptr, *n_recs = nullptr;   // active groups {group, count, first slot, 0} (ascending), count
     float *act = nullptr;    // n x top_k x ffn
     float *ydown = nullptr;  // n x top_k x hdim
+    bool fixed = false;      // the library's fixed array: the call may take no other scratch
 };
 
 struct DecodeLayer {
@@ -314,6 +315,9 @@ int launch_mfma_matmul(soso_hip *h, const Weight &w, const float *x, size_t n, f
 // are the faster ones for a shape, and their launch (DECLINED: no scratch)
 bool gemm_wins(uint8_t dtype, size_t rows, size_t cols, size_t n);
 int launch_gemm(soso_hip *h, const Weight &w, const float *x, size_t n, float *y);
+int launch_gemm_moe(soso_hip *h, int nmat, const uint8_t *const *tiled, const uint8_t *const *row_major, size_t n_groups,
+                    size_t rows, size_t cols, size_t slots, size_t max_recs, const float *xs, size_t n, int xdiv,
+                    const int *list, const int *recs, const int *n_recs, bool fixed, float *out);
 size_t moe_max_items(const soso_hip *h, size_t slots, size_t n_groups);
 int launch_router_topk(soso_hip *h, const float *w_dev, const float *x_dev, size_t n, size_t hdim,
                        size_t n_exp, size_t top_k, int32_t *idx_dev, float *wgt_dev, float *logits_dev);

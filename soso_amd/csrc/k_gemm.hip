@@ -42,7 +42,7 @@ typedef float gm_f16v __attribute__((ext_vector_type(16)));
 typedef uint32_t gm_u4 __attribute__((ext_vector_type(4))); // (a HIP uint4 array here ends up in scratch memory)
 
 // Staged x, for tiles of 32 tokens (rows past n are zeros):
-//   F [tile][unit][step 4][hi, lo][lane 64][16 B]   8 KiB per unit
+//   F [tile][unit][step 4][hi, lo][half f][32 x 16 B]   8 KiB per unit
 //   M [tile][super-block][lane 64][16 B]            eight sub-block sums, hi (f = 0) and lo (f = 1)
 //   P [tile][super-block][32] f32                   2^-s per token
 struct GmX {
@@ -50,6 +50,22 @@ struct GmX {
     const float *p;
 };
 constexpr int GM_UNIT = 8192, GM_SUMS = 1024;
+
+// Where x is written to LDS token by token, token m's 16 bytes of a piece sit at
+// place m ^ gm_swz(unit, step, lo): a token's pieces would else all meet in the
+// same banks (two thirds of the LDS cycles of a MoE layer of 512 tokens, gate /
+// up 123 -> 98 us).  The 16 places that span the banks are distinct over the
+// units and steps of one token (gm_stage_rows), and, with bit 0 of the token,
+// over the steps and parts of one unit (the MoE kernel's gather).
+__device__ __forceinline__ constexpr int gm_swz(int unit, int step, int lo)
+{
+    return 4 * step + 2 * (lo ^ ((unit >> 1) & 1)) + (unit & 1);
+}
+// Lane (n, f)'s fragment of a unit written so (x: its 8 KiB in LDS).
+__device__ __forceinline__ gm_h8 gm_frag_at(const uint8_t *x, int lane, int unit, int step, int lo)
+{
+    return *(const gm_h8 *)(x + step * 2048 + lo * 1024 + ((16 * lane) ^ (16 * gm_swz(unit, step, lo))));
+}
 
 __device__ __forceinline__ uint32_t gm_pack(float a, float b)
 {
@@ -89,12 +105,24 @@ __device__ __forceinline__ float gm_outlier_thr(gm_f4 v)
     return third > 0.0f ? 16384.0f * third : INFINITY;
 }
 
-// One token's 256 columns (four per lane) as a tile's row m: the fragments of
-// its four units at xf, the sub-blocks' sums at xm (Q4_K) and 2^-s.  c8, this
-// lane's group of eight columns, sits in unit u, step st, half f.
-template <int FMT>
-__device__ __forceinline__ void gm_stage_row(gm_f4 v, int lane, int m, uint8_t *xf, uint8_t *xm, float *xp)
+// Where the pieces of a token's 256 columns go: as a row of a 32-token tile
+// (above), or for TOK token by token -- unit u at 256 u, then step, hi / lo,
+// half f of 16 bytes each; sums hi, then lo.
+template <bool TOK> struct GmPlace {
+    static constexpr int UNIT = TOK ? 256 : GM_UNIT, STEP = TOK ? 64 : 2048, LO = TOK ? 32 : 1024, HALF = TOK ? 16 : 512;
+    static constexpr int SUM_LO = TOK ? 16 : 512;
+};
+constexpr int GM_TOK = 1024, GM_TOK_SUMS = 32; // bytes per token and super-block, TOK
+
+// 256 columns of R tokens (four per lane and token, v[k]) in f16 parts: the
+// fragments at xf(k), the sub-blocks' sums at xm(k) (Q4_K) and 2^-s at xp(k), for
+// the tokens k < count.  The tokens' steps interleave: one token after another
+// left each with the latency of a dozen dependent lane moves.
+// row(k): the token's row of its tile (not TOK).
+template <int FMT, int R, bool TOK, class Row, class XF, class XM, class XP>
+__device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count, Row row, XF xf, XM xm, XP xp)
 {
+    // this lane's group of eight columns: unit u, step st, half f
     const int c8 = lane >> 1;
     int u, st, f;
     if constexpr (FMT == FMT_Q6K) {
@@ -106,62 +134,107 @@ __device__ __forceinline__ void gm_stage_row(gm_f4 v, int lane, int m, uint8_t *
         st = 2 * ((c8 >> 2) & 1) + (c8 & 1);
         f = (c8 >> 1) & 1;
     }
-    uint8_t *dst = xf + u * GM_UNIT + st * 2048 + f * 512 + 8 * (lane & 1) + 16 * m;
-    float mx = gm_abs_max(v);
-    float sm = (v[0] + v[1]) + (v[2] + v[3]);
-    if (sm != sm) mx = INFINITY; // a NaN element (or Inf - Inf): the block is non-finite
+    using P = GmPlace<TOK>;
+    const int at = u * P::UNIT + st * P::STEP + f * P::HALF + 8 * (lane & 1);
+    auto st_max = [](float a, uint32_t b) { return fmaxf(a, __uint_as_float(b)); };
+    auto st_min = [](float a, uint32_t b) { return fminf(a, __uint_as_float(b)); };
+    float mx[R], mn[R], sm[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        mx[k] = gm_abs_max(v[k]);
+        sm[k] = (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+        if (sm[k] != sm[k]) mx[k] = INFINITY; // a NaN element (or Inf - Inf): the block is non-finite
+    }
     // the maximum over the wavefront and the smallest maximum of its 32-column
     // groups: within 2^14 of each other, no element is an outlier (the two
     // largest 8-column maxima sit in at most two groups of each 128)
-    auto st_max = [](float a, uint32_t b) { return fmaxf(a, __uint_as_float(b)); };
-    auto st_min = [](float a, uint32_t b) { return fminf(a, __uint_as_float(b)); };
-    mx = st_max(mx, dpp_keep<0xB1>(__float_as_uint(mx)));
-    mx = st_max(mx, dpp_keep<0x4E>(__float_as_uint(mx)));
-    mx = st_max(mx, dpp_keep<0x141>(__float_as_uint(mx)));
-    float mn = st_min(mx, dpp_keep<0x140>(__float_as_uint(mx)));
-    mx = st_max(mx, dpp_keep<0x140>(__float_as_uint(mx)));
-    mn = st_min(mn, dpp_keep<0x142, 0xA>(__float_as_uint(mn)));
-    mx = st_max(mx, dpp_keep<0x142, 0xA>(__float_as_uint(mx)));
-    mn = st_min(mn, dpp_keep<0x143, 0xC>(__float_as_uint(mn)));
-    mx = st_max(mx, dpp_keep<0x143, 0xC>(__float_as_uint(mx)));
-    mn = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mn), 63));
-    mx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx), 63));
-    const bool finite = mx < INFINITY;
-    bool out = false;
-    if (__builtin_expect(finite && mx > 16384.0f * mn, 0)) { // uniform
-        const float thr = gm_outlier_thr(v);
-        bool mine = false;
+#define GM_STEP(C, ROWS)                                                                                               \
+    _Pragma("unroll") for (int k = 0; k < R; k++) mx[k] = st_max(mx[k], dpp_keep<C, ROWS>(__float_as_uint(mx[k])));
+    GM_STEP(0xB1, 0xf)
+    GM_STEP(0x4E, 0xf)
+    GM_STEP(0x141, 0xf)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (fabsf(v[i]) > thr) {
-                v[i] = 0.0f;
-                mine = true;
+    for (int k = 0; k < R; k++) mn[k] = mx[k];
+#define GM_STEP2(C, ROWS)                                                                                              \
+    GM_STEP(C, ROWS)                                                                                                   \
+    _Pragma("unroll") for (int k = 0; k < R; k++) mn[k] = st_min(mn[k], dpp_keep<C, ROWS>(__float_as_uint(mn[k])));
+    GM_STEP2(0x140, 0xf)
+    GM_STEP2(0x142, 0xA)
+    GM_STEP2(0x143, 0xC)
+#undef GM_STEP2
+#undef GM_STEP
+    bool odd = false;
+    float sign[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        mx[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[k]), 63));
+        mn[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mn[k]), 63));
+        sign[k] = 1.0f;
+        odd = odd || !(mx[k] <= 16384.0f * mn[k]) || !(mx[k] < INFINITY);
+    }
+    if (__builtin_expect(odd, 0)) { // uniform; rare
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            if (!(mx[k] < INFINITY)) {
+                v[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
+                mx[k] = sm[k] = 0.0f;
+                sign[k] = __builtin_nanf("");
+            } else if (mx[k] > 16384.0f * mn[k]) {
+                const float thr = gm_outlier_thr(v[k]);
+                bool mine = false;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (fabsf(v[k][i]) > thr) {
+                        v[k][i] = 0.0f;
+                        mine = true;
+                    }
+                if (__ballot(mine) != 0) sign[k] = -1.0f;
+                mx[k] = wave_max_dpp(gm_abs_max(v[k]));
+                sm[k] = (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
             }
-        out = __ballot(mine) != 0;
-        mx = wave_max_dpp(gm_abs_max(v));
-        sm = (v[0] + v[1]) + (v[2] + v[3]);
-    }
-    const int s = mx > 0.0f && finite ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
-    float e[4], lo[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        e[i] = finite ? ldexpf(v[i], s) : 0.0f;
-        lo[i] = e[i] - (float)(_Float16)e[i];
-    }
-    *(uint2 *)dst = make_uint2(gm_pack(e[0], e[2]), gm_pack(e[1], e[3]));
-    *(uint2 *)(dst + 1024) = make_uint2(gm_pack(lo[0], lo[2]), gm_pack(lo[1], lo[3]));
-    if constexpr (FMT == FMT_Q4K) {
-        // the sub-block's sum (8 lanes), scaled by 2^(s - 5): at most 2^15
-        sm = seg_sum_dpp<8>(sm);
-        if ((lane & 7) == 0) {
-            const float q = finite ? ldexpf(sm, s - 5) : 0.0f;
-            const _Float16 hi = (_Float16)q;
-            _Float16 *d = (_Float16 *)xm + 8 * m + (lane >> 3);
-            d[0] = hi;
-            d[256] = (_Float16)(q - (float)hi);
         }
     }
-    if (lane == 0) *xp = !finite ? __builtin_nanf("") : out ? -ldexpf(1.0f, -s) : ldexpf(1.0f, -s);
+    int s[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        s[k] = 15 - __builtin_amdgcn_frexp_expf(mx[k]);
+        float e[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            e[i] = ldexpf(v[k][i], s[k]);
+            lo[i] = e[i] - (float)(_Float16)e[i];
+        }
+        if (k < count) { // uniform
+            uint8_t *hd = xf(k) + at, *ld = hd + P::LO;
+            if constexpr (!TOK) {
+                hd += 16 * (row(k) ^ gm_swz(u, st, 0));
+                ld += 16 * (row(k) ^ gm_swz(u, st, 1));
+            }
+            *(uint2 *)hd = make_uint2(gm_pack(e[0], e[2]), gm_pack(e[1], e[3]));
+            *(uint2 *)ld = make_uint2(gm_pack(lo[0], lo[2]), gm_pack(lo[1], lo[3]));
+        }
+    }
+    if constexpr (FMT == FMT_Q4K) {
+        // the sub-blocks' sums (8 lanes), scaled by 2^(s - 5): at most 2^15
+#pragma unroll
+        for (int k = 0; k < R; k++) sm[k] = seg_sum_dpp<8>(sm[k]);
+        if ((lane & 7) == 0) {
+#pragma unroll
+            for (int k = 0; k < R; k++)
+                if (k < count) {
+                    const float q = ldexpf(sm[k], s[k] - 5);
+                    const _Float16 hi = (_Float16)q;
+                    uint8_t *d = xm(k) + 2 * (lane >> 3);
+                    *(_Float16 *)d = hi;
+                    *(_Float16 *)(d + P::SUM_LO) = (_Float16)(q - (float)hi);
+                }
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < R; k++)
+            if (k < count) *xp(k) = sign[k] * ldexpf(1.0f, -s[k]);
+    }
 }
 
 // One workgroup per (32-token tile, super-block): eight wavefronts of four
@@ -183,16 +256,43 @@ __global__ void __launch_bounds__(512) k_gm_stage(const float *__restrict__ x, i
         v[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
         if (in && t < n) v[k] = *(const gm_f4 *)(x + (size_t)t * cols + 256 * sb + 4 * lane);
     }
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-        gm_stage_row<FMT>(v[k], lane, 4 * wave + k, (uint8_t *)frag, (uint8_t *)sums,
-                          xp + (size_t)blockIdx.x * 32 + 4 * wave + k);
+    gm_stage_rows<FMT, 4, false>(
+        v, lane, 4, [&](int k) { return 4 * wave + k; }, [&](int) { return (uint8_t *)frag; },
+        [&](int k) { return (uint8_t *)sums + 16 * (4 * wave + k); },
+        [&](int k) { return xp + (size_t)blockIdx.x * 32 + 4 * wave + k; });
     __syncthreads();
     uint4 *of = (uint4 *)(xf + (size_t)blockIdx.x * (4 * GM_UNIT));
 #pragma unroll
-    for (int i = 0; i < 4; i++) of[i * 512 + threadIdx.x] = frag[i * 512 + threadIdx.x];
+    for (int i = 0; i < 4; i++) {
+        const int w = i * 512 + threadIdx.x, pc = (w >> 5) & 15; // unit i, piece pc (step, part, half), token w % 32
+        of[w] = frag[w ^ gm_swz(i, pc >> 2, (pc >> 1) & 1)];
+    }
     if (FMT == FMT_Q4K && threadIdx.x < 64)
         ((uint4 *)(xm + (size_t)blockIdx.x * GM_SUMS))[threadIdx.x] = sums[threadIdx.x];
+}
+
+// The same token by token (rows whose tiles are not known yet): four rows of
+// one super-block per wavefront.  F [row][super-block][GM_TOK], M [row][super-
+// block][GM_TOK_SUMS], P [row][super-block].
+__global__ void __launch_bounds__(256) k_gm_stage_tok(const float *__restrict__ x, int n, int cols,
+                                                      uint8_t *__restrict__ xf, uint8_t *__restrict__ xm,
+                                                      float *__restrict__ xp)
+{
+    const int nb = cols >> 8, lane = threadIdx.x & 63;
+    const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int sb = (int)(w % nb);
+    const long t0 = w / nb * 4;
+    if (t0 >= n) return; // no barriers here
+    gm_f4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        v[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
+        if (t0 + k < n) v[k] = *(const gm_f4 *)(x + (size_t)(t0 + k) * cols + 256 * sb + 4 * lane);
+    }
+    auto at = [&](int k) { return (size_t)(t0 + k) * nb + sb; };
+    gm_stage_rows<FMT_Q4K, 4, true>(
+        v, lane, (int)min(4l, n - t0), [&](int) { return 0; }, [&](int k) { return xf + at(k) * GM_TOK; },
+        [&](int k) { return xm + at(k) * GM_TOK_SUMS; }, [&](int k) { return xp + at(k); });
 }
 
 // (typedefs of the compiler's own vectors: a HIP uint4 array that a lambda
@@ -249,53 +349,20 @@ __device__ __forceinline__ void gm_swap32(gm_u4 &a, gm_u4 &b)
 template <int FMT, int SETS>
 struct GmW;
 
-template <int SETS>
-struct GmW<FMT_Q4K, SETS> {
+// A half super-block of Q4_K as the operands take it.
+struct GmQ4K {
     static constexpr int PARTS = 1; // operands per step (hi, and lo where a weight needs two f16)
-    gm_u4 L[SETS][2][2], hn;
-    gm_u4 q[2][2]; // [rows 32 j][unit]: the 16 code bytes of plane f
+    gm_u4 q[2][2];                  // [rows 32 j][unit]: the 16 code bytes of plane f
     uint32_t sc4[2][2], m4[2][2], dd[2];
-    uint32_t off_h, off_q, row32, plane;
-    __device__ __forceinline__ void init(int row, int lane, size_t stride, int U)
-    {
-        const int nb = U >> 2;
-        off_h = (uint32_t)((row + lane) * stride);
-        off_q = (uint32_t)((row + (lane & 31)) * stride) + 16u * (uint32_t)(nb + (lane >> 5));
-        row32 = (uint32_t)(32 * stride);
-        plane = 64u * (uint32_t)nb;
-    }
-    __device__ __forceinline__ void head_load(rsrc_t rs, int sb) { hn = gm_ld(rs, off_h + 16u * (uint32_t)sb); }
-    __device__ __forceinline__ void load(rsrc_t rs, int half, int set)
-    {
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int k = 0; k < 2; k++)
-                L[set][j][k] = gm_ld(rs, off_q + (uint32_t)j * row32 + (uint32_t)k * plane + 32u * (uint32_t)half);
-    }
     // the scales of a super-block's eight sub-blocks (get_scale_min_k4,
     // dequant.rs:150-159), four per dword
-    __device__ __forceinline__ void head()
+    __device__ __forceinline__ void scales(gm_u4 h, int j)
     {
-        gm_u4 h[2] = {hn, hn};
-        gm_swap32(h[0], h[1]);
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            dd[j] = h[j][0];
-            sc4[j][0] = h[j][1] & 0x3F3F3F3Fu;
-            m4[j][0] = h[j][2] & 0x3F3F3F3Fu;
-            sc4[j][1] = (h[j][3] & 0x0F0F0F0Fu) | ((h[j][1] >> 2) & 0x30303030u);
-            m4[j][1] = ((h[j][3] >> 4) & 0x0F0F0F0Fu) | ((h[j][2] >> 2) & 0x30303030u);
-        }
-    }
-    __device__ __forceinline__ void split(int, int set)
-    {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            q[j][0] = L[set][j][0];
-            q[j][1] = L[set][j][1];
-            gm_swap32(q[j][0], q[j][1]);
-        }
+        dd[j] = h[0];
+        sc4[j][0] = h[1] & 0x3F3F3F3Fu;
+        m4[j][0] = h[2] & 0x3F3F3F3Fu;
+        sc4[j][1] = (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u);
+        m4[j][1] = ((h[3] >> 4) & 0x0F0F0F0Fu) | ((h[2] >> 2) & 0x30303030u);
     }
     // Step t of unit v of half i.  A masked nibble q is the subnormal f16 q
     // 2^-24 (16 q 2^-24 where the high nibbles stay in place) and its product
@@ -317,6 +384,45 @@ struct GmW<FMT_Q4K, SETS> {
         const gm_h2 k = gm_dup(1024.0f);
         return gm_join(gm_bytes<0, 1>(m4[j][0]) - k, gm_bytes<2, 3>(m4[j][0]) - k, gm_bytes<0, 1>(m4[j][1]) - k,
                        gm_bytes<2, 3>(m4[j][1]) - k);
+    }
+};
+
+template <int SETS>
+struct GmW<FMT_Q4K, SETS> : GmQ4K {
+    gm_u4 L[SETS][2][2], hn;
+    uint32_t off_h, off_q, row32, plane;
+    __device__ __forceinline__ void init(int row, int lane, size_t stride, int U)
+    {
+        const int nb = U >> 2;
+        off_h = (uint32_t)((row + lane) * stride);
+        off_q = (uint32_t)((row + (lane & 31)) * stride) + 16u * (uint32_t)(nb + (lane >> 5));
+        row32 = (uint32_t)(32 * stride);
+        plane = 64u * (uint32_t)nb;
+    }
+    __device__ __forceinline__ void head_load(rsrc_t rs, int sb) { hn = gm_ld(rs, off_h + 16u * (uint32_t)sb); }
+    __device__ __forceinline__ void load(rsrc_t rs, int half, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                L[set][j][k] = gm_ld(rs, off_q + (uint32_t)j * row32 + (uint32_t)k * plane + 32u * (uint32_t)half);
+    }
+    __device__ __forceinline__ void head()
+    {
+        gm_u4 h[2] = {hn, hn};
+        gm_swap32(h[0], h[1]);
+        scales(h[0], 0);
+        scales(h[1], 1);
+    }
+    __device__ __forceinline__ void split(int, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            q[j][0] = L[set][j][0];
+            q[j][1] = L[set][j][1];
+            gm_swap32(q[j][0], q[j][1]);
+        }
     }
 };
 
@@ -490,36 +596,35 @@ __device__ float gm_weight(const uint8_t *__restrict__ row, int c, int U)
     }
 }
 
-// The products of the elements that the staging took out of tokens t0 .. t0 +
-// nt - 1 in super-blocks sb0 .. sb1 - 1, found again by the same rule, into the
-// sums of this lane's rows r and r + 32 (the tile's token t is register 4 (t /
-// 8) + t % 4 of half t / 4 % 2).  Rare: kept out of the streaming loop.
-template <int FMT>
-__device__ __forceinline__ void gm_add_outliers(gm_f16v (&acc)[2], const uint8_t *__restrict__ W, size_t stride,
-                                                int rows, int cols, int r, const float *__restrict__ x, int nt, int sb0,
-                                                int sb1)
+// The products of the elements that the staging took out of a tile's tokens 0
+// .. nt - 1 (x rows xrow(t)) in super-blocks sb0 .. sb1 - 1, found again by the
+// same rule, into the sums of this lane's two weight rows w0 and w1 (null: past
+// the matrix).  Token t of the tile is register 4 (t / 8) + t % 4 of half t / 4
+// % 2.  Rare: kept out of the streaming loop.
+template <int FMT, class XRow>
+__device__ __forceinline__ void gm_add_outliers(gm_f16v (&acc)[2], const uint8_t *w0, const uint8_t *w1, int cols,
+                                                XRow xrow, int nt, int sb0, int sb1)
 {
     const int lane = threadIdx.x & 63;
     for (int sb = sb0; sb < sb1; sb++)
         for (int t = 0; t < nt; t++) {
             gm_f4 v = {0.f, 0.f, 0.f, 0.f};
-            if (256 * sb + 4 * lane < cols) v = *(const gm_f4 *)(x + (size_t)t * cols + 256 * sb + 4 * lane);
-            if (__ballot(!(gm_abs_max(v) < INFINITY) || v[0] + v[1] + v[2] + v[3] != v[0] + v[1] + v[2] + v[3]))
-                continue; // a non-finite block: every output is NaN already
+            if (256 * sb + 4 * lane < cols) v = *(const gm_f4 *)(xrow(t) + 256 * sb + 4 * lane);
+            const float sm = (v[0] + v[1]) + (v[2] + v[3]);
+            if (__ballot(!(gm_abs_max(v) < INFINITY) || sm != sm)) continue; // non-finite: every output is NaN already
             const float thr = gm_outlier_thr(v);
+            const bool mine = ((t >> 2) & 1) == lane >> 5;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 uint64_t todo = __ballot(fabsf(v[i]) > thr);
                 while (todo) { // uniform
-                    const int src = __builtin_ctzll(todo);
+                    const int src = __builtin_ctzll(todo), c = 256 * sb + 4 * src + i;
                     todo &= todo - 1;
                     const float xv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[i]), src));
-                    const int c = 256 * sb + 4 * src + i;
-                    const bool mine = ((t >> 2) & 1) == lane >> 5;
 #pragma unroll
                     for (int j = 0; j < 2; j++) {
-                        const int row = r + 32 * j;
-                        const float p = mine && row < rows ? gm_weight<FMT>(W + (size_t)row * stride, c, cols >> 6) * xv : 0.0f;
+                        const uint8_t *w = j ? w1 : w0;
+                        const float p = mine && w ? gm_weight<FMT>(w, c, cols >> 6) * xv : 0.0f;
 #pragma unroll
                         for (int k = 0; k < 16; k++)
                             if (k == 4 * (t >> 3) + (t & 3)) acc[j][k] += p;
@@ -707,9 +812,10 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
     if (__builtin_expect(taken != 0, 0)) {
 #pragma unroll
         for (int m = 0; m < MT; m++) {
-            const int t0 = 32 * (tt * MT + m);
-            gm_add_outliers<FMT>(acc[m], W, stride, rows, cols, r0 + 64 * wave + nl, xs32 + (size_t)t0 * cols,
-                                 min(32, n - t0), sb0, sb1);
+            const int t0 = 32 * (tt * MT + m), r = r0 + 64 * wave + nl;
+            gm_add_outliers<FMT>(
+                acc[m], r < rows ? W + (size_t)r * stride : nullptr, r + 32 < rows ? W + (size_t)(r + 32) * stride : nullptr,
+                cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1);
         }
     }
     float *o = out + (size_t)sp * n * rows;
@@ -758,22 +864,27 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
     __shared__ gm_u4 xs[2][4 * GM_UNIT / 16];
     __shared__ gm_u4 ms[2][SUMS / 16];
     __shared__ float ps[2][32];
-    // tokens wave + 4 k: a lane's four columns of each
-    gm_f4 xv[8];
+    // tokens wave + 4 k, k = 4 g + i: a lane's four columns of each
+    gm_f4 xv[2][4];
     const int tmax = (n - wave + 3) >> 2; // this wavefront's tokens
     auto load_x = [&](int sb) {
         const bool in = 256 * sb + 4 * lane < cols;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            xv[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
-            if (k < tmax && in) xv[k] = *(const gm_f4 *)(x + (size_t)(wave + 4 * k) * cols + 256 * sb + 4 * lane);
+            xv[k >> 2][k & 3] = gm_f4{0.f, 0.f, 0.f, 0.f};
+            if (k < tmax && in)
+                xv[k >> 2][k & 3] = *(const gm_f4 *)(x + (size_t)(wave + 4 * k) * cols + 256 * sb + 4 * lane);
         }
     };
     auto store_x = [&](int b) {
 #pragma unroll
-        for (int k = 0; k < 8; k++)
-            if (k < tmax)
-                gm_stage_row<FMT>(xv[k], lane, wave + 4 * k, (uint8_t *)xs[b], (uint8_t *)ms[b], &ps[b][wave + 4 * k]);
+        for (int g = 0; g < 2; g++)
+            if (4 * g < tmax) // uniform
+                gm_stage_rows<FMT, 4, false>(
+                    xv[g], lane, tmax - 4 * g, [&](int k) { return wave + 16 * g + 4 * k; },
+                    [&](int) { return (uint8_t *)xs[b]; },
+                    [&](int k) { return (uint8_t *)ms[b] + 16 * (wave + 16 * g + 4 * k); },
+                    [&](int k) { return &ps[b][wave + 16 * g + 4 * k]; });
     };
     load_x(sb0);
     __builtin_amdgcn_sched_barrier(0);
@@ -795,6 +906,12 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
         const int cur = (sb - sb0) & 1, sn = min(sb + 1, sb1 - 1);
         wt.head();
         wt.head_load(rs, sn);
+        // a step's x is read from LDS a step ahead, where the registers hold it
+        constexpr bool AHEAD = FMT == FMT_Q4K;
+        const uint8_t *xb = (const uint8_t *)xs[cur];
+        gm_h8 ah[2], al[2];
+        ah[0] = gm_frag_at(xb, lane, 0, 0, 0);
+        al[0] = gm_frag_at(xb, lane, 0, 0, 1);
 #pragma unroll
         for (int p = 0; p < 4; p++) {
             if (!(p & 1)) {
@@ -802,13 +919,17 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
                 wt.load(rs, 2 * sn + (p >> 1), p >> 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            const uint8_t *xb = (const uint8_t *)xs[cur] + p * GM_UNIT + 16 * lane;
 #pragma unroll
             for (int t = 0; t < 4; t++) {
+                const int i1 = 4 * p + t + (AHEAD ? 1 : 0);
+                if (i1 < 16) {
+                    ah[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, lane, i1 >> 2, i1 & 3, 0);
+                    al[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, lane, i1 >> 2, i1 & 3, 1);
+                }
                 gm_h8 b[2][PARTS];
 #pragma unroll
                 for (int j = 0; j < 2; j++) wt.frag(p >> 1, p & 1, t, j, b[j]);
-                const gm_h8 hi = *(const gm_h8 *)(xb + t * 2048), lo = *(const gm_h8 *)(xb + t * 2048 + 1024);
+                const gm_h8 hi = ah[t & 1], lo = al[t & 1];
                 const bool first = p == 0 && t == 0;
 #pragma unroll
                 for (int j = 0; j < 2; j++)
@@ -851,8 +972,12 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
             __syncthreads();
         }
     }
-    if (__builtin_expect(taken != 0, 0))
-        gm_add_outliers<FMT>(acc, W, stride, rows, cols, r0 + 64 * wave + nl, x, n, sb0, sb1);
+    if (__builtin_expect(taken != 0, 0)) {
+        const int r = r0 + 64 * wave + nl;
+        gm_add_outliers<FMT>(
+            acc, r < rows ? W + (size_t)r * stride : nullptr, r + 32 < rows ? W + (size_t)(r + 32) * stride : nullptr,
+            cols, [&](int t) { return x + (size_t)t * cols; }, n, sb0, sb1);
+    }
     float *o = out + ((size_t)sp * n_all + 32 * tt) * rows;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
@@ -861,6 +986,280 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
         for (int i = 0; i < 16; i++) {
             const int t = 8 * (i >> 2) + 4 * f + (i & 3);
             if (t < n && row < rows) o[(size_t)t * rows + row] = acc[j][i];
+        }
+    }
+}
+
+// Tile-major Q4_K (the registered MoE experts' copies, tile_q4k in k_mfma.hip:
+// per 16-row tile and super-block the rows' headers, then lane 16 g + n's 8 code
+// bytes 8 g of row n of units 0 and 1, then of 2 and 3).  Lane (n, f) of a
+// 32-row tile takes k-groups 2 f and 2 f + 1 of its row: contiguous loads, no
+// swaps.  base: the wavefront's first row of both 32-row tiles.
+template <int SETS>
+struct GmTiled : GmQ4K {
+    gm_u4 L[SETS][2][2], hn[2];
+    uint32_t off[2], sbs;
+    __device__ __forceinline__ void init(int row0, int row1, int lane, int nb)
+    {
+        const uint32_t nl = (uint32_t)(lane & 31);
+        sbs = 2304u;
+        off[0] = ((uint32_t)(row0 >> 4) + (nl >> 4)) * (uint32_t)nb * sbs + 16u * (nl & 15);
+        off[1] = ((uint32_t)(row1 >> 4) + (nl >> 4)) * (uint32_t)nb * sbs + 16u * (nl & 15);
+        g = 512u * (uint32_t)(lane >> 5) + 256u;
+    }
+    uint32_t g;
+    __device__ __forceinline__ void head_load(const rsrc_t (&rs)[2], int sb)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++) hn[j] = gm_ld(rs[j], off[j] + sbs * (uint32_t)sb);
+    }
+    __device__ __forceinline__ void load(const rsrc_t (&rs)[2], int half, int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                L[set][j][k] = gm_ld(rs[j], off[j] + g + sbs * (uint32_t)(half >> 1) + 1024u * (uint32_t)(half & 1) +
+                                                256u * (uint32_t)k);
+    }
+    __device__ __forceinline__ void head()
+    {
+        scales(hn[0], 0);
+        scales(hn[1], 1);
+    }
+    __device__ __forceinline__ void split(int set)
+    {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const gm_u4 a = L[set][j][0], b = L[set][j][1];
+            q[j][0] = gm_u4{a[0], a[1], b[0], b[1]};
+            q[j][1] = gm_u4{a[2], a[3], b[2], b[3]};
+        }
+    }
+};
+
+// The MoE experts of a prompt's tokens (gate / up 303 -> 98 us, down 118 -> 63
+// for 512 tokens of 128 experts of 2048 x 768 at top-8, 0.22 and 0.17 PFLOP/s;
+// the integer kernel's workgroups converted eight tokens at a time and decoded
+// each weight once per eight): k_gemm_few over (tile of 32 slots of an
+// active expert, row block), x gathered by the slot list (x row = slot / xdiv,
+// output row = slot).  NMAT 2: 128 rows of gate and of up side by side, the
+// output silu(gate) * up (gemm.rs:210-226); NMAT 1: 256 rows of down.
+// recs[4 a ..] = {expert, slots, first slot in list, 0}, at most 256 of them;
+// tab*: tile-major experts, row*: the same row-major (for the outliers).
+// STAGED: x's rows come in f16 parts (k_gm_stage_tok); else every workgroup
+// converts its tokens, to the same bits.
+template <int NMAT, bool STAGED>
+__global__ void __launch_bounds__(256, 2)
+    k_gemm_moe(const uint8_t *const *__restrict__ tabA, const uint8_t *const *__restrict__ tabB,
+               const uint8_t *const *__restrict__ rowA, const uint8_t *const *__restrict__ rowB, size_t stride, int rows,
+               int cols, const float *__restrict__ xs, GmX xg, int xdiv, const int *__restrict__ list,
+               const int *__restrict__ recs, const int *__restrict__ n_recs, int nblk, float *__restrict__ out)
+{
+    __shared__ int it_s[4];
+    __shared__ int slot_s[32];
+    const int lane = threadIdx.x & 63, f = lane >> 5, nl = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int item = (int)blockIdx.x / nblk, rb = (int)blockIdx.x % nblk;
+    if (wave == 0) {
+        // the record whose tiles hold this item: a scan over the records'
+        // tile counts, four per lane
+        const int nr = *n_recs;
+        int c[4], tot = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            c[k] = 4 * lane + k < nr ? recs[4 * (4 * lane + k) + 1] : 0;
+            tot += (c[k] + 31) >> 5;
+        }
+        int incl = tot;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        if (lane == 63 && item >= incl) it_s[0] = -1;
+        int run = incl - tot;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int t = (c[k] + 31) >> 5;
+            if (item >= run && item < run + t) {
+                it_s[0] = recs[4 * (4 * lane + k)];
+                it_s[1] = c[k] - 32 * (item - run);
+                it_s[2] = recs[4 * (4 * lane + k) + 2] + 32 * (item - run);
+            }
+            run += t;
+        }
+    }
+    __syncthreads();
+    const int e = __builtin_amdgcn_readfirstlane(it_s[0]);
+    if (e < 0) return; // uniform: fewer tiles than the grid allows
+    const int n = min(32, __builtin_amdgcn_readfirstlane(it_s[1])), first = __builtin_amdgcn_readfirstlane(it_s[2]);
+    constexpr int ROWS = NMAT == 2 ? 128 : 256, WROWS = ROWS / 4;
+    const int nb = cols >> 8, r0 = ROWS * rb, rend = min(rows, r0 + ROWS);
+    const uint32_t strip = (uint32_t)((size_t)(rend - r0) * stride);
+    const rsrc_t rs[2] = {make_rsrc(tabA[e] + (size_t)r0 * stride, strip),
+                          make_rsrc((NMAT == 2 ? tabB : tabA)[e] + (size_t)r0 * stride, strip)};
+    GmTiled<2> wt;
+    wt.init(WROWS * wave, WROWS * wave + (NMAT == 2 ? 0 : 32), lane, nb);
+    wt.head_load(rs, 0);
+    wt.load(rs, 0, 0);
+    wt.load(rs, 1, 1);
+    __shared__ gm_u4 xb_s[2][4 * GM_UNIT / 16];
+    __shared__ gm_u4 ms[2][GM_SUMS / 16];
+    __shared__ float ps[2][32];
+    if ((int)threadIdx.x < n) slot_s[threadIdx.x] = list[first + threadIdx.x];
+    if constexpr (!STAGED) {
+        // tokens past n stay zero in both buffers
+        for (int i = threadIdx.x; i < 2 * 4 * GM_UNIT / 16; i += 256)
+            if ((i & 31) >= n) (&xb_s[0][0])[i] = gm_u4{0u, 0u, 0u, 0u};
+        if (threadIdx.x < 2 * GM_SUMS / 16 && ((int)threadIdx.x & 31) >= n)
+            (&ms[0][0])[threadIdx.x] = gm_u4{0u, 0u, 0u, 0u};
+        if (threadIdx.x < 64) (&ps[0][0])[threadIdx.x] = 0.0f;
+    }
+    __syncthreads();
+    // STAGED: thread (token m, i): pieces 2 i and 2 i + 1 (of 16) of every unit;
+    // a token's 256 bytes of a unit are read by eight lanes
+    const int xm = (int)threadIdx.x >> 3, xi = (int)threadIdx.x & 7;
+    const size_t xtok = STAGED ? (size_t)(slot_s[min(xm, n - 1)] / xdiv) * nb : 0;
+    const size_t mtok = STAGED ? (size_t)(slot_s[min(nl, n - 1)] / xdiv) * nb : 0; // threads 0 .. 63: sums and 2^-s
+    gm_u4 xr[8], mr;
+    float pr = 0.0f;
+    // else: tokens wave + 4 k, k = 4 g + i
+    gm_f4 xv[2][4];
+    const int tmax = (n - wave + 3) >> 2; // this wavefront's tokens
+    const float *xrow[8];
+    if constexpr (!STAGED) {
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            xrow[k] = xs + (size_t)(__builtin_amdgcn_readfirstlane(slot_s[min(wave + 4 * k, n - 1)]) / xdiv) * cols;
+    }
+    auto load_x = [&](int sb) {
+        if constexpr (STAGED) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                xr[k] = gm_u4{0u, 0u, 0u, 0u};
+                if (xm < n) xr[k] = *(const gm_u4 *)(xg.f + (xtok + sb) * GM_TOK + 256 * (k >> 1) + 32 * xi + 16 * (k & 1));
+            }
+            mr = gm_u4{0u, 0u, 0u, 0u};
+            pr = 0.0f;
+            if (wave == 0 && nl < n) {
+                mr = *(const gm_u4 *)(xg.m + (mtok + sb) * GM_TOK_SUMS + 16 * f);
+                pr = xg.p[mtok + sb];
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                xv[k >> 2][k & 3] = gm_f4{0.f, 0.f, 0.f, 0.f};
+                if (k < tmax) xv[k >> 2][k & 3] = *(const gm_f4 *)(xrow[k] + 256 * sb + 4 * lane);
+            }
+        }
+    };
+    auto store_x = [&](int b) {
+        if constexpr (STAGED) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) // unit k / 2's piece 2 xi + k % 2: step xi / 2, part xi % 2, half k % 2
+                xb_s[b][(k >> 1) * (GM_UNIT / 16) + 32 * (2 * xi + (k & 1)) + (xm ^ gm_swz(k >> 1, xi >> 1, xi & 1))] =
+                    xr[k];
+            if (wave == 0) {
+                ms[b][lane] = mr;
+                if (f == 0) ps[b][nl] = pr;
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < 2; g++)
+                if (4 * g < tmax) // uniform
+                    gm_stage_rows<FMT_Q4K, 4, false>(
+                        xv[g], lane, tmax - 4 * g, [&](int k) { return wave + 16 * g + 4 * k; },
+                        [&](int) { return (uint8_t *)xb_s[b]; },
+                        [&](int k) { return (uint8_t *)ms[b] + 16 * (wave + 16 * g + 4 * k); },
+                        [&](int k) { return &ps[b][wave + 16 * g + 4 * k]; });
+        }
+    };
+    load_x(0);
+    store_x(0);
+    load_x(min(1, nb - 1));
+    __syncthreads();
+    gm_f16v acc[2], S[2];
+    const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    acc[0] = acc[1] = zero;
+    uint64_t taken = 0;
+    for (int sb = 0; sb < nb; sb++) {
+        const int cur = sb & 1, sn = min(sb + 1, nb - 1);
+        wt.head();
+        wt.head_load(rs, sn);
+        // a step's x is read from LDS a step ahead, where the registers hold it
+        constexpr bool AHEAD = STAGED;
+        const uint8_t *xb = (const uint8_t *)xb_s[cur];
+        gm_h8 ah[2], al[2];
+        ah[0] = gm_frag_at(xb, lane, 0, 0, 0);
+        al[0] = gm_frag_at(xb, lane, 0, 0, 1);
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            if (!(p & 1)) {
+                wt.split(p >> 1);
+                wt.load(rs, 2 * sn + (p >> 1), p >> 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const int i1 = 4 * p + t + (AHEAD ? 1 : 0);
+                if (i1 < 16) {
+                    ah[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, lane, i1 >> 2, i1 & 3, 0);
+                    al[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, lane, i1 >> 2, i1 & 3, 1);
+                }
+                gm_h8 b[2][1];
+#pragma unroll
+                for (int j = 0; j < 2; j++) wt.frag(p >> 1, p & 1, t, j, b[j]);
+                const gm_h8 hi = ah[t & 1], lo = al[t & 1];
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b[j][0], p == 0 && t == 0 ? zero : S[j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[j][0], S[j], 0, 0, 0);
+            }
+        }
+        taken |= __ballot(ps[cur][lane & 31] < 0.0f);
+        float pt[16];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const gm_f4 v = *(const gm_f4 *)(ps[cur] + 8 * k + 4 * f);
+#pragma unroll
+            for (int i = 0; i < 4; i++) pt[4 * k + i] = v[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float d = wt.scale(j), dm = wt.min_scale(j);
+            const gm_h8 am = *(const gm_h8 *)((const uint8_t *)ms[cur] + 16 * lane);
+            const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wt.mins(j), zero, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[j][i], dm * M[i]), acc[j][i]);
+        }
+        if (sb + 1 < nb) { // uniform
+            store_x(cur ^ 1);
+            load_x(min(sb + 2, nb - 1));
+            __syncthreads();
+        }
+    }
+    const int row = r0 + WROWS * wave + nl; // NMAT 2: of gate and up; NMAT 1: and row + 32
+    if (__builtin_expect(taken != 0, 0)) {
+        const int row1 = NMAT == 2 ? row : row + 32;
+        gm_add_outliers<FMT_Q4K>(
+            acc, row < rows ? rowA[e] + (size_t)row * stride : nullptr,
+            row1 < rows ? (NMAT == 2 ? rowB : rowA)[e] + (size_t)row1 * stride : nullptr, cols,
+            [&](int t) { return xs + (size_t)(slot_s[t] / xdiv) * cols; }, n, 0, nb);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int t = 8 * (i >> 2) + 4 * f + (i & 3);
+        if (t >= n) continue;
+        float *o = out + (size_t)slot_s[t] * rows;
+        if constexpr (NMAT == 2) {
+            const float g = acc[0][i];
+            if (row < rows) o[row] = g / (1.0f + expf(-g)) * acc[1][i];
+        } else {
+            if (row < rows) o[row] = acc[0][i];
+            if (row + 32 < rows) o[row + 32] = acc[1][i];
         }
     }
 }
@@ -1005,4 +1404,37 @@ int launch_gemm(soso_hip *h, const Weight &w, const float *x, size_t n, float *y
     case SOSO_HIP_DTYPE_Q8_0: return launch_gemm_fmt<FMT_Q80>(h, w, x, n, y);
     default: return launch_gemm_fmt<FMT_Q6K>(h, w, x, n, y);
     }
+}
+
+// One grouped product of a registered MoE layer's Q4_K experts with tile-major
+// copies (nmat 2: gate / up, 1: down) over the active-expert records; slots: the
+// call's (token, rank) pairs, each in at most one record's list; n: x's rows.
+// x is converted once per call where scratch may be had (not fixed, and memory),
+// else by every workgroup: the same bits.
+int launch_gemm_moe(soso_hip *h, int nmat, const uint8_t *const *tiled, const uint8_t *const *row_major, size_t n_groups,
+                    size_t rows, size_t cols, size_t slots, size_t max_recs, const float *xs, size_t n, int xdiv,
+                    const int *list, const int *recs, const int *n_recs, bool fixed, float *out)
+{
+    if (max_recs > 256 || !tiled_q4k_ok(SOSO_HIP_DTYPE_Q4_K, rows, cols) ||
+        !gemm_shape_ok(SOSO_HIP_DTYPE_Q4_K, rows, cols))
+        return SOSO_HIP_DECLINED;
+    const size_t nblk = (rows + (nmat == 2 ? 127 : 255)) / (nmat == 2 ? 128 : 256), tiles = slots / 32 + max_recs;
+    const size_t stride = packed_row_stride(SOSO_HIP_DTYPE_Q4_K, cols), nb = cols / 256;
+    const unsigned grid = (unsigned)(tiles * nblk);
+    const size_t f_b = n * nb * GM_TOK, m_b = n * nb * GM_TOK_SUMS, p_b = n * nb * 4;
+    uint8_t *xg = fixed ? nullptr : (uint8_t *)scratch_get(h, 16, f_b + m_b + p_b);
+    GmX gx{xg, xg + f_b, (const float *)(xg + f_b + m_b)};
+    if (xg)
+        k_gm_stage_tok<<<(unsigned)(((n + 3) / 4 * nb + 3) / 4), 256, 0, h->stream>>>(xs, (int)n, (int)cols, xg,
+                                                                                     xg + f_b, (float *)(xg + f_b + m_b));
+#define GM_MOE(NM, ST)                                                                                                 \
+    k_gemm_moe<NM, ST><<<grid, 256, 0, h->stream>>>(tiled, NM == 2 ? tiled + n_groups : nullptr, row_major,           \
+                                                    NM == 2 ? row_major + n_groups : nullptr, stride, (int)rows,      \
+                                                    (int)cols, xs, gx, xdiv, list, recs, n_recs, (int)nblk, out)
+    if (nmat == 2 && xg) GM_MOE(2, true);
+    else if (nmat == 2) GM_MOE(2, false);
+    else if (xg) GM_MOE(1, true);
+    else GM_MOE(1, false);
+#undef GM_MOE
+    return hip_check(h, hipGetLastError(), "gemm moe launch");
 }

@@ -19,7 +19,7 @@
 //                 LDS).  Gate and up rows are read side by side and leave as
 //                 silu(gate.x) * up.x; down rows leave as y[slot].  (Two or
 //                 more tokens per active expert: the matrix-core kernel of
-//                 k_mfma.hip instead.)
+//                 k_mfma.hip instead, from six on that of k_gemm.hip.)
 //   k_moe_down_comb  up to 4 tokens: down and the weighted sum in one launch,
 //                 one wavefront per ranked expert.
 //   k_moe_combine out[t] = sum_j wgt[t,j] * y[t*top_k + j], j in ranking order.
@@ -1110,6 +1110,7 @@ size_t moe_scratch_fixed(const soso_hip *h, size_t n, size_t n_groups, size_t to
     if (need > cap || !base) return need;
     char *b = (char *)base;
     moe_scratch_carve(h, n, n_groups, top_k, ffn, b, (int *)(b + o1), (float *)(b + o2), s);
+    s.fixed = true;
     return need;
 }
 
@@ -1358,6 +1359,13 @@ static int launch_down_comb(soso_hip *h, const uint8_t *const *tab, size_t n_exp
     return hip_check(h, hipGetLastError(), "moe down+combine launch");
 }
 
+// Slots per active expert from which a registered layer's Q4_K experts run on
+// the f16 matrix cores in 32-slot tiles (k_gemm.hip).  128 experts of 2048 x 768
+// at top-8, us per layer on MI355X, before -> there: 65 tokens (4.1 slots per
+// expert) 109 -> 121, 128 162 -> 127, 512 466 -> 217; 16 experts of 1024 x 512
+// at 200 tokens 185 -> 56.
+constexpr size_t MOE_GEMM_SLOTS = 6;
+
 int launch_moe_experts(soso_hip *h, const float *xs, size_t n, size_t hdim, size_t ffn, size_t top_k,
                        uint8_t dt_gu, uint8_t dt_down, const uint8_t *const *tab, size_t n_groups, const float *wgt,
                        const uint8_t *use, const int32_t *route_idx, const MoeScratch &s, float *out,
@@ -1377,7 +1385,13 @@ int launch_moe_experts(soso_hip *h, const float *xs, size_t n, size_t hdim, size
     // a registered layer's tile-major copies, where it has them
     const bool tgu = layer && layer->tiled && layer->tiled_gu, tdn = layer && layer->tiled && layer->tiled_down;
     const uint8_t *const *ttab = layer ? layer->tiled : nullptr;
-    if (many && dt_gu == SOSO_HIP_DTYPE_Q4_K && mfma_shape_ok(dt_gu, ffn, hdim))
+    const bool gemm = !sidx && slots >= MOE_GEMM_SLOTS * max_recs;
+    rc = SOSO_HIP_DECLINED;
+    if (gemm && tgu)
+        rc = launch_gemm_moe(h, 2, ttab, tab, n_groups, ffn, hdim, slots, max_recs, xs, n, (int)top_k, s.list,
+                             s.recs, s.n_recs, s.fixed, s.act);
+    if (rc != SOSO_HIP_DECLINED) {
+    } else if (many && dt_gu == SOSO_HIP_DTYPE_Q4_K && mfma_shape_ok(dt_gu, ffn, hdim))
         rc = launch_mfma_moe(h, 2, tgu ? ttab : tab, (tgu ? ttab : tab) + n_groups, ffn, hdim, max_recs, xs, (int)top_k,
                              s.list, s.recs, s.n_recs, s.act, tgu, sidx, n * top_k);
     else
@@ -1390,7 +1404,12 @@ int launch_moe_experts(soso_hip *h, const float *xs, size_t n, size_t hdim, size
         return launch_down_comb(h, tab + 2 * n_groups, n_groups, hdim, ffn, s.act, route_idx, wgt, n, top_k, nullptr,
                                 out);
     if (rc == SOSO_HIP_OK) {
-        if (many && dt_down == SOSO_HIP_DTYPE_Q4_K && mfma_shape_ok(dt_down, hdim, ffn))
+        rc = SOSO_HIP_DECLINED;
+        if (gemm && tdn)
+            rc = launch_gemm_moe(h, 1, ttab + 2 * n_groups, tab + 2 * n_groups, n_groups, hdim, ffn, slots, max_recs,
+                                 s.act, slots, 1, s.list, s.recs, s.n_recs, s.fixed, s.ydown);
+        if (rc != SOSO_HIP_DECLINED) {
+        } else if (many && dt_down == SOSO_HIP_DTYPE_Q4_K && mfma_shape_ok(dt_down, hdim, ffn))
             rc = launch_mfma_moe(h, 1, (tdn ? ttab : tab) + 2 * n_groups, nullptr, hdim, ffn, max_recs, s.act, 1, s.list,
                                  s.recs, s.n_recs, s.ydown, tdn, sidx, n * top_k);
         else

@@ -1,0 +1,76 @@
+"""MoE layers whose experts get enough tokens for the f16 matrix cores
+(k_gemm.hip's grouped kernel) and the route that serves them, at the edges:
+expert loads around a 32-slot tile, experts without tokens, row blocks that
+end early, the allocation-free entry's bits, non-finite tokens, outliers.
+
+Tolerance: as the matmul's (x within 2^-23, exact products, f32 sums), twice
+over for the two products in a row, with the oracle's own f32 sums: 4e-6.
+"""
+import numpy as np
+import pytest
+
+from test_gpu_moe import Layer, moe_dev
+
+pytestmark = pytest.mark.gpu
+
+TOL = 4e-6
+
+
+@pytest.mark.parametrize("n_exp,h,ffn,top_k,n", [
+    (8, 512, 256, 2, 128),     # 32 slots per expert: about half the experts need a second tile
+    (16, 256, 256, 1, 97),     # one super-block per row, one slot per token
+    (5, 768, 512, 3, 40),      # three super-blocks
+    (128, 256, 256, 8, 300),   # many experts, over 512 slots
+    (200, 512, 256, 5, 260),   # more than 128 experts; 4.. slots each on average
+    (32, 512, 256, 8, 700),    # two route blocks of at most 4096 slots
+])
+def test_moe_many_tokens_match_cpu(gpu, orc, n_exp, h, ffn, top_k, n):
+    layer = Layer(orc, n_exp, h, ffn, top_k, 310 + n)
+    xs = orc.normal(n * h, 1.0, 311, n)
+    try:
+        layer.upload(gpu)
+        print(f"moe gemm {n_exp} experts {h}x{ffn} top-{top_k} n={n}", flush=True)
+        out, idx, wgt = moe_dev(gpu, layer, xs)
+        for t in sorted({0, 1, 31, 32, n // 2, n - 1}):
+            ref, ci, cw = layer.cpu(orc, xs[t * h:(t + 1) * h])
+            assert np.array_equal(idx[t], ci), t
+            assert orc.rel_l2(wgt[t], cw) < 1e-6
+            assert orc.rel_l2(out[t], ref) < TOL, (t, orc.rel_l2(out[t], ref))
+        # the allocation-free entry converts x in every workgroup: the same bits
+        slots_bytes = n * top_k * (h + ffn) * 4
+        if slots_bytes < 7 << 20:
+            xd, od = gpu.dev_alloc(xs.nbytes), gpu.dev_alloc(n * h * 4)
+            try:
+                gpu.h2d(xd, xs)
+                assert gpu.moe_ffn_dev_noalloc(layer.name, xd, n, od), gpu.last_error()
+                gpu.sync()
+                assert np.array_equal(gpu.d2h(od, (n, h), np.float32), out)
+            finally:
+                gpu.dev_free(xd)
+                gpu.dev_free(od)
+    finally:
+        layer.drop(gpu)
+
+
+def test_moe_many_tokens_outliers_and_nonfinite(gpu, orc):
+    """Tokens with elements 1e6 times the rest keep to the CPU's result, a NaN
+    token's outputs are NaN, and neither touches the others."""
+    n_exp, h, ffn, top_k, n = 6, 512, 256, 3, 64
+    layer = Layer(orc, n_exp, h, ffn, top_k, 330)
+    xs = orc.normal(n * h, 1.0, 331, n).reshape(n, h)
+    clean = xs.copy()
+    xs[3, 7] *= np.float32(1e6)
+    xs[3, 300] *= np.float32(1e6)
+    xs[5, 100] = np.nan
+    try:
+        layer.upload(gpu)
+        base, _, _ = moe_dev(gpu, layer, clean.ravel())
+        out, idx, _ = moe_dev(gpu, layer, xs.ravel())
+        assert np.isnan(out[5]).all()
+        same = [t for t in range(n) if t not in (3, 5)]
+        assert np.array_equal(out[same], base[same])
+        ref, ci, _ = layer.cpu(orc, xs[3])
+        assert np.array_equal(idx[3], ci)
+        assert orc.rel_l2(out[3], ref) < TOL, orc.rel_l2(out[3], ref)
+    finally:
+        layer.drop(gpu)

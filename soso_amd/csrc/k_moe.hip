@@ -12,7 +12,8 @@
 //                 counting-sorts the n*top_k slots by expert (cnt, offs, list).
 //                 Calls whose experts scan the ranking themselves (at most 512
 //                 slots on the matrix cores) take the logits alone, then
-//                 k_moe_rank (softmax + top-k, one wavefront per token).
+//                 k_moe_rank (softmax + top-k, one wavefront per token); from
+//                 ROUTE_MANY tokens on k_moe_logits, k_moe_rank, k_moe_sort.
 //   k_moe_rows    workgroups over (expert, row chunk) items of equal work:
 //                 every weight row of an expert is read once from HBM and
 //                 applied to all the tokens routed to it (their x staged in
@@ -95,6 +96,136 @@ __device__ void topk_regs(const float (&lg)[4], int n_exp, int top_k, int32_t *_
     }
 }
 
+// Counting sort of the slots by expert in LDS (a slot's position inside its
+// expert's list does not change any result), the active-expert records and the
+// work items, by one workgroup of at least two wavefronts; get(s): slot s's
+// expert.
+struct RouteSort {
+    int pre[257], c[256], o[257], f[256];
+    int16_t e[MOE_ROUTE_MAX_SLOTS];
+};
+template <class Get>
+__device__ __forceinline__ void route_sort(RouteSort &S, Get get, int slots, int n_exp, int *__restrict__ cnt,
+                                           int *__restrict__ offs, int *__restrict__ list, int *__restrict__ items,
+                                           int *__restrict__ n_items, int target, int *__restrict__ recs,
+                                           int *__restrict__ n_recs)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int x = threadIdx.x; x < n_exp; x += blockDim.x) S.c[x] = S.f[x] = 0;
+    __syncthreads();
+    for (int sl = threadIdx.x; sl < slots; sl += blockDim.x) {
+        const int x = min(max(get(sl), 0), n_exp - 1);
+        S.e[sl] = (int16_t)x;
+        atomicAdd(&S.c[x], 1);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        // exclusive scan over n_exp <= 256 counts, 4 per lane
+        int v[4], tot = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int x = 4 * lane + q;
+            v[q] = x < n_exp ? S.c[x] : 0;
+            tot += v[q];
+        }
+        int incl = tot;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        int run = incl - tot;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int x = 4 * lane + q;
+            if (x < n_exp) S.o[x] = run;
+            run += v[q];
+        }
+        if (lane == 63) S.o[n_exp] = incl;
+    }
+    __syncthreads();
+    for (int sl = threadIdx.x; sl < slots; sl += blockDim.x) {
+        const int x = S.e[sl];
+        list[S.o[x] + atomicAdd(&S.f[x], 1)] = sl;
+    }
+    for (int x = threadIdx.x; x < n_exp; x += blockDim.x) {
+        cnt[x] = S.c[x];
+        offs[x] = S.o[x];
+    }
+    if (threadIdx.x == 0) offs[n_exp] = S.o[n_exp];
+    if (wave == 0) {
+        // work items: expert x with c tokens gets max(1, round(c * target /
+        // slots)) row chunks, so every item carries about the same tokens x
+        // rows; exclusive scan of the chunk counts over the experts
+        int v[4], tot = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int x = 4 * lane + q;
+            const int cx = x < n_exp ? S.c[x] : 0;
+            v[q] = cx > 0 ? min(0xFFFF, max(1, (cx * target + slots / 2) / slots)) : 0;
+            tot += v[q];
+        }
+        int incl = tot;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        int run = incl - tot;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int x = 4 * lane + q;
+            if (x < n_exp) S.pre[x] = run;
+            run += v[q];
+        }
+        if (lane == 63) {
+            S.pre[n_exp] = incl;
+            *n_items = incl;
+        }
+    }
+    if (wave == 1) {
+        // active-expert records, ascending: recs[4a ..] = {expert, slots, first slot, 0}
+        int nact = 0;
+        for (int x0 = 0; x0 < n_exp; x0 += 64) {
+            const int x = x0 + lane;
+            const bool on = x < n_exp && S.c[x] > 0;
+            const unsigned long long m = __ballot(on);
+            if (on) {
+                int *r = recs + 4 * (nact + __popcll(m & ((1ull << lane) - 1ull)));
+                r[0] = x;
+                r[1] = S.c[x];
+                r[2] = S.o[x];
+                r[3] = 0;
+            }
+            nact += __popcll(m);
+        }
+        if (lane == 0) *n_recs = nact;
+    }
+    __syncthreads();
+    // items[4i .. 4i+3] = {expert, its slot count, its first slot, chunk | chunks << 16};
+    // item i belongs to the expert x with S.pre[x] <= i < S.pre[x + 1]
+    const int total = S.pre[n_exp];
+    for (int i = threadIdx.x; i < total; i += blockDim.x) {
+        int lo = 0, hi = n_exp - 1; // last x with S.pre[x] <= i
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (S.pre[mid] <= i) lo = mid;
+            else hi = mid - 1;
+        }
+        const int nx = S.pre[lo + 1] - S.pre[lo];
+        int4 r;
+        r.x = lo;
+        r.y = S.c[lo];
+        r.z = S.o[lo];
+        r.w = (i - S.pre[lo]) | (nx << 16);
+        int *d = items + 4 * i;
+        d[0] = r.x;
+        d[1] = r.y;
+        d[2] = r.z;
+        d[3] = r.w;
+    }
+}
+
 // grid (ceil(n_exp / waves), ceil(n / TT)); wave w of workgroup (bx, by)
 // owns expert bx*waves + w for tokens by*TT .. + TT - 1.  `ticket` is zero
 // between launches (the last workgroup resets it).  The last workgroup also
@@ -124,10 +255,8 @@ __global__ void __launch_bounds__(512) k_moe_route(const float *__restrict__ W, 
                                                     const float *__restrict__ norm_w = nullptr, float eps = 0.0f)
 {
     __shared__ int last;
-    __shared__ int pre_s[257];
     __shared__ float sel[8][64];
-    __shared__ int c_s[256], o_s[257], f_s[256];
-    __shared__ int16_t e_s[ROUTE_MAX_SLOTS];
+    __shared__ RouteSort sort;
     __shared__ int16_t rank_s[ROUTE_TT * 64]; // the ranking of a single token block, for its sort
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int e = blockIdx.x * nw + wave;
@@ -225,126 +354,10 @@ __global__ void __launch_bounds__(512) k_moe_route(const float *__restrict__ W, 
     }
     __syncthreads();
     if (!last) return;
-    // counting sort of the slots by expert in LDS (a slot's position inside
-    // its expert's list does not change any result)
-    const int slots = n * top_k;
-    for (int x = threadIdx.x; x < n_exp; x += blockDim.x) c_s[x] = f_s[x] = 0;
-    __syncthreads();
-    for (int sl = threadIdx.x; sl < slots; sl += blockDim.x) {
-        const int x = min(max((int)(single ? rank_s[sl]
-                                           : __hip_atomic_load(idx + sl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)),
-                              0),
-                          n_exp - 1);
-        e_s[sl] = (int16_t)x;
-        atomicAdd(&c_s[x], 1);
-    }
-    __syncthreads();
-    if (wave == 0) {
-        // exclusive scan over n_exp <= 256 counts, 4 per lane
-        int v[4], tot = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int x = 4 * lane + q;
-            v[q] = x < n_exp ? c_s[x] : 0;
-            tot += v[q];
-        }
-        int incl = tot;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += y;
-        }
-        int run = incl - tot;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int x = 4 * lane + q;
-            if (x < n_exp) o_s[x] = run;
-            run += v[q];
-        }
-        if (lane == 63) o_s[n_exp] = incl;
-    }
-    __syncthreads();
-    for (int sl = threadIdx.x; sl < slots; sl += blockDim.x) {
-        const int x = e_s[sl];
-        list[o_s[x] + atomicAdd(&f_s[x], 1)] = sl;
-    }
-    for (int x = threadIdx.x; x < n_exp; x += blockDim.x) {
-        cnt[x] = c_s[x];
-        offs[x] = o_s[x];
-    }
-    if (threadIdx.x == 0) offs[n_exp] = o_s[n_exp];
-    if (wave == 0) {
-        // work items: expert x with c tokens gets max(1, round(c * target /
-        // slots)) row chunks, so every item carries about the same tokens x
-        // rows; exclusive scan of the chunk counts over the experts
-        int v[4], tot = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int x = 4 * lane + q;
-            const int cx = x < n_exp ? c_s[x] : 0;
-            v[q] = cx > 0 ? min(0xFFFF, max(1, (cx * target + slots / 2) / slots)) : 0;
-            tot += v[q];
-        }
-        int incl = tot;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += y;
-        }
-        int run = incl - tot;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int x = 4 * lane + q;
-            if (x < n_exp) pre_s[x] = run;
-            run += v[q];
-        }
-        if (lane == 63) {
-            pre_s[n_exp] = incl;
-            *n_items = incl;
-            if (!single) *ticket = 0u;
-        }
-    }
-    if (wave == 1) {
-        // active-expert records, ascending: recs[4a ..] = {expert, slots, first slot, 0}
-        int nact = 0;
-        for (int x0 = 0; x0 < n_exp; x0 += 64) {
-            const int x = x0 + lane;
-            const bool on = x < n_exp && c_s[x] > 0;
-            const unsigned long long m = __ballot(on);
-            if (on) {
-                int *r = recs + 4 * (nact + __popcll(m & ((1ull << lane) - 1ull)));
-                r[0] = x;
-                r[1] = c_s[x];
-                r[2] = o_s[x];
-                r[3] = 0;
-            }
-            nact += __popcll(m);
-        }
-        if (lane == 0) *n_recs = nact;
-    }
-    __syncthreads();
-    // items[4i .. 4i+3] = {expert, its slot count, its first slot, chunk | chunks << 16};
-    // item i belongs to the expert x with pre_s[x] <= i < pre_s[x + 1]
-    const int total = pre_s[n_exp];
-    for (int i = threadIdx.x; i < total; i += blockDim.x) {
-        int lo = 0, hi = n_exp - 1; // last x with pre_s[x] <= i
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (pre_s[mid] <= i) lo = mid;
-            else hi = mid - 1;
-        }
-        const int nx = pre_s[lo + 1] - pre_s[lo];
-        int4 r;
-        r.x = lo;
-        r.y = c_s[lo];
-        r.z = o_s[lo];
-        r.w = (i - pre_s[lo]) | (nx << 16);
-        int *d = items + 4 * i;
-        d[0] = r.x;
-        d[1] = r.y;
-        d[2] = r.z;
-        d[3] = r.w;
-    }
+    if (threadIdx.x == 0 && !single) *ticket = 0u;
+    route_sort(
+        sort, [&](int sl) { return (int)(single ? rank_s[sl] : __hip_atomic_load(idx + sl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)); },
+        n * top_k, n_exp, cnt, offs, list, items, n_items, target, recs, n_recs);
 }
 
 // The ranking of calls whose expert kernels scan it (no slot sort): one
@@ -367,6 +380,65 @@ __global__ void __launch_bounds__(256) k_moe_rank(const float *__restrict__ logi
         lg[q] = x < n_exp ? logits[(size_t)t * n_exp + x] : -INFINITY;
     }
     topk_regs(lg, n_exp, top_k, idx + (size_t)t * top_k, wgt + (size_t)t * top_k, sel[wave], rank_s + wave * 64);
+}
+
+__global__ void __launch_bounds__(1024) k_moe_sort(const int32_t *__restrict__ idx, int slots, int n_exp,
+                                                   int *__restrict__ cnt, int *__restrict__ offs,
+                                                   int *__restrict__ list, int *__restrict__ items,
+                                                   int *__restrict__ n_items, int target, int *__restrict__ recs,
+                                                   int *__restrict__ n_recs)
+{
+    __shared__ RouteSort sort;
+    route_sort(sort, [&](int sl) { return (int)idx[sl]; }, slots, n_exp, cnt, offs, list, items, n_items, target, recs,
+               n_recs);
+}
+
+// Logits of many tokens: a workgroup per 16 tokens x 16 experts, its eight
+// wavefronts each taking every eighth 16-column step of the rows on the f32
+// matrix cores (v_mfma_f32_16x16x4_f32: lane l holds token or expert l % 16,
+// columns 4 (l / 16) .. of the step), the eight partial sums added in wavefront
+// order.  (k_moe_route's dot products took a wavefront per expert and four
+// tokens: 47 us with the ranking and the sort for 512 tokens x 128 experts x
+// 2048, against 21 with this, k_moe_rank and k_moe_sort.)
+typedef float moe_f4 __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(512) k_moe_logits(const float *__restrict__ W, const float *__restrict__ xs, int n,
+                                                    int hdim, int n_exp, float *__restrict__ logits)
+{
+    __shared__ float part[8][16][17];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int e = 16 * blockIdx.x + r, t = 16 * blockIdx.y + r;
+    const float *wr = W + (size_t)min(e, n_exp - 1) * hdim, *xr = xs + (size_t)min(t, n - 1) * hdim;
+    const int steps = (hdim + 15) / 16;
+    moe_f4 ac[4] = {}; // one chain per column of four
+    constexpr int Q = 16; // steps in flight
+    for (int i0 = wave; i0 < steps; i0 += 8 * Q) {
+        moe_f4 a[Q], b[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int c = 16 * (i0 + 8 * q) + 4 * g;
+            a[q] = b[q] = moe_f4{0.f, 0.f, 0.f, 0.f};
+            if (c < hdim) { // hdim is a multiple of four
+                a[q] = *(const moe_f4 *)(xr + c);
+                b[q] = *(const moe_f4 *)(wr + c);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) ac[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][k], b[q][k], ac[k], 0, 0, 0);
+    }
+    const moe_f4 acc = (ac[0] + ac[1]) + (ac[2] + ac[3]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) part[wave][4 * g + i][r] = acc[i]; // token 4 g + i, expert r
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        const int tt = threadIdx.x >> 4, ee = threadIdx.x & 15;
+        float s = part[0][tt][ee];
+#pragma unroll
+        for (int w = 1; w < 8; w++) s += part[w][tt][ee];
+        if (16 * (int)blockIdx.y + tt < n && 16 * (int)blockIdx.x + ee < n_exp)
+            logits[(size_t)(16 * blockIdx.y + tt) * n_exp + 16 * blockIdx.x + ee] = s;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1114,6 +1186,12 @@ size_t moe_scratch_fixed(const soso_hip *h, size_t n, size_t n_groups, size_t to
     return need;
 }
 
+// Tokens from which the route runs as three launches (matrix-core logits, the
+// ranking, the sort).  us per layer of 128 experts of 2048 x 768, one launch /
+// three: 128 tokens 125.8 / 126.7, 160 130.7 / 128.9, 200 136.9 / 132.1, 512
+// 215 / 191.
+constexpr size_t ROUTE_MANY = 160;
+
 int launch_moe_route(soso_hip *h, const float *w, const float *x, size_t n, size_t hdim, size_t n_exp, size_t top_k,
                      const MoeScratch &s, bool sort)
 {
@@ -1124,6 +1202,14 @@ int launch_moe_route(soso_hip *h, const float *w, const float *x, size_t n, size
         k_moe_route<1, 8><<<grid, 512, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, (int)top_k, s.logits,
                                                         s.idx, s.wgt, s.cnt, s.offs, s.list, s.items, s.n_items,
                                                         moe_item_target(h), s.recs, s.n_recs, h->ticket);
+    } else if (n >= ROUTE_MANY) {
+        const dim3 grid((unsigned)((n_exp + 15) / 16), (unsigned)((n + 15) / 16));
+        k_moe_logits<<<grid, 512, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, s.logits);
+        k_moe_rank<<<(unsigned)((n + 3) / 4), 256, 0, h->stream>>>(s.logits, (int)n, (int)n_exp, (int)top_k, s.idx,
+                                                                  s.wgt);
+        if (sort)
+            k_moe_sort<<<1, 1024, 0, h->stream>>>(s.idx, (int)(n * top_k), (int)n_exp, s.cnt, s.offs, s.list, s.items,
+                                                  s.n_items, moe_item_target(h), s.recs, s.n_recs);
     } else if (!sort) {
         // logits by two-wavefront workgroups, two tokens per wavefront (batch
         // 32: 87.3 us per layer against 87.6 with four tokens and with one),

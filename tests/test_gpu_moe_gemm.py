@@ -74,3 +74,27 @@ def test_moe_many_tokens_outliers_and_nonfinite(gpu, orc):
         assert orc.rel_l2(out[3], ref) < TOL, orc.rel_l2(out[3], ref)
     finally:
         layer.drop(gpu)
+
+
+@pytest.mark.parametrize("n_exp,h,top_k,n", [(128, 2048, 8, 160), (17, 68, 3, 163), (256, 260, 64, 64), (1, 64, 1, 200),
+                                             (33, 4100, 5, 333)])
+def test_router_topk_many_tokens(gpu, orc, n_exp, h, top_k, n):
+    """The matrix-core logits at tiles that end early, widths that end inside a
+    16-column step, one expert, 256 experts."""
+    w = orc.normal(n_exp * h, 0.05, 340, n_exp)
+    xs = orc.normal(n * h, 1.0, 341, n)
+    idx, wgt = np.full(n * top_k, -1, np.int32), np.zeros(n * top_k, np.float32)
+    key = f"router.many.{n_exp}.{h}.{n}"
+    assert gpu.router_topk(key, w, xs, n, h, n_exp, top_k, idx, wgt), gpu.last_error()
+    # against 64 bits (the oracle's f32 sum of 2048 terms in a row is itself 1e-6 off); a logit here is
+    # within about 2^-22 of its terms' size, some 1e-6, and so are the probabilities
+    W, X = w.reshape(n_exp, h).astype(np.float64), xs.reshape(n, h).astype(np.float64)
+    idx, wgt = idx.reshape(n, top_k), wgt.reshape(n, top_k)
+    for t in range(n):
+        lg = W @ X[t]
+        p = np.exp(lg - lg.max())
+        p /= p.sum()
+        order = np.argsort(-p, kind="stable")[:top_k]
+        assert np.array_equal(idx[t], order) or np.allclose(p[idx[t]], p[order], rtol=1e-5, atol=0), t
+        assert len(set(idx[t].tolist())) == top_k
+        assert orc.rel_l2(wgt[t], p[order] / p[order].sum()) < 4e-6, t

@@ -152,13 +152,16 @@ struct soso_hip {
     // the scratch pointers it was captured with, so a slot outgrown while any
     // graph exists is retired, not freed: retired buffers are freed once no
     // graph is left (graph_destroy) or with the handle.
-    static constexpr int N_SCRATCH = 18;
+    static constexpr int N_SCRATCH = 19;
     void *scratch[N_SCRATCH] = {};
     size_t scratch_cap[N_SCRATCH] = {};
     std::vector<void *> retired;
     // pinned host staging (pinned_get)
     void *pinned = nullptr;
     size_t pinned_cap = 0;
+    // the pieces of a long download (soso_hip_matmul), created on first use
+    static constexpr int N_PIECES = 16;
+    hipEvent_t piece_ev[N_PIECES] = {};
     // SOSO_TICKET_BYTES of "last workgroup" state, zero between launches (each
     // kernel resets what it used): uint 0 the final counter (argmax, MoE
     // route), uints 64 .. 831 argmax partials (winner, index, holds-NaN flag per segment), uints 2048 .. 3071 the MoE

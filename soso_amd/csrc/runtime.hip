@@ -331,6 +331,8 @@ void soso_hip_destroy(soso_hip *h)
         if (h->scratch[i]) (void)hipFree(h->scratch[i]);
     for (void *p : h->retired) (void)hipFree(p);
     if (h->pinned) (void)hipHostFree(h->pinned);
+    for (hipEvent_t e : h->piece_ev)
+        if (e) (void)hipEventDestroy(e);
     for (auto &kv : h->moe_layers) (void)moe_free(h, kv.second);
     for (auto &kv : h->decode_models) (void)decode_free(h, kv.second);
     if (h->ticket) (void)hipFree(h->ticket);
@@ -356,6 +358,12 @@ void soso_hip_stats(const soso_hip *h, soso_hip_stats_t *out)
 
 const char *soso_hip_last_error(const soso_hip *h) { return h ? h->err.c_str() : "null handle"; }
 
+// Bytes of one piece of a long transfer between the caller's buffers and the
+// device.  us per call (Q4_K 14336 x 4096 at 128 tokens / 4096 x 14336 at 100;
+// one piece: 506 / 430): 0.25 MiB 552 / 505, 0.5 485 / 360, 1 438 / 326, 2 438 /
+// 309.
+static constexpr size_t HOST_PIECE = 2u << 20;
+
 int soso_hip_matmul(soso_hip *h, const char *key, size_t key_len, const uint8_t *w, size_t w_len, uint8_t dtype,
                     size_t rows, size_t cols, size_t n, const float *x, float *y)
 {
@@ -367,31 +375,59 @@ int soso_hip_matmul(soso_hip *h, const char *key, size_t key_len, const uint8_t 
     Weight *wt = nullptr;
     rc = get_weight(h, key, key_len, w, w_len, dtype, rows, cols, &wt);
     if (rc != SOSO_HIP_OK) return rc;
-    float *xd = (float *)scratch_get(h, 0, n * cols * 4);
+    const size_t xb = n * cols * 4, yb = n * rows * 4;
+    float *xd = (float *)scratch_get(h, 0, xb);
     // x and y pass through the pinned staging buffer (the caller's buffers are
     // pageable: copies from and to them are staged by the runtime, slowly)
-    float *hx = (float *)pinned_get(h, (n * cols + n * rows) * 4);
+    float *hx = (float *)pinned_get(h, xb + yb);
     if (!xd || !hx) return set_err(h, SOSO_HIP_ERR_NOMEM, "matmul: scratch");
     float *hy = hx + n * cols;
-    memcpy(hx, x, n * cols * 4);
-    rc = hip_check(h, hipMemcpyAsync(xd, hx, n * cols * 4, hipMemcpyHostToDevice, h->stream), "x upload");
-    // the kernel writes y straight into the pinned buffer (host memory the
-    // device addresses), so no download follows it.  Measured on MI355X
-    // (median per call, host wall clock): Q8_0 4096 x 4096 38.5 us from and to
-    // the caller's pageable buffers, 22.7 with a pinned upload and download,
-    // 21.5 with y written by the kernel; Q4_K 14336 x 4096 34.6 / 34.0 / 26.2.
-    // (x read from the pinned buffer by a copy kernel instead of the upload:
-    // the same.)
-    float *hyd = nullptr;
-    if (rc == SOSO_HIP_OK) rc = hip_check(h, hipHostGetDevicePointer((void **)&hyd, hy, 0), "pinned y address");
-    if (rc == SOSO_HIP_OK) rc = launch_matvec(h, *wt, xd, hyd, n);
+    // a piece's upload runs while the next is copied into the staging buffer
+    for (size_t o = 0; o < xb && rc == SOSO_HIP_OK; o += HOST_PIECE) {
+        const size_t c = std::min(HOST_PIECE, xb - o);
+        memcpy((char *)hx + o, (const char *)x + o, c);
+        rc = hip_check(h, hipMemcpyAsync((char *)xd + o, (char *)hx + o, c, hipMemcpyHostToDevice, h->stream), "x upload");
+    }
+    // A short y is written by the kernel straight into the pinned buffer (host
+    // memory the device addresses), so no download follows it.  Measured on
+    // MI355X (median per call, host wall clock): Q8_0 4096 x 4096 38.5 us from
+    // and to the caller's pageable buffers, 22.7 with a pinned upload and
+    // download, 21.5 with y written by the kernel; Q4_K 14336 x 4096 34.6 / 34.0 /
+    // 26.2.  (x read from the pinned buffer by a copy kernel instead of the
+    // upload: the same.)  A long y comes down in pieces, each copied to the
+    // caller while the next is on its way.
+    const size_t piece = std::max(HOST_PIECE, ((yb + soso_hip::N_PIECES - 1) / soso_hip::N_PIECES + 4095) & ~(size_t)4095);
+    const size_t pieces = (yb + piece - 1) / piece;
+    float *yd = pieces > 1 ? (float *)scratch_get(h, 18, yb) : nullptr;
+    for (size_t i = 0; yd && i < pieces; i++)
+        if (!h->piece_ev[i] && hipEventCreateWithFlags(&h->piece_ev[i], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            h->piece_ev[i] = nullptr;
+            yd = nullptr;
+        }
+    if (yd) {
+        if (rc == SOSO_HIP_OK) rc = launch_matvec(h, *wt, xd, yd, n);
+        for (size_t i = 0; i < pieces && rc == SOSO_HIP_OK; i++) {
+            const size_t o = i * piece, c = std::min(piece, yb - o);
+            rc = hip_check(h, hipMemcpyAsync((char *)hy + o, (char *)yd + o, c, hipMemcpyDeviceToHost, h->stream), "y");
+            if (rc == SOSO_HIP_OK) rc = hip_check(h, hipEventRecord(h->piece_ev[i], h->stream), "y piece");
+        }
+        for (size_t i = 0; i < pieces && rc == SOSO_HIP_OK; i++) {
+            const size_t o = i * piece, c = std::min(piece, yb - o);
+            rc = hip_check(h, hipEventSynchronize(h->piece_ev[i]), "y piece sync");
+            if (rc == SOSO_HIP_OK) memcpy((char *)y + o, (char *)hy + o, c);
+        }
+    } else {
+        float *hyd = nullptr;
+        if (rc == SOSO_HIP_OK) rc = hip_check(h, hipHostGetDevicePointer((void **)&hyd, hy, 0), "pinned y address");
+        if (rc == SOSO_HIP_OK) rc = launch_matvec(h, *wt, xd, hyd, n);
+        if (rc == SOSO_HIP_OK) rc = hip_check(h, hipStreamSynchronize(h->stream), "matmul sync");
+        if (rc == SOSO_HIP_OK) memcpy(y, hy, yb);
+    }
     if (rc != SOSO_HIP_OK) {
         (void)hip_release(h, hipStreamSynchronize(h->stream), "matmul drain");
         return rc;
     }
-    rc = hip_check(h, hipStreamSynchronize(h->stream), "matmul sync");
-    if (rc != SOSO_HIP_OK) return rc;
-    memcpy(y, hy, n * rows * 4);
     h->stats.bytes_up += n * cols * 4;
     h->stats.bytes_down += n * rows * 4;
     clk.done();

@@ -134,3 +134,24 @@ def test_matmul_captured_before_any_scratch(orc):
         assert np.array_equal(g.d2h(yd, (n, rows), np.float32), out)
         g.dev_free(xd)
         g.dev_free(yd)
+
+
+@pytest.mark.parametrize("rows,cols,n", [(4096, 1024, 128), (4096, 1024, 129), (8192, 4096, 200), (70000, 256, 130)])
+def test_matmul_host_long_transfers(gpu, orc, rows, cols, n):
+    """Host-buffer calls whose y is one, just over one, several and over sixteen
+    2 MiB pieces, x up to two: the device entry's bits."""
+    w = orc.synth(Q8, rows, cols, 211, n)
+    xs = orc.normal(n * cols, 1.0, 212, n).reshape(n, cols)
+    key = f"gemm.host.{rows}.{n}"
+    out = np.full((n, rows), np.nan, np.float32)
+    xd, yd = gpu.dev_alloc(xs.nbytes), gpu.dev_alloc(out.nbytes)
+    try:
+        assert gpu.matmul(key, w, Q8, rows, cols, n, xs, out), gpu.last_error()
+        gpu.h2d(xd, xs)
+        assert gpu.matmul_dev(key, n, xd, yd), gpu.last_error()
+        gpu.sync()
+        assert np.array_equal(gpu.d2h(yd, (n, rows), np.float32), out)
+    finally:
+        gpu.weight_drop(key)
+        gpu.dev_free(xd)
+        gpu.dev_free(yd)

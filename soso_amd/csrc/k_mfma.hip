@@ -1,7 +1,9 @@
 // k_mfma.hip -- products of several tokens per weight row on the matrix
-// cores: the Q4_K MoE experts when a call routes two or more tokens to each
-// active expert on average, and Q4_K or Q8_0 `matmul` (GpuDispatch::matmul,
-// crates/soso-llm-core/src/gpu.rs:443-455) from 16 tokens up.
+// cores in exact integers: the Q4_K MoE experts when a call routes two or more
+// tokens to each active expert on average (up to six, MOE_GEMM_SLOTS), and Q4_K
+// or Q8_0 `matmul` (GpuDispatch::matmul, crates/soso-llm-core/src/gpu.rs:443-455)
+// from 16 tokens up in the shapes that gemm_wins (k_gemm.hip) leaves here: small
+// weights, and Q8_0 up to 4096 columns of fewer tokens.
 //
 // Exact integer arithmetic, as in the single-token kernels: x is staged as
 // three balanced signed base-256 digits of X = rint(x 2^e), one exponent e per
@@ -1698,7 +1700,7 @@ static int launch_mm_q4k(soso_hip *h, const Weight &w, const float *x, size_t n,
         nblk * rounds * 5 < cu * 4)
         return SOSO_HIP_DECLINED; // k_mfma_q4k's launch, which picks its shape from the grid, takes it
     uint8_t *xg = (uint8_t *)scratch_get(h, 16, n * (size_t)mm_tok_bytes((int)cols));
-    if (!xg) return set_err(h, SOSO_HIP_ERR_NOMEM, "mfma: staged x");
+    if (!xg) return SOSO_HIP_DECLINED; // no memory, or a capture that may not grow it: the launch that stages its own rounds
     const size_t waves = n * ((cols + 511) / 512);
     k_mm_stage<<<(unsigned)((waves + 3) / 4), 256, 0, h->stream>>>(x, (int)n, (int)cols, xg);
     int rc = hip_check(h, hipGetLastError(), "mm stage launch");
@@ -1740,7 +1742,7 @@ static int launch_mm_q80(soso_hip *h, const Weight &w, const float *x, size_t n,
         nblk * (n / (4 * MT)) * 5 < (size_t)h->num_cu * 4)
         return SOSO_HIP_DECLINED; // k_mfma_q80's launch takes it
     uint8_t *xg = (uint8_t *)scratch_get(h, 16, n * (size_t)mm_tok_bytes((int)cols));
-    if (!xg) return set_err(h, SOSO_HIP_ERR_NOMEM, "mfma: staged x");
+    if (!xg) return SOSO_HIP_DECLINED; // no memory, or a capture that may not grow it: the launch that stages its own rounds
     const size_t waves = n * ((cols + 511) / 512);
     k_mm_stage<<<(unsigned)((waves + 3) / 4), 256, 0, h->stream>>>(x, (int)n, (int)cols, xg);
     int rc = hip_check(h, hipGetLastError(), "mm stage launch");

@@ -95,7 +95,10 @@ void *scratch_get(soso_hip *h, int slot, size_t bytes)
     }
     size_t cap = bytes + bytes / 4 + 4096;
     void *p = nullptr;
-    if (hipMalloc(&p, cap) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, cap) != hipSuccess) {
+        (void)hipGetLastError(); // a caller may do without: its next launch check must not find this error
+        return nullptr;
+    }
     h->scratch[slot] = p;
     h->scratch_cap[slot] = cap;
     return p;

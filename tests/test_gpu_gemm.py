@@ -102,15 +102,19 @@ def test_matmul_f16_nonfinite_and_extreme_tokens(gpu, orc, dtype, rows, cols, n)
         assert orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t])) < TOL, t
 
 
-def test_matmul_captured_before_any_scratch(orc):
+@pytest.mark.parametrize("dtype,rows,cols,n", [
+    (Q4K, 4096, 4352, 6),    # the batched vector kernel
+    (Q4K, 14336, 4096, 64),  # the integer kernels, which would stage x in scratch too
+    (Q8, 4096, 4096, 64),
+])
+def test_matmul_captured_before_any_scratch(orc, dtype, rows, cols, n):
     """A capture that comes before any eager call finds no scratch to grow: the
     kernels that need none take it, and the replays give the product."""
     from soso_amd.dispatch import HipGpu
-    rows, cols, n = 4096, 4352, 6
-    w = orc.synth(Q4K, rows, cols, 209, 1)
+    w = orc.synth(dtype, rows, cols, 209, 1)
     xs = orc.normal(n * cols, 1.0, 210, 1).reshape(n, cols)
     with HipGpu(0) as g:
-        assert g.gemma_subir("w", w, Q4K, rows, cols), g.last_error()
+        assert g.gemma_subir("w", w, dtype, rows, cols), g.last_error()
         xd, yd = g.dev_alloc(xs.nbytes), g.dev_alloc(n * rows * 4)
         g.h2d(xd, xs)
         g.graph_begin()
@@ -122,8 +126,8 @@ def test_matmul_captured_before_any_scratch(orc):
             g.graph_launch(gid)
             g.sync()
             out = g.d2h(yd, (n, rows), np.float32)
-            for t in range(n):
-                assert orc.rel_l2(out[t], orc.matvec_f64(Q4K, w, rows, cols, xs[t])) < 1e-5, t
+            for t in {0, 3, n - 1}:
+                assert orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t])) < 1e-5, t
         # an eager call grows the scratch; the graph's replays go on
         assert g.matmul_dev("w", n, xd, yd), g.last_error()
         g.sync()

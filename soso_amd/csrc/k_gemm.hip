@@ -1300,45 +1300,62 @@ static bool gemm_shape_ok(uint8_t dtype, size_t rows, size_t cols)
 //    6 (79 -> 58; at 4: 53 -> 59).
 //  * Q4_K up to 4096 columns: against the batched vector kernel (below 16
 //    tokens) from 8 tokens and 2^22 weights (14336 x 4096 36.5 -> 20.2, 2048 x
-//    2048 10.1 -> 9.5; 768 x 2048 8.8 -> 9.4).  Against the integer matrix-core
-//    kernels, whose time is one chain along the columns, everywhere from 4096
-//    columns and 2^22 weights on (1024 x 4096 at 16 / 64 / 128 tokens 15.9 /
-//    16.1 / 24.8 -> 11.1 / 13.8 / 16.6); with fewer columns past 64 tokens
-//    (11305 x 768 at 64 / 100: 16.0 / 30.2 -> 18.8 / 18.0; 1000 x 1024 at 128:
-//    7.0 -> 11.9) or past 2^24 weights at 17 to 32 (14336 x 2048 at 16 / 24 /
-//    32 / 48: 15.1 / 25.3 / 24.4 / 23.2 -> 16.5 / 18.7 / 20.7 / 27.2).  Their
-//    form with x staged once (whole rounds of 16 tokens, whole 1024-column
-//    chunks) holds out longer: 2048 x 2048 at 128 / 300 tokens 14.9 / 35.3 ->
-//    16.1 / 26.8, 14336 x 2048 at 128 47.6 -> 34.4.
+//    2048 10.1 -> 9.8; 768 x 2048 8.8 -> 9.4), from 9 for smaller ones of 4096
+//    columns (100 x 4096 10.9 -> 10.0; at 8: 10.4 -> 10.2).  Against the integer
+//    matrix-core kernels, whose time is one chain along the columns, everywhere
+//    at 4096 columns (512 x 4096 at 16 tokens 15.9 -> 10.8, 1024 x 4096 at 64 /
+//    128 16.1 / 24.8 -> 13.8 / 16.6); with fewer columns past 2^24 weights at 17
+//    to 32 tokens (14336 x 2048 at 16 / 20 / 32 / 48: 15.1 / 25.3 / 24.2 / 23.2
+//    -> 16.5 / 18.4 / 20.7 / 27.2), and past 64 tokens from 2.1e8 products at
+//    2048 columns (1024 x 2048 at 100: 14.1 -> 12.7; 100 x 2048 at 1000: 11.6 ->
+//    12.4), 8e8 below (14336 x 768 at 70 20.8 -> 17.5, 1000 x 1280 at 600 23.8 ->
+//    20.0; 1000 x 1024 at 700 18.2 -> 19.2, 8192 x 512 at 128 11.5 -> 13.4).
+//    Their form with x staged once (whole rounds of 16 tokens, whole 1024-column
+//    chunks, a full grid) holds out longer: 2048 x 2048 at 128 / 256 tokens 14.8 /
+//    24.8 -> 16.1 / 21.3, 4096 x 1024 at 256 / 400 / 512 16.6 / 28.3 / 29.9 ->
+//    21.2 / 22.1 / 23.9, 14336 x 1024 at 144 27.9 -> 30.7.
 //  * Q6_K up to 4096 columns: past 2^24 weights from 8 tokens (14336 x 4096
 //    41.7 -> 27.6); smaller ones from 48 tokens (1000 x 1024 38.9 -> 15.4),
 //    below which they keep the batched vector kernel and with it the bits of
 //    single matvecs.
 //  * Q8_0, whose four code planes cost its lines four visits: past 2^24 weights
-//    from 33 tokens (14336 x 4096 at 64: 97 -> 51; at 32: 51 -> 53), from 2^22
-//    weights at 16 tokens where a row has 4096 columns (1024 x 4096 24.1 ->
-//    14.4) and at 64 where it has fewer (2048 x 2048 21.7 -> 16.5; at 32: 13.2
-//    -> 15.5).  Widths that are no multiple of 256 ran on the batched vector
-//    kernel: from 16 tokens (5000 x 1440 26.3 -> 17.2), if 2^22 weights or
-//    1024 columns (2014 x 768 at 149: 15.6 -> 16.3).
+//    from 33 tokens (14336 x 4096 at 64: 97 -> 51; at 32: 51 -> 53), smaller ones
+//    from 16: always from 3072 columns (512 x 4096 24.1 -> 14.4, 1000 x 3072 18.9
+//    -> 14.4; at 12: 17 -> 14, at 8: 10 -> 14), from 1.9e8 products at 2048 (1500
+//    x 2048 at 64 21.8 -> 15.3, 4096 x 2048 at 32 21.8 -> 16.9; 512 x 2048 at 128
+//    13.2 -> 14.9), 5e8 at 1024 (4096 x 1536 at 80 25.3 -> 22.6; at 64 16.1 ->
+//    18.0, 300 x 1536 at 1000 25.9 -> 27.5) and 1e9 below (300 x 768 at 4500 54.8
+//    -> 39.0; 8192 x 512 at 128 14.8 -> 16.4).  Against the form with x staged
+//    once, from 1e9 products (2048 x 2048 at 128 / 256: 17.0 / 30.8 -> 20.5 / 27.4,
+//    4096 x 4096 at 64 27.4 -> 25.2), 1.5e9 at 1024 columns (4096 x 1024 at 64 /
+//    256 / 512: 10.5 / 23.3 / 41.6 -> 15.7 / 28.8 / 33.8).  Widths that are no
+//    multiple of 256 ran on the batched vector kernel: from 16 tokens (5000 x
+//    1440 26.3 -> 17.2), if 2^22 weights or 1024 columns (2014 x 768 at 149:
+//    15.6 -> 16.3).
+constexpr size_t MM_FULL = 205; // 64-row x 16-token workgroups that fill four fifths of 256 CUs
 bool gemm_wins(uint8_t dtype, size_t rows, size_t cols, size_t n)
 {
     if (n < 4 || n > (1u << 20) || !gemm_shape_ok(dtype, rows, cols)) return false;
-    const size_t weights = rows * cols;
+    const size_t weights = rows * cols, work = weights * n;
     const bool large = weights > (1u << 24), small = weights < (1u << 22);
     if (dtype == SOSO_HIP_DTYPE_Q8_0) {
         if (cols > 4096) return n >= 6;
         if (cols % 256) return n >= 16 && (!small || cols >= 1024);
-        if (large) return n >= 33;
-        return !small && n >= (cols >= 4096 ? 16 : 64);
+        if (n < (large ? 33 : 16)) return false;
+        if (n % 16 == 0 && cols % 1024 == 0 && (rows + 63) / 64 * (n / 16) >= MM_FULL)
+            return work >= (cols >= 2048 ? 1000000000u : 1500000000u);
+        return cols >= 3072 || work >= (cols >= 2048 ? 190000000u : cols >= 1024 ? 500000000u : 1000000000u);
     }
     if (cols > 4096) return true;
     if (dtype == SOSO_HIP_DTYPE_Q6_K) return n >= (large ? 8 : 48);
+    if (cols == 4096) return n >= (small ? 9 : 8);
     if (!small && n < 16) return n >= 8;
-    if (!small && cols >= 4096) return true;
     if (n <= 64) return large && n > 16 && n <= 32;
-    if (n % 16 == 0 && cols % 1024 == 0 && n <= 128) return weights * n >= 3000000000u;
-    return weights * n >= 200000000u;
+    if (n % 16 == 0 && cols % 1024 == 0) {
+        if (n <= (cols < 2048 ? 240 : 128)) return work >= 3000000000u;
+        if (cols < 2048 && (rows + 255) / 256 * (n / 16) >= MM_FULL) return work >= 1500000000u;
+    }
+    return work >= (cols >= 2048 ? 210000000u : 800000000u);
 }
 
 static int gm_reduce(soso_hip *h, const float *part, size_t count, size_t nsplit, float *y)

@@ -38,6 +38,8 @@ def run(gpu, orc, dtype, rows, cols, xs, w, key):
     (Q4K, 14336, 4096, 64), (Q4K, 4099, 14336, 65), (Q6K, 4096, 14336, 127), (Q6K, 2500, 512, 1700),
     # Q8_0: whole and partial last super-blocks (64, 128 and 192 columns of one; an odd block padded)
     (Q8, 4096, 4096, 17), (Q8, 1300, 4160, 33), (Q8, 4099, 1152, 40), (Q8, 4097, 1216, 16), (Q8, 333, 4448, 6),
+    # small weights of 4096 and 2048 columns, on both sides of the line
+    (Q4K, 100, 4096, 9), (Q8, 100, 4096, 16), (Q8, 512, 3072, 17), (Q8, 300, 2048, 313), (Q4K, 300, 1536, 1751),
     # odd row and token counts whose product is no multiple of four, over several splits
     (Q4K, 4097, 4096, 17), (Q8, 1301, 6400, 19),
 ])

@@ -197,7 +197,9 @@ __device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count
     int s[R];
 #pragma unroll
     for (int k = 0; k < R; k++) {
-        s[k] = 15 - __builtin_amdgcn_frexp_expf(mx[k]);
+        // at most 126: 2^-s is a normal number, so that its sign can mark
+        // outliers above a block of subnormals (whose bits all fit at 2^126)
+        s[k] = min(126, 15 - __builtin_amdgcn_frexp_expf(mx[k]));
         float e[4], lo[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {

@@ -161,3 +161,19 @@ def test_matmul_host_long_transfers(gpu, orc, rows, cols, n):
         gpu.weight_drop(key)
         gpu.dev_free(xd)
         gpu.dev_free(yd)
+
+
+@pytest.mark.parametrize("dtype,rows,cols,n", [(Q4K, 4200, 4096, 9), (Q4K, 14400, 4096, 70), (Q6K, 300, 4352, 9),
+                                               (Q6K, 4100, 4352, 130), (Q8, 1100, 4224, 33)])
+def test_matmul_f16_outliers_above_subnormals(gpu, orc, dtype, rows, cols, n):
+    """Two elements of ordinary size in every 256, the others subnormal (what a
+    SwiGLU that underflows leaves): the large ones are taken out of the scale,
+    2^-s of the rest leaves f32's range, and they must still be added."""
+    w = orc.synth(dtype, rows, cols, 213, n)
+    xs = (orc.normal(n * cols, 1.0, 214, n) * np.float32(1e-42)).reshape(n, cols)
+    xs[:, 10::256] = np.float32(1.0)
+    xs[:, 200::256] = np.float32(0.5)
+    out = run(gpu, orc, dtype, rows, cols, xs, w, f"gemm.subn.{dtype}.{n}")
+    for t in (0, 1, n // 2, n - 1):
+        e = orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t]))
+        assert e < TOL, (t, e)

@@ -16,6 +16,19 @@ pytestmark = pytest.mark.gpu
 TOL = 4e-6
 
 
+def moe_noalloc(gpu, layer, xs):
+    n = xs.size // layer.h
+    xd, od = gpu.dev_alloc(xs.nbytes), gpu.dev_alloc(xs.nbytes)
+    try:
+        gpu.h2d(xd, xs)
+        assert gpu.moe_ffn_dev_noalloc(layer.name, xd, n, od), gpu.last_error()
+        gpu.sync()
+        return gpu.d2h(od, (n, layer.h), np.float32)
+    finally:
+        gpu.dev_free(xd)
+        gpu.dev_free(od)
+
+
 @pytest.mark.parametrize("n_exp,h,ffn,top_k,n", [
     (8, 512, 256, 2, 128),     # 32 slots per expert: about half the experts need a second tile
     (16, 256, 256, 1, 97),     # one super-block per row, one slot per token
@@ -98,3 +111,22 @@ def test_router_topk_many_tokens(gpu, orc, n_exp, h, top_k, n):
         assert np.array_equal(idx[t], order) or np.allclose(p[idx[t]], p[order], rtol=1e-5, atol=0), t
         assert len(set(idx[t].tolist())) == top_k
         assert orc.rel_l2(wgt[t], p[order] / p[order].sum()) < 4e-6, t
+
+
+def test_moe_many_tokens_outliers_above_subnormals(gpu, orc):
+    """Tokens of a few ordinary elements among subnormal ones, 600 slots of six
+    experts: the elements taken out must be added though 2^-s of the rest of
+    their block leaves f32's range; the allocation-free entry too."""
+    n_exp, h, ffn, top_k, n = 6, 512, 256, 3, 200
+    layer = Layer(orc, n_exp, h, ffn, top_k, 333)
+    xs = (orc.normal(n * h, 1.0, 334, n) * np.float32(1e-42)).reshape(n, h)
+    xs[:, 10::256] = orc.normal(n * (h // 256), 1.0, 335, n).reshape(n, -1)
+    xs[:, 200::256] = np.float32(3.0)
+    try:
+        layer.upload(gpu)
+        for name, out in (("eager", moe_dev(gpu, layer, xs.ravel())[0]), ("noalloc", moe_noalloc(gpu, layer, xs.ravel()))):
+            for t in (0, 1, n // 2, n - 1):
+                ref, _, _ = layer.cpu(orc, xs[t])
+                assert orc.rel_l2(out[t], ref) < TOL, (name, t, orc.rel_l2(out[t], ref))
+    finally:
+        layer.drop(gpu)

@@ -3,14 +3,15 @@
 // split into two f16 parts, on the f16 matrix cores.
 //
 // Arithmetic.  x is scaled by a power of two 2^s per token and 256-column
-// super-block (its largest element into [2^14, 2^15)) and written as hi + lo,
-// two f16 numbers whose sum is within 2^-23 of every element above 2^-17 of
-// the block's largest, and within 2^-40 of the largest below that (the integer
-// kernels' digits: within 2^-23 of the largest).  An element above 2^14 times
-// the third largest of its 128-column block's 8-column maxima (at most 16 can
-// be) is taken out, marked by a negative 2^-s, and its products are added at
-// the end with the weights dequantized exactly, so that it cannot push the rest
-// of its block below that floor.  Weights times the block scales are whole
+// super-block (its largest element into [2^14, 2^15); s <= 126) and written as hi + lo,
+// two f16 numbers whose sum is within 2^-23 of every element above 2^-16 of
+// the block's largest, and within 2^-39 of the largest below that (the integer
+// kernels' digits: within 2^-22 of the largest of 128 or 256 columns).  What
+// would push the rest below that floor is taken out (gm_take_out) and marked by
+// a negative 2^-s: single elements, whose products are added at the end with the
+// weights dequantized exactly, and where the two 128-column halves are too far
+// apart for one scale the larger half, which goes through the matrix cores by
+// itself at the end.  Weights times the block scales are whole
 // numbers: Q4_K's sc q (up to 945) exact in f16, Q6_K's sc (q - 32) (up to
 // 4096) exact as two f16, Q8_0's codes exact (its f32 scales are applied to the
 // block's sums).  Every product is exact in the f32 accumulators; a
@@ -88,21 +89,50 @@ __device__ __forceinline__ float gm_abs_max(gm_f4 v)
 {
     return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
 }
-// Above this an element of a 128-column block (32 lanes, four finite columns
-// each) is taken out: 2^14 times the third largest of the block's 16 maxima of
-// 8 columns.  Where that is zero no element needs the room.
-__device__ __forceinline__ float gm_outlier_thr(gm_f4 v)
+// Above this an element of a 128-column half (32 lanes, four finite columns
+// each) is taken out: 2^14 times ref, the third largest of its 16 maxima of 8
+// columns, so that what stays loses less to the parts' floor than to digits of
+// its own (22 bits of up to 16 times its third largest).  A half with no more than
+// two such maxima (at most 16 elements) has no third: ref is its smallest
+// element, and where the largest is beyond 2^14 times that all are taken out.
+__device__ __forceinline__ float gm_outlier_thr(gm_f4 v, float &ref)
 {
     const int lane = threadIdx.x & 63;
-    float cm = gm_abs_max(v);
+    float cm = gm_abs_max(v), least = INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (v[i] != 0.0f) least = fminf(least, fabsf(v[i]));
+    least = -gm_half_max(-least);
     cm = fmaxf(cm, dpp_f<0xB1>(cm));
+    const float largest = gm_half_max(cm);
     for (int r = 0; r < 2; r++) {
         const uint64_t top = __ballot(cm == gm_half_max(cm));
         const uint32_t mine = lane < 32 ? (uint32_t)top : (uint32_t)(top >> 32);
         if (__builtin_ctz(mine) >> 1 == (lane & 31) >> 1) cm = -1.0f;
     }
     const float third = gm_half_max(cm);
-    return third > 0.0f ? 16384.0f * third : INFINITY;
+    ref = third > 0.0f ? third : least;
+    return third > 0.0f || largest <= 16384.0f * least ? 16384.0f * ref : 0.0f;
+}
+
+// Takes a super-block's outliers out of v (finite) and returns whether there were
+// any (uniform); larger: the lanes of the larger half, where it is beyond 2^14
+// times the other's ref.
+__device__ __forceinline__ bool gm_take_out(gm_f4 &v, bool &larger)
+{
+    float ref;
+    const float thr = gm_outlier_thr(v, ref);
+    bool mine = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (fabsf(v[i]) > thr) {
+            v[i] = 0.0f;
+            mine = true;
+        }
+    const float m = gm_half_max(gm_abs_max(v)), all = wave_max_dpp(m);
+    const float least = -wave_max_dpp(m > 0.0f ? -ref : -INFINITY); // (every lane takes part)
+    larger = m == all && all > 16384.0f * least;
+    return __ballot(mine) != 0;
 }
 
 // Where the pieces of a token's 256 columns go: as a row of a 32-token tile
@@ -118,9 +148,11 @@ constexpr int GM_TOK = 1024, GM_TOK_SUMS = 32; // bytes per token and super-bloc
 // fragments at xf(k), the sub-blocks' sums at xm(k) (Q4_K) and 2^-s at xp(k), for
 // the tokens k < count.  The tokens' steps interleave: one token after another
 // left each with the latency of a dozen dependent lane moves.
-// row(k): the token's row of its tile (not TOK).
+// row(k): the token's row of its tile (not TOK).  halves: only the larger halves
+// that were left out without it (2^-s negative where there is one).
 template <int FMT, int R, bool TOK, class Row, class XF, class XM, class XP>
-__device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count, Row row, XF xf, XM xm, XP xp)
+__device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count, Row row, XF xf, XM xm, XP xp,
+                                              bool halves = false)
 {
     // this lane's group of eight columns: unit u, step st, half f
     const int c8 = lane >> 1;
@@ -146,8 +178,9 @@ __device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count
         if (sm[k] != sm[k]) mx[k] = INFINITY; // a NaN element (or Inf - Inf): the block is non-finite
     }
     // the maximum over the wavefront and the smallest maximum of its 32-column
-    // groups: within 2^14 of each other, no element is an outlier (the two
-    // largest 8-column maxima sit in at most two groups of each 128)
+    // groups: within 2^14 of each other, nothing is taken out (the two largest
+    // 8-column maxima sit in at most two groups of each 128, so both halves'
+    // third is at least the smallest group's maximum)
 #define GM_STEP(C, ROWS)                                                                                               \
     _Pragma("unroll") for (int k = 0; k < R; k++) mx[k] = st_max(mx[k], dpp_keep<C, ROWS>(__float_as_uint(mx[k])));
     GM_STEP(0xB1, 0xf)
@@ -172,25 +205,38 @@ __device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count
         sign[k] = 1.0f;
         odd = odd || !(mx[k] <= 16384.0f * mn[k]) || !(mx[k] < INFINITY);
     }
-    if (__builtin_expect(odd, 0)) { // uniform; rare
-#pragma unroll
+    if (__builtin_expect(odd || halves, 0)) { // uniform; rare, so one copy of the code for all tokens
+#pragma unroll 1
         for (int k = 0; k < R; k++) {
-            if (!(mx[k] < INFINITY)) {
-                v[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
-                mx[k] = sm[k] = 0.0f;
-                sign[k] = __builtin_nanf("");
-            } else if (mx[k] > 16384.0f * mn[k]) {
-                const float thr = gm_outlier_thr(v[k]);
-                bool mine = false;
+            gm_f4 w = v[0];
+            float m = mx[0], least = mn[0], sum = sm[0], sg = 1.0f;
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (fabsf(v[k][i]) > thr) {
-                        v[k][i] = 0.0f;
-                        mine = true;
-                    }
-                if (__ballot(mine) != 0) sign[k] = -1.0f;
-                mx[k] = wave_max_dpp(gm_abs_max(v[k]));
-                sm[k] = (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+            for (int i = 1; i < R; i++) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) w[q] = k == i ? v[i][q] : w[q];
+                m = k == i ? mx[i] : m;
+                least = k == i ? mn[i] : least;
+                sum = k == i ? sm[i] : sum;
+            }
+            if (!(m < INFINITY)) {
+                w = gm_f4{0.f, 0.f, 0.f, 0.f};
+                m = sum = 0.0f;
+                sg = __builtin_nanf("");
+            } else if (halves || m > 16384.0f * least) {
+                bool larger;
+                const bool outliers = gm_take_out(w, larger);
+                if ((outliers && !halves) || __ballot(larger) != 0) sg = -1.0f;
+                if (larger != halves) w = gm_f4{0.f, 0.f, 0.f, 0.f};
+                m = wave_max_dpp(gm_abs_max(w));
+                sum = (w[0] + w[1]) + (w[2] + w[3]);
+            }
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[i][q] = k == i ? w[q] : v[i][q];
+                mx[i] = k == i ? m : mx[i];
+                sm[i] = k == i ? sum : sm[i];
+                sign[i] = k == i ? sg : sign[i];
             }
         }
     }
@@ -614,7 +660,8 @@ __device__ __forceinline__ void gm_add_outliers(gm_f16v (&acc)[2], const uint8_t
             if (256 * sb + 4 * lane < cols) v = *(const gm_f4 *)(xrow(t) + 256 * sb + 4 * lane);
             const float sm = (v[0] + v[1]) + (v[2] + v[3]);
             if (__ballot(!(gm_abs_max(v) < INFINITY) || sm != sm)) continue; // non-finite: every output is NaN already
-            const float thr = gm_outlier_thr(v);
+            float ref;
+            const float thr = gm_outlier_thr(v, ref);
             const bool mine = ((t >> 2) & 1) == lane >> 5;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -634,6 +681,103 @@ __device__ __forceinline__ void gm_add_outliers(gm_f16v (&acc)[2], const uint8_t
                 }
             }
         }
+}
+
+// acc += 2^-s (d S - 32 dmin M), Q6_K and Q8_0 without M (and Q8_0's scales, d,
+// are in S already): a super-block's sums S of the 32 tokens whose 2^-s is at p;
+// am: their sub-blocks' sums (Q4_K), wt: the weights after head().
+template <int FMT, class W>
+__device__ __forceinline__ void gm_fold(gm_f16v (&acc)[2], const gm_f16v (&S)[2], const W &wt, const float *p, int f,
+                                        gm_h8 am)
+{
+    float pt[16]; // 2^-s of this lane's tokens
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const gm_f4 v = *(const gm_f4 *)(p + 8 * k + 4 * f);
+#pragma unroll
+        for (int i = 0; i < 4; i++) pt[4 * k + i] = v[i];
+    }
+    const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if constexpr (FMT == FMT_Q4K) {
+            const float d = wt.scale(j), dm = wt.min_scale(j);
+            const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wt.mins(j), zero, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[j][i], dm * M[i]), acc[j][i]);
+        } else if constexpr (FMT == FMT_Q6K) {
+            const float d = wt.scale(j);
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), d * S[j][i], acc[j][i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), S[j][i], acc[j][i]);
+        }
+    }
+}
+
+// The larger halves that the staging left out of a tile's super-blocks sb0 .. sb1
+// - 1, found again by the same rule: staged by themselves and multiplied as the
+// rest were.  Rare, so without prefetching; the workgroup's four wavefronts call it
+// together.  head(sb), half(sb, i): load a super-block's, a half's weights into wt;
+// xf (four units), xm, xp: LDS of a staged tile.  With every other half of x 1e6
+// times its neighbour, 14336 x 4096 in Q4_K takes 111 us per call at 8 tokens and
+// 370 at 128, ordinary x 31 and 64 (by gm_add_outliers 2849 and 30415).  A scale
+// per half, folded in mid-block, took 44 and 72, but its registers cost k_gemm_few
+// 5 to 47 % on ordinary x, a second pass of k_gemm_few 10 to 20 %.
+template <int FMT, class W, class XRow, class Head, class Half>
+__device__ __forceinline__ void gm_add_halves(gm_f16v (&acc)[2], W &wt, int cols, XRow xrow, int nt, int sb0, int sb1,
+                                              Head head, Half half, uint8_t *xf, uint8_t *xm, float *xp)
+{
+    const int lane = threadIdx.x & 63, f = lane >> 5, wave = threadIdx.x >> 6;
+    constexpr int PARTS = W::PARTS;
+    const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int sb = sb0; sb < sb1; sb++) {
+        __syncthreads(); // the last tile's readers are done
+#pragma unroll 1
+        for (int t0 = wave; t0 < 32; t0 += 16) { // tokens t0 + 4 k; past nt zeros
+            gm_f4 v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] = gm_f4{0.f, 0.f, 0.f, 0.f};
+                if (t0 + 4 * k < nt && 256 * sb + 4 * lane < cols)
+                    v[k] = *(const gm_f4 *)(xrow(t0 + 4 * k) + 256 * sb + 4 * lane);
+            }
+            gm_stage_rows<FMT, 4, false>(
+                v, lane, 4, [&](int k) { return t0 + 4 * k; }, [&](int) { return xf; },
+                [&](int k) { return xm + 16 * (t0 + 4 * k); }, [&](int k) { return xp + t0 + 4 * k; }, true);
+        }
+        __syncthreads();
+        if (__ballot(xp[lane & 31] < 0.0f) == 0) continue; // uniform over the workgroup
+        head(sb);
+        gm_f16v S[2] = {zero, zero}, T[2] = {zero, zero}; // T: Q8_0, its scales applied
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            if (!(p & 1)) half(sb, p >> 1);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                __builtin_amdgcn_sched_barrier(0); // (no loads ahead: the registers are the kernels')
+                const gm_h8 hi = gm_frag_at(xf + p * GM_UNIT, lane, p, t, 0), lo = gm_frag_at(xf + p * GM_UNIT, lane, p, t, 1);
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    gm_h8 b[PARTS];
+                    wt.frag(p >> 1, p & 1, t, j, b);
+                    S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b[0], S[j], 0, 0, 0);
+                    if constexpr (PARTS == 2) S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[1], S[j], 0, 0, 0);
+                    S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[0], S[j], 0, 0, 0);
+                    if constexpr (FMT == FMT_Q80) {
+                        if (t & 1) {
+                            T[j] += wt.block_scale(p & 1, t >> 1, j) * S[j];
+                            S[j] = zero;
+                        }
+                    }
+                }
+            }
+        }
+        gm_fold<FMT>(acc, FMT == FMT_Q80 ? T : S, wt, xp, f, *(const gm_h8 *)(xm + (FMT == FMT_Q4K ? 16 * lane : 0)));
+    }
+    __syncthreads();
 }
 
 // A workgroup of four wavefronts owns 256 rows (64 per wavefront, two 32-row
@@ -667,8 +811,9 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
     const int r0 = 256 * rb, rend = min(rows, r0 + 256);
     const rsrc_t rs = make_rsrc(W + (size_t)r0 * stride, (uint32_t)((size_t)(rend - r0) * stride));
     constexpr int XW = 2 * MT; // 16-byte words of a unit's x per thread
-    __shared__ gm_u4 xs[2][MT * GM_UNIT / 16];
+    __shared__ gm_u4 xs[2][(MT > 2 ? MT : 2) * GM_UNIT / 16]; // (four units for gm_add_halves)
     __shared__ float ps[2][MT * 32];
+    __shared__ gm_u4 ms[FMT == FMT_Q4K ? GM_SUMS / 16 : 1]; // (gm_add_halves)
     // this workgroup's token tiles, MT * U units
     const rsrc_t rx = make_rsrc(x.f + (size_t)tt * MT * U * GM_UNIT, (uint32_t)((size_t)MT * U * GM_UNIT));
     const float *xp = x.p + ((size_t)(tt * MT + (int)(threadIdx.x >> 5)) * nb) * 32 + (threadIdx.x & 31);
@@ -704,7 +849,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
     __syncthreads();
     for (int sb = sb0; sb < sb1; sb++) {
         wt.head();
-        gm_h8 am[MT];
+        gm_h8 am[MT] = {};
         float pv = 0.0f;
 #pragma unroll
         for (int p = 0; p < 4; p++) {
@@ -779,37 +924,10 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
             if (p == 3 && (int)threadIdx.x < MT * 32) ps[sb & 1][threadIdx.x] = pv;
             __syncthreads();
         }
-        // out += 2^-s (d S - 32 dmin M), Q6_K without M, Q8_0 2^-s T
         taken |= __ballot(ps[sb & 1][lane & (32 * MT - 1)] < 0.0f);
 #pragma unroll
-        for (int m = 0; m < MT; m++) {
-            float pt[16]; // 2^-s of this lane's tokens
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const float4 v = *(const float4 *)(ps[sb & 1] + 32 * m + 8 * k + 4 * f);
-                pt[4 * k] = v.x;
-                pt[4 * k + 1] = v.y;
-                pt[4 * k + 2] = v.z;
-                pt[4 * k + 3] = v.w;
-            }
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                if constexpr (FMT == FMT_Q4K) {
-                    const float d = wt.scale(j), dm = wt.min_scale(j);
-                    const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[m], wt.mins(j), zero, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        acc[m][j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[m][j][i], dm * M[i]), acc[m][j][i]);
-                } else if constexpr (FMT == FMT_Q6K) {
-                    const float d = wt.scale(j);
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[m][j][i] = fmaf(fabsf(pt[i]), d * S[m][j][i], acc[m][j][i]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[m][j][i] = fmaf(fabsf(pt[i]), T[m][j][i], acc[m][j][i]);
-                }
-            }
-        }
+        for (int m = 0; m < MT; m++)
+            gm_fold<FMT>(acc[m], *(FMT == FMT_Q80 ? &T[FMT == FMT_Q80 ? m : 0] : &S[m]), wt, ps[sb & 1] + 32 * m, f, am[m]);
     }
     if (__builtin_expect(taken != 0, 0)) {
 #pragma unroll
@@ -818,6 +936,11 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
             gm_add_outliers<FMT>(
                 acc[m], r < rows ? W + (size_t)r * stride : nullptr, r + 32 < rows ? W + (size_t)(r + 32) * stride : nullptr,
                 cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1);
+            gm_add_halves<FMT>(
+                acc[m], wt, cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1,
+                [&](int sb) { wt.head_load(rs, sb), wt.head(); },
+                [&](int sb, int i) { wt.load(rs, 2 * sb + i, 0), wt.split(2 * sb + i, 0); }, (uint8_t *)xs, (uint8_t *)ms,
+                ps[0]);
         }
     }
     float *o = out + (size_t)sp * n * rows;
@@ -923,10 +1046,13 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
             }
 #pragma unroll
             for (int t = 0; t < 4; t++) {
+                // (Q6_K: the 16 addresses anew, not kept in registers that would spill)
+                int ln = lane;
+                if (FMT == FMT_Q6K) asm volatile("" : "+v"(ln));
                 const int i1 = 4 * p + t + (AHEAD ? 1 : 0);
                 if (i1 < 16) {
-                    ah[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, lane, i1 >> 2, i1 & 3, 0);
-                    al[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, lane, i1 >> 2, i1 & 3, 1);
+                    ah[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, ln, i1 >> 2, i1 & 3, 0);
+                    al[i1 & 1] = gm_frag_at(xb + (i1 >> 2) * GM_UNIT, ln, i1 >> 2, i1 & 3, 1);
                 }
                 gm_h8 b[2][PARTS];
 #pragma unroll
@@ -947,27 +1073,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
             }
         }
         taken |= __ballot(ps[cur][lane & 31] < 0.0f);
-        float pt[16];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const gm_f4 v = *(const gm_f4 *)(ps[cur] + 8 * k + 4 * f);
-#pragma unroll
-            for (int i = 0; i < 4; i++) pt[4 * k + i] = v[i];
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if constexpr (FMT == FMT_Q4K) {
-                const float d = wt.scale(j), dm = wt.min_scale(j);
-                const gm_h8 am = *(const gm_h8 *)((const uint8_t *)ms[cur] + 16 * lane);
-                const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wt.mins(j), zero, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[j][i], dm * M[i]), acc[j][i]);
-            } else {
-                const float d = wt.scale(j);
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), d * S[j][i], acc[j][i]);
-            }
-        }
+        gm_fold<FMT>(acc, S, wt, ps[cur], f, *(const gm_h8 *)((const uint8_t *)ms[cur] + (FMT == FMT_Q4K ? 16 * lane : 0)));
         if (sb + 1 < sb1) { // uniform
             store_x(cur ^ 1);
             load_x(min(sb + 2, sb1 - 1));
@@ -975,6 +1081,11 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
         }
     }
     if (__builtin_expect(taken != 0, 0)) {
+        gm_add_halves<FMT>(
+            acc, wt, cols, [&](int t) { return x + (size_t)t * cols; }, n, sb0, sb1,
+            [&](int sb) { wt.head_load(rs, sb), wt.head(); },
+            [&](int sb, int i) { wt.load(rs, 2 * sb + i, i), wt.split(2 * sb + i, i); }, (uint8_t *)xs[0],
+            (uint8_t *)ms[0], ps[0]);
         const int r = r0 + 64 * wave + nl;
         gm_add_outliers<FMT>(
             acc, r < rows ? W + (size_t)r * stride : nullptr, r + 32 < rows ? W + (size_t)(r + 32) * stride : nullptr,
@@ -1222,21 +1333,7 @@ __global__ void __launch_bounds__(256, 2)
             }
         }
         taken |= __ballot(ps[cur][lane & 31] < 0.0f);
-        float pt[16];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const gm_f4 v = *(const gm_f4 *)(ps[cur] + 8 * k + 4 * f);
-#pragma unroll
-            for (int i = 0; i < 4; i++) pt[4 * k + i] = v[i];
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const float d = wt.scale(j), dm = wt.min_scale(j);
-            const gm_h8 am = *(const gm_h8 *)((const uint8_t *)ms[cur] + 16 * lane);
-            const gm_f16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wt.mins(j), zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[j][i] = fmaf(fabsf(pt[i]), fmaf(d, S[j][i], dm * M[i]), acc[j][i]);
-        }
+        gm_fold<FMT_Q4K>(acc, S, wt, ps[cur], f, *(const gm_h8 *)((const uint8_t *)ms[cur] + 16 * lane));
         if (sb + 1 < nb) { // uniform
             store_x(cur ^ 1);
             load_x(min(sb + 2, nb - 1));
@@ -1245,6 +1342,10 @@ __global__ void __launch_bounds__(256, 2)
     }
     const int row = r0 + WROWS * wave + nl; // NMAT 2: of gate and up; NMAT 1: and row + 32
     if (__builtin_expect(taken != 0, 0)) {
+        gm_add_halves<FMT_Q4K>(
+            acc, wt, cols, [&](int t) { return xs + (size_t)(slot_s[t] / xdiv) * cols; }, n, 0, nb,
+            [&](int sb) { wt.head_load(rs, sb), wt.head(); },
+            [&](int sb, int i) { wt.load(rs, 2 * sb + i, i), wt.split(i); }, (uint8_t *)xb_s[0], (uint8_t *)ms[0], ps[0]);
         const int row1 = NMAT == 2 ? row : row + 32;
         gm_add_outliers<FMT_Q4K>(
             acc, row < rows ? rowA[e] + (size_t)row * stride : nullptr,

@@ -177,3 +177,51 @@ def test_matmul_f16_outliers_above_subnormals(gpu, orc, dtype, rows, cols, n):
     for t in (0, 1, n // 2, n - 1):
         e = orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t]))
         assert e < TOL, (t, e)
+
+
+HALVES = [(Q4K, 4200, 4096, 9), (Q4K, 14400, 4096, 70), (Q6K, 300, 4352, 9), (Q8, 1100, 4224, 33)]
+
+
+@pytest.mark.parametrize("dtype,rows,cols,n", HALVES)
+@pytest.mark.parametrize("ratio", [1e4, 1e6, 1e7, 1e9])
+def test_matmul_f16_halves_apart(gpu, orc, dtype, rows, cols, n, ratio):
+    """One 128-column half of a super-block `ratio` times the rest throughout,
+    zero weights under it: the other half, which shares its scale, must keep
+    its precision."""
+    nb = cols // 256
+    zc = np.array([c for c in range(256 * nb) if (c >> 7) % 2 == (c >> 8) % 2])
+    w = zero_columns(dtype, orc.synth(dtype, rows, cols, 215, n), rows, cols, zc)
+    xs = orc.normal(n * cols, 1.0, 216, n).reshape(n, cols)
+    for t in range(n):
+        h = 256 * (t % nb) + 128 * (t % nb % 2)
+        xs[t, h:h + 128] *= np.float32(ratio)
+    out = run(gpu, orc, dtype, rows, cols, xs, w, f"gemm.half.{dtype}.{ratio}")
+    for t in (0, 1, n // 2, n - 1):
+        e = orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t]))
+        assert e < TOL, (t, e)
+
+
+@pytest.mark.parametrize("dtype,rows,cols,n", HALVES)
+@pytest.mark.parametrize("ratio", [1e5, 1e7, 1e9])
+def test_matmul_f16_sparse_halves(gpu, orc, dtype, rows, cols, n, ratio):
+    """Halves of one or two elements, one of them `ratio` times the rest of the
+    super-block and under a zero weight: beside a full half (t % 3 = 0, 1), and
+    two such halves (2)."""
+    nb = cols // 256
+    zc = np.sort(np.concatenate([np.arange(5, 256 * nb, 256), np.arange(192, 256 * nb, 256)]))
+    w = zero_columns(dtype, orc.synth(dtype, rows, cols, 217, n), rows, cols, zc)
+    xs = orc.normal(n * cols, 1.0, 218, n).reshape(n, cols)
+    for t in range(n):
+        b = xs[t, :256 * nb].reshape(nb, 256)
+        if t % 3 < 2:
+            b[:, :128] = 0.0
+            b[:, 5] = ratio
+            b[:, 60] = t % 3
+        else:
+            b[:] = 0.0
+            b[:, 3::128] = 7.0
+            b[:, 192] = -ratio
+    out = run(gpu, orc, dtype, rows, cols, xs, w, f"gemm.sparse.{dtype}.{ratio}")
+    for t in (0, 1, 2, n - 1):
+        e = orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t]))
+        assert e < TOL, (t, e)

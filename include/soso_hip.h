@@ -223,7 +223,7 @@ int soso_hip_gdn_block(soso_hip *h, const float *hist, const float *conv, const 
                        size_t n_v, size_t d, size_t kernel, float eps);
 /* The same with every buffer in device memory, queued on the library's
  * stream (no synchronisation; capturable in a HIP graph once its scratch of
- * n * (C + n_k) floats has been grown by an earlier call). */
+ * n * (C + n_k) floats has been grown by an earlier call).  out may be z. */
 int soso_hip_gdn_block_dev(soso_hip *h, const float *hist, const float *conv, const float *z, const float *decay,
                            const float *beta, const float *norm, float *state, float *out, size_t n, size_t n_k,
                            size_t n_v, size_t d, size_t kernel, float eps);

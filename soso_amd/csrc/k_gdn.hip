@@ -16,7 +16,8 @@
 //   k_gdn_rec   the recurrence in eight workgroups per value head, the state
 //               in registers for the whole block, read once and written once;
 //               both sums of a token in one pass over the rows, then DPP adds
-//               across a column's lanes: no barrier per token
+//               across a column's lanes: no barrier per token; o takes v's place
+//               in u, so that out may be z's buffer
 //   k_gdn_norm  the norm and the gate, a wavefront per token and head
 //   k_gdn_rec_few  up to GDN_FEW tokens: a workgroup per head, norm and gate
 //               included (one launch less)
@@ -136,10 +137,10 @@ __device__ __forceinline__ void gdn_update(float (&S)[8], const float4 (&k)[2], 
 // groups 2 r and 2 r + 1 (whole rows of the state per load).  The groups' sums
 // meet in LDS, one barrier per token; every thread of a column adds them.
 __global__ void __launch_bounds__(1024) k_gdn_rec_few(const float *__restrict__ u, const float *__restrict__ kq,
-                                                      const float *__restrict__ z, const float *__restrict__ decay,
+                                                      const float *z, const float *__restrict__ decay,
                                                       const float *__restrict__ beta, const float *__restrict__ norm,
-                                                      float *__restrict__ state, float *__restrict__ out, int n, int n_k,
-                                                      int n_v, float eps)
+                                                      float *__restrict__ state, float *out, int n, int n_k, int n_v,
+                                                      float eps)
 {
     constexpr int D = GDN_D;
     __shared__ float qk[GDN_FEW][2 * D];
@@ -204,10 +205,9 @@ __global__ void __launch_bounds__(1024) k_gdn_rec_few(const float *__restrict__ 
 // Bound by the chain of one token's instructions (about 70, 0.15 us): 256 tokens
 // of 16 q/k and 32 value heads took 385 us per call on MI355X with a workgroup
 // and four barriers per token and head, 55 us now; 64 tokens 86.8 -> 19.8.
-__global__ void __launch_bounds__(256) k_gdn_rec(const float *__restrict__ u, const float *__restrict__ kq,
+__global__ void __launch_bounds__(256) k_gdn_rec(float *__restrict__ u, const float *__restrict__ kq,
                                                  const float *__restrict__ decay, const float *__restrict__ beta,
-                                                 float *__restrict__ state, float *__restrict__ out, int n, int n_k,
-                                                 int n_v)
+                                                 float *__restrict__ state, int n, int n_k, int n_v)
 {
     constexpr int D = GDN_D, COLS = 16, NT = 256, TC = GDN_CHUNK, KQ = TC * 2 * D / 4 / NT, VW = TC * COLS / NT;
     __shared__ float qk[2][TC][2 * D];
@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(256) k_gdn_rec(const float *__restrict__ u, co
     __shared__ float os[TC][COLS];
     const int vh = (int)blockIdx.x % n_v, c0 = (int)blockIdx.x / n_v * COLS, kh = vh % n_k;
     const int tid = threadIdx.x, cl = tid >> 4, rg = tid & 15; // column of the workgroup, row group
-    const int qd = n_k * D, C = 2 * qd + n_v * D, vd = n_v * D;
+    const int qd = n_k * D, C = 2 * qd + n_v * D;
     float *st = state + (size_t)vh * D * D + c0 + cl;
     float S[8];
 #pragma unroll
@@ -297,7 +297,8 @@ __global__ void __launch_bounds__(256) k_gdn_rec(const float *__restrict__ u, co
         __syncthreads(); // the chunk's outputs, and the next chunk, are in LDS
         for (int w = tid; w < m * (COLS / 4); w += NT) {
             const int tt = w / (COLS / 4), c = w % (COLS / 4) * 4;
-            *(float4 *)(out + (size_t)(t0 + tt) * vd + vh * D + c0 + c) = *(const float4 *)&os[tt][c];
+            // in v's place: this workgroup alone reads it, and has
+            *(float4 *)(u + (size_t)(t0 + tt) * C + 2 * qd + vh * D + c0 + c) = *(const float4 *)&os[tt][c];
         }
         __syncthreads(); // os is rewritten by the next chunk
         b ^= 1;
@@ -306,15 +307,17 @@ __global__ void __launch_bounds__(256) k_gdn_rec(const float *__restrict__ u, co
     for (int i = 0; i < 8; i++) st[(size_t)(64 * (i >> 2) + 4 * rg + (i & 3)) * D] = S[i];
 }
 
-// Wavefront per (token, value head), in place.
-__global__ void __launch_bounds__(256) k_gdn_norm(float *__restrict__ out, const float *__restrict__ z,
-                                                  const float *__restrict__ norm, long heads, float eps)
+// Wavefront per (token, value head): o from u to out (which may be z).
+__global__ void __launch_bounds__(256) k_gdn_norm(const float *__restrict__ u, const float *z,
+                                                  const float *__restrict__ norm, float *out, unsigned heads, unsigned n_k,
+                                                  unsigned n_v, float eps)
 {
     const int lane = threadIdx.x & 63;
-    const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const unsigned w = blockIdx.x * 4 + (threadIdx.x >> 6), t = w / n_v; // below 65536^2 (gdn_unsupported)
     if (w >= heads) return;
-    const size_t o = (size_t)w * GDN_D + 2 * lane;
-    *(float2 *)(out + o) = gdn_norm2(*(const float2 *)(out + o), *(const float2 *)(z + o), norm, lane, eps);
+    const size_t o = (size_t)w * GDN_D + 2 * lane, C = (size_t)(2 * n_k + n_v) * GDN_D;
+    const float2 x = *(const float2 *)(u + t * C + (2 * n_k + (w - t * n_v)) * GDN_D + 2 * lane);
+    *(float2 *)(out + o) = gdn_norm2(x, *(const float2 *)(z + o), norm, lane, eps);
 }
 
 const char *gdn_unsupported(size_t n, size_t n_k, size_t n_v, size_t d, size_t kernel)
@@ -348,10 +351,11 @@ int launch_gdn_block(soso_hip *h, const float *hist, const float *conv, const fl
         k_gdn_rec_few<<<(unsigned)n_v, 1024, 0, h->stream>>>(u, kq, z, decay, beta, norm, state, out, n, n_k, n_v, eps);
         return hip_check(h, hipGetLastError(), "gdn recurrence launch");
     }
-    k_gdn_rec<<<(unsigned)n_v * (GDN_D / 16), 256, 0, h->stream>>>(u, kq, decay, beta, state, out, n, n_k, n_v);
+    k_gdn_rec<<<(unsigned)n_v * (GDN_D / 16), 256, 0, h->stream>>>(u, kq, decay, beta, state, n, n_k, n_v);
     rc = hip_check(h, hipGetLastError(), "gdn recurrence launch");
     if (rc != SOSO_HIP_OK) return rc;
     const long heads = (long)n * n_v;
-    k_gdn_norm<<<(unsigned)((heads + 3) / 4), 256, 0, h->stream>>>(out, z, norm, heads, eps);
+    k_gdn_norm<<<(unsigned)((heads + 3) / 4), 256, 0, h->stream>>>(u, z, norm, out, (unsigned)heads, (unsigned)n_k,
+                                                                  (unsigned)n_v, eps);
     return hip_check(h, hipGetLastError(), "gdn norm launch");
 }

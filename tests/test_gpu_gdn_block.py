@@ -67,3 +67,24 @@ def test_gdn_block_dev_pointers_off_by_a_float(gpu, orc, n):
     finally:
         for p in ptrs:
             gpu.dev_free(p)
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 33, 70])
+def test_gdn_block_dev_out_is_z(gpu, orc, n):
+    """The output may take z's buffer: the same bits as with one of its own."""
+    n_k, n_v, kernel = 2, 4, 4
+    bufs = make_block(orc, n, n_k, n_v, D, kernel, 780 + n)
+    st = bufs[6].copy()
+    out = gpu.gdn_block(*bufs[:6], st, n, n_k, n_v, D, kernel, EPS)
+    ptrs = []
+    try:
+        for b in bufs:
+            ptrs.append(gpu.dev_alloc(b.nbytes))
+            gpu.h2d(ptrs[-1], b)
+        assert gpu.gdn_block_dev(*ptrs, ptrs[2], n, n_k, n_v, D, kernel, EPS), gpu.last_error()
+        gpu.sync()
+        assert np.array_equal(gpu.d2h(ptrs[2], out.shape, np.float32), out)
+        assert np.array_equal(gpu.d2h(ptrs[6], st.shape, np.float32), st)
+    finally:
+        for p in ptrs:
+            gpu.dev_free(p)

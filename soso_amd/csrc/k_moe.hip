@@ -393,52 +393,59 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int32_t *__restrict__ i
                n_recs);
 }
 
-// Logits of many tokens: a workgroup per 16 tokens x 16 experts, its eight
-// wavefronts each taking every eighth 16-column step of the rows on the f32
-// matrix cores (v_mfma_f32_16x16x4_f32: lane l holds token or expert l % 16,
-// columns 4 (l / 16) .. of the step), the eight partial sums added in wavefront
-// order.  (k_moe_route's dot products took a wavefront per expert and four
-// tokens: 47 us with the ranking and the sort for 512 tokens x 128 experts x
-// 2048, against 21 with this, k_moe_rank and k_moe_sort.)
-typedef float moe_f4 __attribute__((ext_vector_type(4)));
-__global__ void __launch_bounds__(512) k_moe_logits(const float *__restrict__ W, const float *__restrict__ xs, int n,
+// Logits of many tokens, each the same sum, in the same order, as k_moe_route's
+// (so that a token's ranking does not depend on how many others its call has): a
+// wavefront per LOGITS_E experts and LOGITS_T tokens, lane l the columns 4 l .. 4
+// l + 3 of every 256, both sides' next 256 columns requested ahead of the products.
+// Workgroups go round the XCDs token tile by token tile, so an XCD reads x once.
+constexpr int LOGITS_E = 4, LOGITS_T = 8;
+__global__ void __launch_bounds__(256) k_moe_logits(const float *__restrict__ W, const float *__restrict__ xs, int n,
                                                     int hdim, int n_exp, float *__restrict__ logits)
 {
-    __shared__ float part[8][16][17];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    const int e = 16 * blockIdx.x + r, t = 16 * blockIdx.y + r;
-    const float *wr = W + (size_t)min(e, n_exp - 1) * hdim, *xr = xs + (size_t)min(t, n - 1) * hdim;
-    const int steps = (hdim + 15) / 16;
-    moe_f4 ac[4] = {}; // one chain per column of four
-    constexpr int Q = 16; // steps in flight
-    for (int i0 = wave; i0 < steps; i0 += 8 * Q) {
-        moe_f4 a[Q], b[Q];
+    constexpr int E = LOGITS_E, T = LOGITS_T;
+    const int lane = threadIdx.x & 63, nv = hdim >> 2;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int e0 = E * (4 * (int)blockIdx.y + wave), t0 = T * (int)blockIdx.x;
+    if (e0 >= n_exp) return; // no barriers here
+    const float4 *w4 = (const float4 *)W, *x4 = (const float4 *)xs;
+    float acc[E][T] = {};
+    float4 w[2][E], x[2][T];
+    auto load = [&](int b, int i0) {
+        const int i = i0 + lane;
 #pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const int c = 16 * (i0 + 8 * q) + 4 * g;
-            a[q] = b[q] = moe_f4{0.f, 0.f, 0.f, 0.f};
-            if (c < hdim) { // hdim is a multiple of four
-                a[q] = *(const moe_f4 *)(xr + c);
-                b[q] = *(const moe_f4 *)(wr + c);
+        for (int e = 0; e < E; e++)
+            w[b][e] = i < nv ? w4[(size_t)min(e0 + e, n_exp - 1) * nv + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            x[b][t] = i < nv ? x4[(size_t)min(t0 + t, n - 1) * nv + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    auto dot = [&](int b) {
+#pragma unroll
+        for (int e = 0; e < E; e++)
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                acc[e][t] = fmaf(w[b][e].x, x[b][t].x, acc[e][t]);
+                acc[e][t] = fmaf(w[b][e].y, x[b][t].y, acc[e][t]);
+                acc[e][t] = fmaf(w[b][e].z, x[b][t].z, acc[e][t]);
+                acc[e][t] = fmaf(w[b][e].w, x[b][t].w, acc[e][t]);
             }
+    };
+    load(0, 0);
+    for (int i0 = 0; i0 < nv; i0 += 128) { // (past the row's end: zeros)
+        load(1, i0 + 64);
+        __builtin_amdgcn_sched_barrier(0);
+        dot(0);
+        load(0, i0 + 128);
+        __builtin_amdgcn_sched_barrier(0);
+        dot(1);
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++)
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            const float sum = seg_sum_dpp<64>(acc[e][t]); // lane 63 holds it
+            if (lane == 63 && e0 + e < n_exp && t0 + t < n) logits[(size_t)(t0 + t) * n_exp + e0 + e] = sum;
         }
-#pragma unroll
-        for (int q = 0; q < Q; q++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) ac[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][k], b[q][k], ac[k], 0, 0, 0);
-    }
-    const moe_f4 acc = (ac[0] + ac[1]) + (ac[2] + ac[3]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) part[wave][4 * g + i][r] = acc[i]; // token 4 g + i, expert r
-    __syncthreads();
-    if (threadIdx.x < 256) {
-        const int tt = threadIdx.x >> 4, ee = threadIdx.x & 15;
-        float s = part[0][tt][ee];
-#pragma unroll
-        for (int w = 1; w < 8; w++) s += part[w][tt][ee];
-        if (16 * (int)blockIdx.y + tt < n && 16 * (int)blockIdx.x + ee < n_exp)
-            logits[(size_t)(16 * blockIdx.y + tt) * n_exp + 16 * blockIdx.x + ee] = s;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1203,8 +1210,8 @@ int launch_moe_route(soso_hip *h, const float *w, const float *x, size_t n, size
                                                         s.idx, s.wgt, s.cnt, s.offs, s.list, s.items, s.n_items,
                                                         moe_item_target(h), s.recs, s.n_recs, h->ticket);
     } else if (n >= ROUTE_MANY) {
-        const dim3 grid((unsigned)((n_exp + 15) / 16), (unsigned)((n + 15) / 16));
-        k_moe_logits<<<grid, 512, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, s.logits);
+        const dim3 grid((unsigned)((n + LOGITS_T - 1) / LOGITS_T), (unsigned)((n_exp + 4 * LOGITS_E - 1) / (4 * LOGITS_E)));
+        k_moe_logits<<<grid, 256, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, s.logits);
         k_moe_rank<<<(unsigned)((n + 3) / 4), 256, 0, h->stream>>>(s.logits, (int)n, (int)n_exp, (int)top_k, s.idx,
                                                                   s.wgt);
         if (sort)

@@ -113,6 +113,27 @@ def test_router_topk_many_tokens(gpu, orc, n_exp, h, top_k, n):
         assert orc.rel_l2(wgt[t], p[order] / p[order].sum()) < 4e-6, t
 
 
+@pytest.mark.parametrize("n_exp,h,top_k,n", [(128, 2048, 8, 520), (17, 68, 3, 163), (256, 260, 16, 160), (33, 4100, 5, 333)])
+def test_routing_does_not_depend_on_the_call(gpu, orc, n_exp, h, top_k, n):
+    """A token's experts and weights have the same bits whether it is routed
+    alone, with a few others or with many (also where a call ends in a smaller
+    block): a near-tie must not go another way."""
+    w = orc.normal(n_exp * h, 0.05, 343, n_exp)
+    xs = orc.normal(n * h, 1.0, 344, n).reshape(n, h)
+
+    def route(rows):
+        idx, wgt = np.full(len(rows) * top_k, -1, np.int32), np.zeros(len(rows) * top_k, np.float32)
+        assert gpu.router_topk(f"router.cut.{n_exp}.{h}", w, np.ascontiguousarray(rows).ravel(), len(rows), h, n_exp, top_k,
+                               idx, wgt), gpu.last_error()
+        return idx.reshape(-1, top_k), wgt.reshape(-1, top_k)
+
+    many = route(xs)
+    for t0, c in ((0, 1), (1, 8), (9, 33), (n - 3, 3), (n // 2, 1)):
+        few = route(xs[t0:t0 + c])
+        assert np.array_equal(many[0][t0:t0 + c], few[0]), t0
+        assert np.array_equal(many[1][t0:t0 + c].view(np.uint32), few[1].view(np.uint32)), t0
+
+
 def test_moe_many_tokens_outliers_above_subnormals(gpu, orc):
     """Tokens of a few ordinary elements among subnormal ones, 600 slots of six
     experts: the elements taken out must be added though 2^-s of the rest of

@@ -644,18 +644,36 @@ __device__ float gm_weight(const uint8_t *__restrict__ row, int c, int U)
     }
 }
 
+// Of a workgroup's super-blocks and tokens, those whose 2^-s is negative: 64 of
+// each in turn, so a set bit may stand for others too.  (With every super-block of
+// a tile looked at where one had a mark, @MARK@)
+struct GmTaken {
+    uint64_t blocks = 0, tokens = 0;
+    __device__ __forceinline__ void mark(int sb, float p)
+    {
+        const uint64_t t = __ballot(p < 0.0f);
+        tokens |= t;
+        blocks |= (uint64_t)(t != 0) << (sb & 63);
+    }
+    __device__ __forceinline__ bool any() const { return blocks != 0; }
+    __device__ __forceinline__ bool block(int sb) const { return (blocks >> (sb & 63)) & 1; }
+    __device__ __forceinline__ bool has(int sb, int t) const { return block(sb) && ((tokens >> t) & 1); }
+};
+
 // The products of the elements that the staging took out of a tile's tokens 0
 // .. nt - 1 (x rows xrow(t)) in super-blocks sb0 .. sb1 - 1, found again by the
 // same rule, into the sums of this lane's two weight rows w0 and w1 (null: past
 // the matrix).  Token t of the tile is register 4 (t / 8) + t % 4 of half t / 4
-// % 2.  Rare: kept out of the streaming loop.
+// % 2.  taken: which tokens and super-blocks to look at.  Rare: kept out of the
+// streaming loop.
 template <int FMT, class XRow>
 __device__ __forceinline__ void gm_add_outliers(gm_f16v (&acc)[2], const uint8_t *w0, const uint8_t *w1, int cols,
-                                                XRow xrow, int nt, int sb0, int sb1)
+                                                XRow xrow, int nt, int sb0, int sb1, const GmTaken &taken, int m)
 {
     const int lane = threadIdx.x & 63;
     for (int sb = sb0; sb < sb1; sb++)
         for (int t = 0; t < nt; t++) {
+            if (!taken.has(sb - sb0, 32 * m + t)) continue; // uniform
             gm_f4 v = {0.f, 0.f, 0.f, 0.f};
             if (256 * sb + 4 * lane < cols) v = *(const gm_f4 *)(xrow(t) + 256 * sb + 4 * lane);
             const float sm = (v[0] + v[1]) + (v[2] + v[3]);
@@ -727,13 +745,15 @@ __device__ __forceinline__ void gm_fold(gm_f16v (&acc)[2], const gm_f16v (&S)[2]
 // 5 to 47 % on ordinary x, a second pass of k_gemm_few 10 to 20 %.
 template <int FMT, class W, class XRow, class Head, class Half>
 __device__ __forceinline__ void gm_add_halves(gm_f16v (&acc)[2], W &wt, int cols, XRow xrow, int nt, int sb0, int sb1,
-                                              Head head, Half half, uint8_t *xf, uint8_t *xm, float *xp)
+                                              const GmTaken &taken, Head head, Half half, uint8_t *xf, uint8_t *xm,
+                                              float *xp)
 {
     const int lane = threadIdx.x & 63, f = lane >> 5, wave = threadIdx.x >> 6;
     constexpr int PARTS = W::PARTS;
     const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int sb = sb0; sb < sb1; sb++) {
+        if (!taken.block(sb - sb0)) continue; // uniform over the workgroup
         __syncthreads(); // the last tile's readers are done
 #pragma unroll 1
         for (int t0 = wave; t0 < 32; t0 += 16) { // tokens t0 + 4 k; past nt zeros
@@ -841,7 +861,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
     };
     // Q8_0: the super-block's sums, each block's scale applied
     gm_f16v T[FMT == FMT_Q80 ? MT : 1][2];
-    uint64_t taken = 0; // whether a token of the tiles had outliers
+    GmTaken taken;
     load_x(4 * sb0);
     wt.head_load(rs, sb0);
     wt.load(rs, 2 * sb0, 0);
@@ -924,20 +944,20 @@ __global__ void __launch_bounds__(256, 2) k_gemm(const uint8_t *__restrict__ W, 
             if (p == 3 && (int)threadIdx.x < MT * 32) ps[sb & 1][threadIdx.x] = pv;
             __syncthreads();
         }
-        taken |= __ballot(ps[sb & 1][lane & (32 * MT - 1)] < 0.0f);
+        taken.mark(sb - sb0, ps[sb & 1][lane & (32 * MT - 1)]);
 #pragma unroll
         for (int m = 0; m < MT; m++)
             gm_fold<FMT>(acc[m], *(FMT == FMT_Q80 ? &T[FMT == FMT_Q80 ? m : 0] : &S[m]), wt, ps[sb & 1] + 32 * m, f, am[m]);
     }
-    if (__builtin_expect(taken != 0, 0)) {
+    if (__builtin_expect(taken.any(), 0)) {
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             const int t0 = 32 * (tt * MT + m), r = r0 + 64 * wave + nl;
             gm_add_outliers<FMT>(
                 acc[m], r < rows ? W + (size_t)r * stride : nullptr, r + 32 < rows ? W + (size_t)(r + 32) * stride : nullptr,
-                cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1);
+                cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1, taken, m);
             gm_add_halves<FMT>(
-                acc[m], wt, cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1,
+                acc[m], wt, cols, [&](int t) { return xs32 + (size_t)(t0 + t) * cols; }, min(32, n - t0), sb0, sb1, taken,
                 [&](int sb) { wt.head_load(rs, sb), wt.head(); },
                 [&](int sb, int i) { wt.load(rs, 2 * sb + i, 0), wt.split(2 * sb + i, 0); }, (uint8_t *)xs, (uint8_t *)ms,
                 ps[0]);
@@ -1026,7 +1046,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
     gm_f16v acc[2], S[2];
     const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     acc[0] = acc[1] = zero;
-    uint64_t taken = 0;
+    GmTaken taken;
     for (int sb = sb0; sb < sb1; sb++) {
         const int cur = (sb - sb0) & 1, sn = min(sb + 1, sb1 - 1);
         wt.head();
@@ -1072,7 +1092,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
                     S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[j][0], S[j], 0, 0, 0);
             }
         }
-        taken |= __ballot(ps[cur][lane & 31] < 0.0f);
+        taken.mark(sb - sb0, ps[cur][lane & 31]);
         gm_fold<FMT>(acc, S, wt, ps[cur], f, *(const gm_h8 *)((const uint8_t *)ms[cur] + (FMT == FMT_Q4K ? 16 * lane : 0)));
         if (sb + 1 < sb1) { // uniform
             store_x(cur ^ 1);
@@ -1080,16 +1100,16 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
             __syncthreads();
         }
     }
-    if (__builtin_expect(taken != 0, 0)) {
+    if (__builtin_expect(taken.any(), 0)) {
         gm_add_halves<FMT>(
-            acc, wt, cols, [&](int t) { return x + (size_t)t * cols; }, n, sb0, sb1,
+            acc, wt, cols, [&](int t) { return x + (size_t)t * cols; }, n, sb0, sb1, taken,
             [&](int sb) { wt.head_load(rs, sb), wt.head(); },
             [&](int sb, int i) { wt.load(rs, 2 * sb + i, i), wt.split(2 * sb + i, i); }, (uint8_t *)xs[0],
             (uint8_t *)ms[0], ps[0]);
         const int r = r0 + 64 * wave + nl;
         gm_add_outliers<FMT>(
             acc, r < rows ? W + (size_t)r * stride : nullptr, r + 32 < rows ? W + (size_t)(r + 32) * stride : nullptr,
-            cols, [&](int t) { return x + (size_t)t * cols; }, n, sb0, sb1);
+            cols, [&](int t) { return x + (size_t)t * cols; }, n, sb0, sb1, taken, 0);
     }
     float *o = out + ((size_t)sp * n_all + 32 * tt) * rows;
 #pragma unroll
@@ -1295,7 +1315,7 @@ __global__ void __launch_bounds__(256, 2)
     gm_f16v acc[2], S[2];
     const gm_f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     acc[0] = acc[1] = zero;
-    uint64_t taken = 0;
+    GmTaken taken;
     for (int sb = 0; sb < nb; sb++) {
         const int cur = sb & 1, sn = min(sb + 1, nb - 1);
         wt.head();
@@ -1332,7 +1352,7 @@ __global__ void __launch_bounds__(256, 2)
                     S[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[j][0], S[j], 0, 0, 0);
             }
         }
-        taken |= __ballot(ps[cur][lane & 31] < 0.0f);
+        taken.mark(sb, ps[cur][lane & 31]);
         gm_fold<FMT_Q4K>(acc, S, wt, ps[cur], f, *(const gm_h8 *)((const uint8_t *)ms[cur] + 16 * lane));
         if (sb + 1 < nb) { // uniform
             store_x(cur ^ 1);
@@ -1341,16 +1361,16 @@ __global__ void __launch_bounds__(256, 2)
         }
     }
     const int row = r0 + WROWS * wave + nl; // NMAT 2: of gate and up; NMAT 1: and row + 32
-    if (__builtin_expect(taken != 0, 0)) {
+    if (__builtin_expect(taken.any(), 0)) {
         gm_add_halves<FMT_Q4K>(
-            acc, wt, cols, [&](int t) { return xs + (size_t)(slot_s[t] / xdiv) * cols; }, n, 0, nb,
+            acc, wt, cols, [&](int t) { return xs + (size_t)(slot_s[t] / xdiv) * cols; }, n, 0, nb, taken,
             [&](int sb) { wt.head_load(rs, sb), wt.head(); },
             [&](int sb, int i) { wt.load(rs, 2 * sb + i, i), wt.split(i); }, (uint8_t *)xb_s[0], (uint8_t *)ms[0], ps[0]);
         const int row1 = NMAT == 2 ? row : row + 32;
         gm_add_outliers<FMT_Q4K>(
             acc, row < rows ? rowA[e] + (size_t)row * stride : nullptr,
             row1 < rows ? (NMAT == 2 ? rowB : rowA)[e] + (size_t)row1 * stride : nullptr, cols,
-            [&](int t) { return xs + (size_t)(slot_s[t] / xdiv) * cols; }, n, 0, nb);
+            [&](int t) { return xs + (size_t)(slot_s[t] / xdiv) * cols; }, n, 0, nb, taken, 0);
     }
 #pragma unroll
     for (int i = 0; i < 16; i++) {

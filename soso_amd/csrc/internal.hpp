@@ -316,7 +316,7 @@ int launch_tile_q4k(soso_hip *h, const void *src_dev, void *dst_dev, size_t rows
 int launch_mfma_matmul(soso_hip *h, const Weight &w, const float *x, size_t n, float *y);
 // (k_gemm.hip) -- several tokens per row on the f16 matrix cores: whether they
 // are the faster ones for a shape, and their launch (DECLINED: no scratch)
-bool gemm_wins(uint8_t dtype, size_t rows, size_t cols, size_t n);
+bool gemm_wins(const soso_hip *h, uint8_t dtype, size_t rows, size_t cols, size_t n);
 int launch_gemm(soso_hip *h, const Weight &w, const float *x, size_t n, float *y);
 int launch_gemm_moe(soso_hip *h, int nmat, const uint8_t *const *tiled, const uint8_t *const *row_major, size_t n_groups,
                     size_t rows, size_t cols, size_t slots, size_t max_recs, const float *xs, size_t n, int xdiv,

@@ -645,8 +645,10 @@ __device__ float gm_weight(const uint8_t *__restrict__ row, int c, int U)
 }
 
 // Of a workgroup's super-blocks and tokens, those whose 2^-s is negative: 64 of
-// each in turn, so a set bit may stand for others too.  (With every super-block of
-// a tile looked at where one had a mark, @MARK@)
+// each in turn, so a set bit may stand for others too.  (Every super-block and token
+// of a tile looked at where one had a mark: MoE layers with heavy-tailed activations,
+// 16 experts of 1024 x 512 at 72 tokens 122 us against 71, 128 of 2048 x 768 at 512
+// tokens 338 against 256.)
 struct GmTaken {
     uint64_t blocks = 0, tokens = 0;
     __device__ __forceinline__ void mark(int sb, float p)
@@ -1422,25 +1424,36 @@ static bool gemm_shape_ok(uint8_t dtype, size_t rows, size_t cols)
 //    (Q6_K); at 3 small matrices lose (300 x 8192: 17 -> 20).  Q8_0 wins from
 //    6 (79 -> 58; at 4: 53 -> 59).
 //  * Q4_K up to 4096 columns: against the batched vector kernel (below 16
-//    tokens) from 8 tokens and 2^22 weights (14336 x 4096 36.5 -> 20.2, 2048 x
-//    2048 10.1 -> 9.8; 768 x 2048 8.8 -> 9.4), from 9 for smaller ones of 4096
-//    columns (100 x 4096 10.9 -> 10.0; at 8: 10.4 -> 10.2).  Against the integer
+//    tokens) from 8 tokens and 2^22 weights (14336 x 4096 36.5 -> 20.9, 2048 x
+//    2048 10.1 -> 9.8; 768 x 2048 8.8 -> 9.4), from 9 for smaller ones of 3584
+//    and more (300 x 3584 11.7 -> 10.4; at 8: 10.2 -> 10.2).  Against the integer
 //    matrix-core kernels, whose time is one chain along the columns, everywhere
-//    at 4096 columns (512 x 4096 at 16 tokens 15.9 -> 10.8, 1024 x 4096 at 64 /
-//    128 16.1 / 24.8 -> 13.8 / 16.6); with fewer columns past 2^24 weights at 17
+//    from 3584 columns (300 / 1024 / 4096 / 14336 rows at 16 tokens 13.9 / 14.0 /
+//    14.3 / 24.4 -> 10.8 / 11.2 / 13.0 / 20.9, at 64 14.4 / 14.6 / 24.9 / 58.4 ->
+//    12.4 / 13.7 / 20.3 / 36.6; at 3072 columns 14336 rows at 48 tokens 30.3 ->
+//    34.3, 300 at 33 11.5 -> 12.3); with fewer columns past 2^24 weights at 17
 //    to 32 tokens (14336 x 2048 at 16 / 20 / 32 / 48: 15.1 / 25.3 / 24.2 / 23.2
 //    -> 16.5 / 18.4 / 20.7 / 27.2), and past 64 tokens from 2.1e8 products at
 //    2048 columns (1024 x 2048 at 100: 14.1 -> 12.7; 100 x 2048 at 1000: 11.6 ->
 //    12.4), 8e8 below (14336 x 768 at 70 20.8 -> 17.5, 1000 x 1280 at 600 23.8 ->
 //    20.0; 1000 x 1024 at 700 18.2 -> 19.2, 8192 x 512 at 128 11.5 -> 13.4).
-//    Their form with x staged once (whole rounds of 16 tokens, whole 1024-column
-//    chunks, a full grid) holds out longer: 2048 x 2048 at 128 / 256 tokens 14.8 /
-//    24.8 -> 16.1 / 21.3, 4096 x 1024 at 256 / 400 / 512 16.6 / 28.3 / 29.9 ->
-//    21.2 / 22.1 / 23.9, 14336 x 1024 at 144 27.9 -> 30.7.
+//    Near these lines a call can be up to a tenth slower than it was: 14336 rows
+//    one or two tokens past 64, which the integer kernels take by themselves (x
+//    1536 at 65 / 66 29.4 / 27.6 -> 30.4 / 29.8), 1000 x 2304 at 70 11.8 -> 13.0.
+//    Whole rounds of 16 tokens go through the integer kernels in one pass while
+//    all their workgroups fit the GPU: four per CU up to 1024 columns (4096 x 768
+//    at 256 16.7 -> 22.3, 8192 x 768 at 128 16.5 -> 18.8, 2048 x 1024 at 400 19.0
+//    -> 21.1; past it 14336 x 768 at 80 28.5 -> 18.8), two below 2048 (4096 x 1536
+//    at 128 17.2 -> 20.8; at 144 28.2 -> 21.4), one up to 2816 and 256 tokens (2048 x 2304
+//    at 128 17.3 -> 21.2, 1000 x 2560 at 256 18.8 -> 20.8; 300 x 2304 at 512 20.8
+//    -> 18.3).  Their form with x staged once (whole 1024-column chunks, a full
+//    grid) holds out longer: 2048 x 2048 at 128 / 256 tokens 14.8 / 24.8 -> 16.1 /
+//    21.3, 4096 x 1024 at 400 / 512 28.3 / 29.9 -> 22.1 / 23.9, 14336 x 1024 at 144
+//    27.9 -> 30.7.
 //  * Q6_K up to 4096 columns: past 2^24 weights from 8 tokens (14336 x 4096
-//    41.7 -> 27.6); smaller ones from 48 tokens (1000 x 1024 38.9 -> 15.4),
-//    below which they keep the batched vector kernel and with it the bits of
-//    single matvecs.
+//    41.7 -> 27.6); smaller ones, 2^24 itself among them, from 48 tokens (1000 x
+//    1024 38.9 -> 15.4): not for the times, but because below that they keep the
+//    batched vector kernel and with it the bits of single matvecs.
 //  * Q8_0, whose four code planes cost its lines four visits: past 2^24 weights
 //    from 33 tokens (14336 x 4096 at 64: 97 -> 51; at 32: 51 -> 53), smaller ones
 //    from 16: always from 3072 columns (512 x 4096 24.1 -> 14.4, 1000 x 3072 18.9
@@ -1455,28 +1468,31 @@ static bool gemm_shape_ok(uint8_t dtype, size_t rows, size_t cols)
 //    multiple of 256 ran on the batched vector kernel: from 16 tokens (5000 x
 //    1440 26.3 -> 17.2), if 2^22 weights or 1024 columns (2014 x 768 at 149:
 //    15.6 -> 16.3).
-constexpr size_t MM_FULL = 205; // 64-row x 16-token workgroups that fill four fifths of 256 CUs
-bool gemm_wins(uint8_t dtype, size_t rows, size_t cols, size_t n)
+bool gemm_wins(const soso_hip *h, uint8_t dtype, size_t rows, size_t cols, size_t n)
 {
     if (n < 4 || n > (1u << 20) || !gemm_shape_ok(dtype, rows, cols)) return false;
-    const size_t weights = rows * cols, work = weights * n;
+    const size_t weights = rows * cols, work = weights * n, cu = (size_t)h->num_cu;
     const bool large = weights > (1u << 24), small = weights < (1u << 22);
+    // the integer kernels' workgroups (64 rows x 16 tokens) where every one has 16 tokens
+    const size_t wgs = (rows + 63) / 64 * (n / 16);
     if (dtype == SOSO_HIP_DTYPE_Q8_0) {
         if (cols > 4096) return n >= 6;
         if (cols % 256) return n >= 16 && (!small || cols >= 1024);
         if (n < (large ? 33 : 16)) return false;
-        if (n % 16 == 0 && cols % 1024 == 0 && (rows + 63) / 64 * (n / 16) >= MM_FULL)
-            return work >= (cols >= 2048 ? 1000000000u : 1500000000u);
+        if (n % 16 == 0 && cols % 1024 == 0 && wgs * 5 >= cu * 4) return work >= (cols >= 2048 ? 1000000000u : 1500000000u);
         return cols >= 3072 || work >= (cols >= 2048 ? 190000000u : cols >= 1024 ? 500000000u : 1000000000u);
     }
     if (cols > 4096) return true;
     if (dtype == SOSO_HIP_DTYPE_Q6_K) return n >= (large ? 8 : 48);
-    if (cols == 4096) return n >= (small ? 9 : 8);
+    if (cols >= 3584) return n >= (small ? 9 : 8);
     if (!small && n < 16) return n >= 8;
     if (n <= 64) return large && n > 16 && n <= 32;
-    if (n % 16 == 0 && cols % 1024 == 0) {
-        if (n <= (cols < 2048 ? 240 : 128)) return work >= 3000000000u;
-        if (cols < 2048 && (rows + 255) / 256 * (n / 16) >= MM_FULL) return work >= 1500000000u;
+    if (n % 16 == 0) {
+        if (wgs <= cu * (cols <= 1024 ? 4 : cols < 2048 ? 2 : cols > 2048 && cols < 3072 && n <= 256 ? 1 : 0)) return false;
+        if (cols % 1024 == 0) {
+            if (n <= (cols < 2048 ? 240 : 128)) return work >= 3000000000u;
+            if (cols < 2048 && (rows + 255) / 256 * (n / 16) * 5 >= cu * 4) return work >= 1500000000u;
+        }
     }
     return work >= (cols >= 2048 ? 210000000u : 800000000u);
 }

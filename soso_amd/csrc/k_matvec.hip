@@ -945,7 +945,7 @@ int launch_matvec(soso_hip *h, const Weight &w, const float *x, float *y, size_t
         if (rc != SOSO_HIP_OK) return rc;
         x = xp;
     }
-    if (gemm_wins(w.dtype, w.rows, kc, n)) {
+    if (gemm_wins(h, w.dtype, w.rows, kc, n)) {
         const int rc = launch_gemm(h, w, x, n, y);
         if (rc != SOSO_HIP_DECLINED) return rc;
     }

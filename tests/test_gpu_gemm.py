@@ -42,6 +42,10 @@ def run(gpu, orc, dtype, rows, cols, xs, w, key):
     (Q4K, 100, 4096, 9), (Q8, 100, 4096, 16), (Q8, 512, 3072, 17), (Q8, 300, 2048, 313), (Q4K, 300, 1536, 1751),
     # odd row and token counts whose product is no multiple of four, over several splits
     (Q4K, 4097, 4096, 17), (Q8, 1301, 6400, 19),
+    # Q4_K from 3584 columns, on both sides of the line and of its token counts
+    (Q4K, 1025, 3328, 16), (Q4K, 300, 3584, 9), (Q4K, 1025, 3584, 16), (Q4K, 1000, 3840, 33), (Q4K, 4097, 3840, 64),
+    # whole rounds of 16 tokens in one pass of the integer kernels, and one round past it
+    (Q4K, 4096, 1536, 128), (Q4K, 4096, 1536, 144), (Q4K, 2048, 2304, 128), (Q4K, 2048, 2304, 144),
 ])
 def test_matmul_f16_matrix_cores(gpu, orc, dtype, rows, cols, n):
     w = orc.synth(dtype, rows, cols, 201, rows + n)

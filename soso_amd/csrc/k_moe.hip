@@ -13,7 +13,8 @@
 //                 Calls whose experts scan the ranking themselves (at most 512
 //                 slots on the matrix cores) take the logits alone, then
 //                 k_moe_rank (softmax + top-k, one wavefront per token); from
-//                 ROUTE_MANY tokens on k_moe_logits, k_moe_rank, k_moe_sort.
+//                 ROUTE_MANY tokens and ROUTE_LOGITS logits on k_moe_logits,
+//                 k_moe_rank, k_moe_sort.
 //   k_moe_rows    workgroups over (expert, row chunk) items of equal work:
 //                 every weight row of an expert is read once from HBM and
 //                 applied to all the tokens routed to it (their x staged in
@@ -1193,11 +1194,13 @@ size_t moe_scratch_fixed(const soso_hip *h, size_t n, size_t n_groups, size_t to
     return need;
 }
 
-// Tokens from which the route runs as three launches (matrix-core logits, the
-// ranking, the sort).  us per layer of 128 experts of 2048 x 768, one launch /
-// three: 128 tokens 125.8 / 126.7, 160 130.7 / 128.9, 200 136.9 / 132.1, 512
-// 215 / 191.
-constexpr size_t ROUTE_MANY = 160;
+// Tokens and (token, expert) logits from which the route runs as three launches
+// (the logits by k_moe_logits, the ranking, the sort).  us per layer, one launch /
+// three: 128 experts of 2048 x 768 at top-8 and 160 tokens 142.6 / 144.0, 200 151.9 /
+// 148.7, 512 235 / 215; 256 of 2048 x 512 at 160 168 / 161; 64 of 2048 x 768 at 256
+// 127.7 / 130.4, 512 184 / 178; 32 at 512 107.5 / 111.7; 16 of 1024 x 512 at 512 90.7 /
+// 93.9.
+constexpr size_t ROUTE_MANY = 160, ROUTE_LOGITS = 24576;
 
 int launch_moe_route(soso_hip *h, const float *w, const float *x, size_t n, size_t hdim, size_t n_exp, size_t top_k,
                      const MoeScratch &s, bool sort)
@@ -1209,7 +1212,7 @@ int launch_moe_route(soso_hip *h, const float *w, const float *x, size_t n, size
         k_moe_route<1, 8><<<grid, 512, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, (int)top_k, s.logits,
                                                         s.idx, s.wgt, s.cnt, s.offs, s.list, s.items, s.n_items,
                                                         moe_item_target(h), s.recs, s.n_recs, h->ticket);
-    } else if (n >= ROUTE_MANY) {
+    } else if (n >= ROUTE_MANY && n * n_exp >= ROUTE_LOGITS) {
         const dim3 grid((unsigned)((n + LOGITS_T - 1) / LOGITS_T), (unsigned)((n_exp + 4 * LOGITS_E - 1) / (4 * LOGITS_E)));
         k_moe_logits<<<grid, 256, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, s.logits);
         k_moe_rank<<<(unsigned)((n + 3) / 4), 256, 0, h->stream>>>(s.logits, (int)n, (int)n_exp, (int)top_k, s.idx,

@@ -1,7 +1,9 @@
 """MoE layers whose experts get enough tokens for the f16 matrix cores
-(k_gemm.hip's grouped kernel) and the route that serves them, at the edges:
-expert loads around a 32-slot tile, experts without tokens, row blocks that
-end early, the allocation-free entry's bits, non-finite tokens, outliers.
+(k_gemm.hip's grouped kernel: over 512 slots, six or more per active expert; of
+fewer slots the integer kernel that scans the ranking takes them, some cases here
+among them) and the route that serves them, at the edges: expert loads around a
+32-slot tile, experts without tokens, row blocks that end early, the
+allocation-free entry's bits, non-finite tokens, outliers.
 
 Tolerance: as the matmul's (x within 2^-23, exact products, f32 sums), twice
 over for the two products in a row, with the oracle's own f32 sums: 4e-6.
@@ -36,6 +38,9 @@ def moe_noalloc(gpu, layer, xs):
     (128, 256, 256, 8, 300),   # many experts, over 512 slots
     (200, 512, 256, 5, 260),   # more than 128 experts; 4.. slots each on average
     (32, 512, 256, 8, 700),    # two route blocks of at most 4096 slots
+    # over 512 slots: 65 per expert, one slot per token and super-block, three
+    # super-blocks, row blocks of 128 and 256 that end early, just over the line
+    (8, 512, 256, 2, 260), (16, 256, 256, 1, 520), (5, 768, 512, 3, 180), (6, 1280, 768, 3, 171),
 ])
 def test_moe_many_tokens_match_cpu(gpu, orc, n_exp, h, ffn, top_k, n):
     layer = Layer(orc, n_exp, h, ffn, top_k, 310 + n)
@@ -65,10 +70,11 @@ def test_moe_many_tokens_match_cpu(gpu, orc, n_exp, h, ffn, top_k, n):
         layer.drop(gpu)
 
 
-def test_moe_many_tokens_outliers_and_nonfinite(gpu, orc):
+@pytest.mark.parametrize("n", [64, 200])  # 192 slots (the integer kernel), 600 (the f16 one)
+def test_moe_many_tokens_outliers_and_nonfinite(gpu, orc, n):
     """Tokens with elements 1e6 times the rest keep to the CPU's result, a NaN
     token's outputs are NaN, and neither touches the others."""
-    n_exp, h, ffn, top_k, n = 6, 512, 256, 3, 64
+    n_exp, h, ffn, top_k = 6, 512, 256, 3
     layer = Layer(orc, n_exp, h, ffn, top_k, 330)
     xs = orc.normal(n * h, 1.0, 331, n).reshape(n, h)
     clean = xs.copy()
@@ -85,6 +91,35 @@ def test_moe_many_tokens_outliers_and_nonfinite(gpu, orc):
         ref, ci, _ = layer.cpu(orc, xs[3])
         assert np.array_equal(idx[3], ci)
         assert orc.rel_l2(out[3], ref) < TOL, orc.rel_l2(out[3], ref)
+        # the allocation-free entry: the same bits
+        bare = moe_noalloc(gpu, layer, xs.ravel())
+        assert np.isnan(bare[5]).all()
+        assert np.array_equal(np.delete(bare, 5, 0), np.delete(out, 5, 0))
+    finally:
+        layer.drop(gpu)
+
+
+def test_moe_many_tokens_intermediate_outliers(gpu, orc):
+    """Three rows of every expert's gate and up 2^11 times the others, so that
+    where their gate is positive the intermediate activations hold elements some
+    2^22 times the rest: down must add them, from staged x and without.
+
+    Few elements carry such a result, so a product's error (4e-7 of its terms'
+    size) meets gates that cancel to a tenth of that size: 2e-5."""
+    n_exp, h, ffn, top_k, n = 6, 512, 256, 3, 200
+    layer = Layer(orc, n_exp, h, ffn, top_k, 336)
+    for w in layer.gate + layer.up:
+        dm = w.reshape(ffn, h // 256, 144)[:, :, :4].view(np.float16)
+        dm[..., 0], dm[..., 1] = 2.0 ** -10, 2.0 ** -7
+        dm[[7, 40, 200]] *= np.float16(2.0 ** 11)
+    xs = orc.normal(n * h, 1.0, 337, n).reshape(n, h)
+    try:
+        layer.upload(gpu)
+        out = moe_dev(gpu, layer, xs.ravel())[0]
+        assert np.array_equal(moe_noalloc(gpu, layer, xs.ravel()), out)
+        for t in (0, 1, 2, n // 2, n - 1):
+            ref, _, _ = layer.cpu(orc, xs[t])
+            assert orc.rel_l2(out[t], ref) < 2e-5, (t, orc.rel_l2(out[t], ref))
     finally:
         layer.drop(gpu)
 
@@ -113,7 +148,10 @@ def test_router_topk_many_tokens(gpu, orc, n_exp, h, top_k, n):
         assert orc.rel_l2(wgt[t], p[order] / p[order].sum()) < 4e-6, t
 
 
-@pytest.mark.parametrize("n_exp,h,top_k,n", [(128, 2048, 8, 520), (17, 68, 3, 163), (256, 260, 16, 160), (33, 4100, 5, 333)])
+@pytest.mark.parametrize("n_exp,h,top_k,n", [
+    (128, 2048, 8, 520), (256, 260, 16, 160), (33, 4100, 5, 800), (131, 68, 3, 190),  # past ROUTE_LOGITS
+    (17, 68, 3, 163),
+])
 def test_routing_does_not_depend_on_the_call(gpu, orc, n_exp, h, top_k, n):
     """A token's experts and weights have the same bits whether it is routed
     alone, with a few others or with many (also where a call ends in a smaller

@@ -1035,13 +1035,9 @@ __global__ void __launch_bounds__(256, 2) k_gemm_few(const uint8_t *__restrict__
     };
     load_x(sb0);
     __builtin_amdgcn_sched_barrier(0);
-    // tokens past n stay zero in both buffers
-    for (int i = threadIdx.x; i < 2 * 4 * GM_UNIT / 16; i += 256)
-        if ((i & 31) >= n) (&xs[0][0])[i] = gm_u4{0u, 0u, 0u, 0u};
-    if (FMT == FMT_Q4K && threadIdx.x < 2 * SUMS / 16 && ((int)threadIdx.x & 31) >= n)
-        (&ms[0][0])[threadIdx.x] = gm_u4{0u, 0u, 0u, 0u};
-    if (threadIdx.x < 64) (&ps[0][0])[threadIdx.x] = 0.0f;
-    __syncthreads();
+    // (the products' rows of tokens past n are never stored, whatever their x; their
+    // 2^-s must not be a mark)
+    if (threadIdx.x < 64 && ((int)threadIdx.x & 31) >= n) (&ps[0][0])[threadIdx.x] = 0.0f;
     store_x(0);
     load_x(min(sb0 + 1, sb1 - 1));
     __syncthreads();
@@ -1243,13 +1239,8 @@ __global__ void __launch_bounds__(256, 2)
     __shared__ gm_u4 ms[2][GM_SUMS / 16];
     __shared__ float ps[2][32];
     if ((int)threadIdx.x < n) slot_s[threadIdx.x] = list[first + threadIdx.x];
-    if constexpr (!STAGED) {
-        // tokens past n stay zero in both buffers
-        for (int i = threadIdx.x; i < 2 * 4 * GM_UNIT / 16; i += 256)
-            if ((i & 31) >= n) (&xb_s[0][0])[i] = gm_u4{0u, 0u, 0u, 0u};
-        if (threadIdx.x < 2 * GM_SUMS / 16 && ((int)threadIdx.x & 31) >= n)
-            (&ms[0][0])[threadIdx.x] = gm_u4{0u, 0u, 0u, 0u};
-        if (threadIdx.x < 64) (&ps[0][0])[threadIdx.x] = 0.0f;
+    if constexpr (!STAGED) { // (as in k_gemm_few)
+        if (threadIdx.x < 64 && ((int)threadIdx.x & 31) >= n) (&ps[0][0])[threadIdx.x] = 0.0f;
     }
     __syncthreads();
     // STAGED: thread (token m, i): pieces 2 i and 2 i + 1 (of 16) of every unit;

@@ -1005,14 +1005,14 @@ def main():
             "us_kernel": round(ms_mm * 1e3, 3), "GB_s": round(b_mm / (ms_mm * 1e-3) / 1e9, 1),
             "frac_hbm": round(b_mm / (ms_mm * 1e-3) / 1e9 / PEAK_GBS, 4),
             "gemm_TFLOP_s": round(2 * mm_n * 14336 * 4096 / (ms_mm * 1e-3) / 1e12, 2), "tokens": mm_n,
-            "path": "int8 MFMA 16x16x64 (exact codes x 3 digit planes of x)"}
+            "path": "f16 MFMA 32x32x16 (codes x block scales, exact, by x in two f16 parts)"}
         ms_q8 = time_matmul(g, 4096, 4096, mm_n, 28, max(20, args.steps // 10), min(args.warmup, 10), dtype=Q8)
         b_q8 = algo_bytes(Q8, 4096, 4096) + (mm_n - 1) * 4096 * 8
         extra["q8_0_matmul_4096x4096_n64"] = {
             "us_kernel": round(ms_q8 * 1e3, 3), "GB_s": round(b_q8 / (ms_q8 * 1e-3) / 1e9, 1),
             "frac_hbm": round(b_q8 / (ms_q8 * 1e-3) / 1e9 / PEAK_GBS, 4),
             "gemm_TFLOP_s": round(2 * mm_n * 4096 * 4096 / (ms_q8 * 1e-3) / 1e12, 2), "tokens": mm_n,
-            "path": "int8 MFMA 16x16x32, one per 32-element block and 4-token tile"}
+            "path": "f16 MFMA 32x32x16 (codes, exact, by x in two f16 parts; block scales on the sums)"}
         for n in (1, 32):
             ms_m, b_m, u_m, _ = time_moe(g, n, max(40, args.steps // 10))
             extra[f"moe_qwen3_30b_a3b_batch{n}"] = {

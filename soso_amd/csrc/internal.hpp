@@ -132,8 +132,9 @@ struct HostMoe {
 
 constexpr size_t SOSO_TICKET_BYTES = 16384;
 // (token, rank) slots one route launch sorts in LDS; larger MoE calls run in
-// blocks of at most MOE_ROUTE_MAX_SLOTS / top_k tokens (a token's routing and
-// expert work do not depend on the other tokens of the call)
+// blocks of at most MOE_ROUTE_MAX_SLOTS / top_k tokens (a token's routing does not
+// depend on the other tokens of the call, to the bit; its experts' products do in
+// their last bits, as the kernels differ with a block's slots)
 constexpr int MOE_ROUTE_MAX_SLOTS = 4096;
 inline size_t moe_block_tokens(size_t top_k) { return top_k ? (size_t)MOE_ROUTE_MAX_SLOTS / top_k : 1; }
 

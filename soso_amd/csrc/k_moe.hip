@@ -21,7 +21,8 @@
 //                 LDS).  Gate and up rows are read side by side and leave as
 //                 silu(gate.x) * up.x; down rows leave as y[slot].  (Two or
 //                 more tokens per active expert: the matrix-core kernel of
-//                 k_mfma.hip instead, from six on that of k_gemm.hip.)
+//                 k_mfma.hip instead; over 512 slots, from six per expert on that
+//                 of k_gemm.hip.)
 //   k_moe_down_comb  up to 4 tokens: down and the weighted sum in one launch,
 //                 one wavefront per ranked expert.
 //   k_moe_combine out[t] = sum_j wgt[t,j] * y[t*top_k + j], j in ranking order.
@@ -1458,10 +1459,13 @@ static int launch_down_comb(soso_hip *h, const uint8_t *const *tab, size_t n_exp
 }
 
 // Slots per active expert from which a registered layer's Q4_K experts run on
-// the f16 matrix cores in 32-slot tiles (k_gemm.hip).  128 experts of 2048 x 768
+// the f16 matrix cores in 32-slot tiles (k_gemm.hip), in calls of more than 512
+// slots: up to 512 the integer kernel that scans the ranking takes them
+// (mfma_moe_scan_ok), however many slots an expert has.  128 experts of 2048 x 768
 // at top-8, us per layer on MI355X, before -> there: 65 tokens (4.1 slots per
-// expert) 109 -> 121, 128 162 -> 127, 512 466 -> 217; 16 experts of 1024 x 512
-// at 200 tokens 185 -> 56.
+// expert) 109 -> 121, 128 162 -> 127, 512 466 -> 213; 16 experts of 1024 x 512
+// at 200 tokens 185 -> 56.  (That layer at 40 / 64 tokens, 20 / 32 slots per expert
+// in the scanning form: 64 / 93 us, against 52 at 65 tokens here.)
 constexpr size_t MOE_GEMM_SLOTS = 6;
 
 int launch_moe_experts(soso_hip *h, const float *xs, size_t n, size_t hdim, size_t ffn, size_t top_k,

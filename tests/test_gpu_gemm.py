@@ -2,7 +2,8 @@
 gpu.rs:443-455): Q4_K, Q6_K and Q8_0 against x in two f16 parts, at the sizes
 where the tiles, splits and dispatch can go wrong.
 
-Tolerance: x is within 2^-23 per element, every product exact, and a result
+Tolerance: x is within 2^-23 of each element above 2^-16 of its block's largest
+(2^-39 of the largest below), every product exact, and a result
 takes one f32 rounding per 16 columns of a super-block and per super-block:
 about sqrt(33) * 2^-25 of the summed products' size, which the codes' offset
 (mean 7.5 of 0..15) makes up to three times the result's.  2e-6 covers both

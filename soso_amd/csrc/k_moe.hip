@@ -400,8 +400,9 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int32_t *__restrict__ i
 // wavefront per LOGITS_E experts and LOGITS_T tokens, lane l the columns 4 l .. 4
 // l + 3 of every 256, both sides' next 256 columns requested ahead of the products.
 // Workgroups go round the XCDs token tile by token tile, so an XCD reads x once.
-// 512 tokens x 128 experts x 2048: 14.3 us (4 x 4 per wavefront 16.2, 2 x 8 19.4, 8 x
-// 4 15.5; on the f32 matrix cores, which add in another order, 12.2).
+// 512 tokens x 128 experts x 2048: 13.3 us (with a branch per load and a store per
+// logit 14.3, and so 4 x 4 per wavefront 16.2, 2 x 8 19.4, 8 x 4 15.5; on the f32
+// matrix cores, which add in another order, 12.2).
 constexpr int LOGITS_E = 4, LOGITS_T = 8;
 __global__ void __launch_bounds__(256) k_moe_logits(const float *__restrict__ W, const float *__restrict__ xs, int n,
                                                     int hdim, int n_exp, float *__restrict__ logits)
@@ -411,17 +412,23 @@ __global__ void __launch_bounds__(256) k_moe_logits(const float *__restrict__ W,
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int e0 = E * (4 * (int)blockIdx.y + wave), t0 = T * (int)blockIdx.x;
     if (e0 >= n_exp) return; // no barriers here
-    const float4 *w4 = (const float4 *)W, *x4 = (const float4 *)xs;
+    // (lanes past a row's end ask past the buffers' and get zeros)
+    const uint32_t row = 16u * (uint32_t)nv;
+    const int ne = min(E, n_exp - e0), nt = min(T, n - t0);
+    const rsrc_t rw = make_rsrc((const uint8_t *)(W + (size_t)e0 * hdim), (uint32_t)ne * row);
+    const rsrc_t rx = make_rsrc((const uint8_t *)(xs + (size_t)t0 * hdim), (uint32_t)nt * row);
     float acc[E][T] = {};
     float4 w[2][E], x[2][T];
     auto load = [&](int b, int i0) {
-        const int i = i0 + lane;
+        const uint32_t c = i0 + lane < nv ? 16u * (uint32_t)(i0 + lane) : 0x80000000u;
 #pragma unroll
         for (int e = 0; e < E; e++)
-            w[b][e] = i < nv ? w4[(size_t)min(e0 + e, n_exp - 1) * nv + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            w[b][e] = __builtin_bit_cast(
+                float4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(c + (uint32_t)min(e, ne - 1) * row), 0, 0));
 #pragma unroll
         for (int t = 0; t < T; t++)
-            x[b][t] = i < nv ? x4[(size_t)min(t0 + t, n - 1) * nv + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            x[b][t] = __builtin_bit_cast(
+                float4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(c + (uint32_t)min(t, nt - 1) * row), 0, 0));
     };
     auto dot = [&](int b) {
 #pragma unroll
@@ -443,13 +450,16 @@ __global__ void __launch_bounds__(256) k_moe_logits(const float *__restrict__ W,
         __builtin_amdgcn_sched_barrier(0);
         dot(1);
     }
+    float mine = 0.0f; // lane E t + e: the pair's logit
 #pragma unroll
     for (int e = 0; e < E; e++)
 #pragma unroll
         for (int t = 0; t < T; t++) {
-            const float sum = seg_sum_dpp<64>(acc[e][t]); // lane 63 holds it
-            if (lane == 63 && e0 + e < n_exp && t0 + t < n) logits[(size_t)(t0 + t) * n_exp + e0 + e] = sum;
+            const int sum = __builtin_amdgcn_readlane(__float_as_int(seg_sum_dpp<64>(acc[e][t])), 63);
+            mine = lane == E * t + e ? __int_as_float(sum) : mine;
         }
+    const int e = lane % E, t = lane / E;
+    if (e < ne && t < nt) logits[(size_t)(t0 + t) * n_exp + e0 + e] = mine;
 }
 
 // ---------------------------------------------------------------------------
@@ -1215,7 +1225,7 @@ int launch_moe_route(soso_hip *h, const float *w, const float *x, size_t n, size
         k_moe_route<1, 8><<<grid, 512, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, (int)top_k, s.logits,
                                                         s.idx, s.wgt, s.cnt, s.offs, s.list, s.items, s.n_items,
                                                         moe_item_target(h), s.recs, s.n_recs, h->ticket);
-    } else if (n >= ROUTE_MANY && n * n_exp >= ROUTE_LOGITS) {
+    } else if (n >= ROUTE_MANY && n * n_exp >= ROUTE_LOGITS && hdim < ((size_t)1 << 24)) { // (k_moe_logits' 32-bit offsets)
         const dim3 grid((unsigned)((n + LOGITS_T - 1) / LOGITS_T), (unsigned)((n_exp + 4 * LOGITS_E - 1) / (4 * LOGITS_E)));
         k_moe_logits<<<grid, 256, 0, h->stream>>>(w, x, (int)n, (int)hdim, (int)n_exp, s.logits);
         k_moe_rank<<<(unsigned)((n + 3) / 4), 256, 0, h->stream>>>(s.logits, (int)n, (int)n_exp, (int)top_k, s.idx,

@@ -1,8 +1,7 @@
 """Benchmark of the decode hot path on one MI355X.
 
-Headline (BASELINE.json metric, configs[1]): single-token Q4_K matvec at the
-Llama FFN-up shape 14336 x 4096 in GB/s and as a fraction of the 8 TB/s HBM
-peak.  A "step" is one matvec over one resident weight; 16 weight copies
+Headline: single-token Q4_K matvec at the Llama FFN-up shape 14336 x 4096 in
+GB/s and as a fraction of the 8 TB/s HBM peak.  A "step" is one matvec over one resident weight; 16 weight copies
 (528 MB, above the 256 MB Infinity Cache) are rotated so HBM, not MALL,
 serves them.  Inputs are synthetic (seeded counter-based generator) and
 already resident in HBM when the timed region starts.
@@ -11,9 +10,8 @@ Prints ONE JSON line.  `value` and `roofline.achieved` are algorithmic bytes
 over the average launch duration, measured with HIP events on the library's
 stream around a graph of back-to-back launches; `cpu_baseline` times the
 AVX2 restatement of soso's CPU kernels (oracle/) on the host cores for a
-bounded sample.  Other configs of
-BASELINE.json are reported under "configs" (they are parity cases, not the
-headline).
+bounded sample.  Other workloads are reported under "configs" (they are parity
+cases, not the headline).
 """
 import argparse
 import json
@@ -321,7 +319,7 @@ def time_gdn(g, n, steps, layers=8, n_k=16, n_v=32, d=128, kernel=4, seed=41, ea
 
 
 def time_moe(g, n, steps, layers=4, n_x=8, seed=11, eager=False):
-    """configs[3]: Qwen3-30B-A3B-like MoE FFN (hidden 2048, 128 experts of
+    """Qwen3-30B-A3B-like MoE FFN (hidden 2048, 128 experts of
     intermediate 768, top-8, Q4_K experts, f32 router ~ N(0, 0.02)), `n`
     tokens ~ N(0, 1) per call, routing from the seeded inputs.  `layers`
     independent layers and `n_x` input batches are rotated so that successive
@@ -391,7 +389,7 @@ def time_moe(g, n, steps, layers=4, n_x=8, seed=11, eager=False):
 
 
 def time_decode_8b(g, steps, ctx=4096, seed=21, kv_f16=False, eager=False):
-    """one greedy decode step of a random-init Llama-style 8B
+    """One greedy decode step of a random-init Llama-style 8B
     (32 layers, hidden 4096, 32 q / 8 KV heads of 128, RoPE theta 5e5,
     SwiGLU 14336, RMSNorm eps 1e-5, Q4_K projections, Q6_K head over 128256)
     with an f32 KV cache prefilled with N(0, 1) to `ctx` positions (kv_f16:
@@ -683,7 +681,7 @@ def time_single_launch(g, dtype, rows, cols, reps=50, seed=1):
 
 
 def head_parity(g, threads, seed=1):
-    """configs[2] checked in the bench run: the Q6_K head 128256 x 4096 on the
+    """Checked in the bench run: the Q6_K head 128256 x 4096 on the
     GPU (matvec + argmax on the device) against the CPU restatement on the
     same seeded bytes (oracle/, `threads` host threads).  Returns the GPU and
     CPU argmax, the CPU logits' top-2 gap and the relative L2 of the logits."""
@@ -718,7 +716,7 @@ def head_parity(g, threads, seed=1):
 def cpu_extra(seconds, threads):
     """The rest of the CPU baseline (oracle/ restatements, bounded samples,
     every one rotating >= 512 MB): host DRAM read bandwidth (STREAM-like sum,
-    the CPU roofline), configs[0] Q8_0, and configs[2]'s head both ways soso
+    the CPU roofline), Q8_0 4096 x 4096, and the Q6_K head both ways soso
     could run it -- the restated Q6_K dequant+dot, and Q6_K requantized to
     Q8_0 (gguf2som/src/lib.rs:1592-1609) then AVX2 matvec_q8_0 -- on row
     samples.  GB/s are algorithmic bytes of the format the kernel reads."""
@@ -761,7 +759,7 @@ def cpu_extra(seconds, threads):
 
 
 def cpu_more_configs(seconds, threads, head_q8_ms):
-    """CPU baselines of configs[3] and configs[4] and of the 64-token matmul,
+    """CPU baselines of the MoE FFN, the 8B decode step and of the 64-token matmul,
     the oracle's restatements on the same host threads: the MoE FFN of one
     token (forward_moe_ffn's CPU branch, layer.rs:1938-2105) over 2 rotated
     layers of 128 Q4_K experts; one dense 8B decode layer at position 4096 of
@@ -921,7 +919,7 @@ def main():
                 res[f"gdn_block_n{n}_GB_s"] = round(nb / (ms * 1e-3) / 1e9, 1)
         elif args.only == "readprobe":
             nb = 14336 * ROW_BYTES[Q4K](4096)  # the headline's weight bytes
-            nq = 4096 * ROW_BYTES[Q8](4096)  # configs[0]'s Q8_0 weight bytes
+            nq = 4096 * ROW_BYTES[Q8](4096)  # the Q8_0 4096 x 4096 weight's bytes
             small = time_read_probe(g, nb, 16, MIN_TIMED // 2, 20)
             q8 = time_read_probe(g, nq, 28, MIN_TIMED // 2, 20)
             big = time_read_probe(g, 512 << 20, 2, 20, 4)
@@ -956,7 +954,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "q4_k",
-        "data": "synthetic (seeded counter-based generator, BASELINE configs[1] distributions)",
+        "data": "synthetic (seeded counter-based generator)",
         "config": {"workload": "Q4_K matvec 14336x4096, batch 1, 16 rotating resident copies (528 MB)",
                    "rows": rows, "cols": cols, "bytes_per_step": nbytes, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_GBS, "unit": "GB/s",

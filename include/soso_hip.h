@@ -244,7 +244,7 @@ int soso_hip_gdn_block_dev(soso_hip *h, const float *hist, const float *conv, co
  * elements, zeroed) and the step's buffers; drop_sources = 1 drops the q, k, v,
  * gate and up weights once fused.  RoPE is non-NeoX (pairs 2i, 2i+1) with
  * rope_theta.
- * kv_f16 = 0: the KV cache holds f32 (BASELINE configs[4]).  kv_f16 = 1: it holds
+ * kv_f16 = 0: the KV cache holds f32.  kv_f16 = 1: it holds
  * IEEE half bits, as soso's KvCache does (KvDtype::F16, kv.rs:258-266, the only
  * KV type soso's device decode accepts, runtime/decode_gpu.rs:63): new rows are
  * rounded with soso's f32_to_f16 (f16.rs:10-36: nearest, ties away from zero,

@@ -6,7 +6,7 @@
 // rope_cabezas (gemm.rs:1452-1490) -> KV append -> attention -> o-proj +
 // residual -> ffn_norm -> gate/up -> swiglu -> down + residual; then
 // Runtime::logits_gpu + argmax (crates/soso-llm-core/src/runtime.rs:1976-2028).
-// The KV cache holds f32 (configs[4]) or, as soso's KvCache (kv.rs:258-266),
+// The KV cache holds f32 or, as soso's KvCache (kv.rs:258-266),
 // f16 bits rounded with soso's f32_to_f16 (f16.rs:10-36).
 //
 // Launches per layer (every weight byte read once, activations stay in HBM):

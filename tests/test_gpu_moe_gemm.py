@@ -189,3 +189,32 @@ def test_moe_many_tokens_outliers_above_subnormals(gpu, orc):
                 assert orc.rel_l2(out[t], ref) < TOL, (name, t, orc.rel_l2(out[t], ref))
     finally:
         layer.drop(gpu)
+
+
+def test_moe_many_tokens_marks_in_long_rows(gpu, orc):
+    """Rows of 68 super-blocks, more than the 64 that marks are kept for: tokens
+    with a large element, and with one half 1e6 times the other, in super-blocks on
+    either side of that and in one whose place another shares, keep the CPU's result
+    and leave the others' bits."""
+    n_exp, h, ffn, top_k, n = 2, 17408, 256, 2, 260
+    layer = Layer(orc, n_exp, h, ffn, top_k, 338)
+    clean = orc.normal(n * h, 1.0, 339, n).reshape(n, h)
+    xs = clean.copy()
+    marked = (3, 40, 41, 259)
+    xs[3, 7] *= np.float32(1e6)                         # super-block 0
+    xs[40, 256 * 64 + 128:256 * 65] *= np.float32(1e6)  # 64, which shares 0's place
+    xs[41, 256 * 63 + 5] *= np.float32(1e6)
+    xs[259, 256 * 67:256 * 67 + 128] *= np.float32(1e6)
+    xs[259, 256 * 30 + 200] *= np.float32(1e6)
+    try:
+        layer.upload(gpu)
+        base = moe_dev(gpu, layer, clean.ravel())[0]
+        out, idx, _ = moe_dev(gpu, layer, xs.ravel())
+        same = [t for t in range(n) if t not in marked]
+        assert np.array_equal(out[same], base[same])
+        for t in marked:
+            ref, ci, _ = layer.cpu(orc, xs[t])
+            assert np.array_equal(idx[t], ci), t
+            assert orc.rel_l2(out[t], ref) < TOL, (t, orc.rel_l2(out[t], ref))
+    finally:
+        layer.drop(gpu)

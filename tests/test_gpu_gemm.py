@@ -59,7 +59,9 @@ def test_matmul_f16_matrix_cores(gpu, orc, dtype, rows, cols, n):
 
 
 @pytest.mark.parametrize("dtype,rows,cols,n", [(Q4K, 4200, 4096, 9), (Q4K, 14400, 4096, 70), (Q6K, 300, 4352, 9),
-                                               (Q6K, 1000, 1024, 1300), (Q8, 1100, 4224, 33)])
+                                               (Q6K, 1000, 1024, 1300), (Q8, 1100, 4224, 33),
+                                               (Q8, 333, 4160, 33), (Q8, 300, 4544, 40), (Q8, 300, 4128, 20),
+                                               (Q8, 300, 4256, 20)])
 @pytest.mark.parametrize("ratio", [1e4, 1e6, 1e9])
 def test_matmul_f16_outliers_under_zero_weights(gpu, orc, dtype, rows, cols, n, ratio):
     """Two elements of every 128 columns `ratio` times the rest, zero weights
@@ -169,7 +171,8 @@ def test_matmul_host_long_transfers(gpu, orc, rows, cols, n):
 
 
 @pytest.mark.parametrize("dtype,rows,cols,n", [(Q4K, 4200, 4096, 9), (Q4K, 14400, 4096, 70), (Q6K, 300, 4352, 9),
-                                               (Q6K, 4100, 4352, 130), (Q8, 1100, 4224, 33)])
+                                               (Q6K, 4100, 4352, 130), (Q8, 1100, 4224, 33), (Q8, 333, 4160, 33),
+                                               (Q8, 300, 4544, 40), (Q8, 300, 4128, 20), (Q8, 300, 4256, 20)])
 def test_matmul_f16_outliers_above_subnormals(gpu, orc, dtype, rows, cols, n):
     """Two elements of ordinary size in every 256, the others subnormal (what a
     SwiGLU that underflows leaves): the large ones are taken out of the scale,

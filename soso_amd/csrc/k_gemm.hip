@@ -227,6 +227,24 @@ __device__ __forceinline__ void gm_stage_rows(gm_f4 (&v)[R], int lane, int count
         sign[k] = 1.0f;
         odd = odd || !(mx[k] <= 16384.0f * mn[k]) || !(mx[k] < INFINITY);
     }
+    if (__builtin_expect(odd, 0) && !halves) {
+        // Zero groups alone call for nothing: where a half has three 8-column maxima
+        // above zero its third is at least the smallest of them.  (14336 x 4096 in Q4_K
+        // with a zero 32-column group per super-block, 8 / 32 tokens: 28.8 / 54.8 us
+        // through the code below, 22.2 / 31.3 with this.)
+        odd = false;
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            float c = gm_abs_max(v[k]);
+            c = fmaxf(c, dpp_f<0xB1>(c));
+            const uint64_t some = __ballot(c > 0.0f); // two lanes per maximum
+            const int n0 = __popc((uint32_t)some), n1 = __popc((uint32_t)(some >> 32));
+            const float least = -wave_max_dpp(c > 0.0f ? -c : -INFINITY);
+            const bool fine = mx[k] <= 16384.0f * least && mx[k] < INFINITY && (n0 == 0 || n0 >= 6) && (n1 == 0 || n1 >= 6);
+            mn[k] = fine ? mx[k] : 0.0f;
+            odd = odd || !fine;
+        }
+    }
     if (__builtin_expect(odd || halves, 0)) { // uniform; rare, so one copy of the code for all tokens
 #pragma unroll 1
         for (int k = 0; k < R; k++) {

@@ -233,3 +233,31 @@ def test_matmul_f16_sparse_halves(gpu, orc, dtype, rows, cols, n, ratio):
     for t in (0, 1, 2, n - 1):
         e = orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t]))
         assert e < TOL, (t, e)
+
+
+@pytest.mark.parametrize("dtype,rows,cols,n", HALVES)
+@pytest.mark.parametrize("ratio", [1.0, 1e4, 1e7])
+def test_matmul_f16_zero_groups(gpu, orc, dtype, rows, cols, n, ratio):
+    """Super-blocks with whole groups of zeros: a zero 32-column group (t % 4 = 0),
+    halves of three, two and one 8-column groups, one of whose elements is `ratio`
+    times the rest and under a zero weight (1, 2, 3): the rest keeps its precision."""
+    nb = cols // 256
+    zc = np.arange(5, 256 * nb, 256)
+    w = zero_columns(dtype, orc.synth(dtype, rows, cols, 221, n), rows, cols, zc)
+    xs = orc.normal(n * cols, 1.0, 222, n).reshape(n, cols)
+    for t in range(n):
+        b = xs[t, :256 * nb].reshape(nb, 256)
+        if t % 4 == 0:
+            b[:, 64:96] = 0.0
+        else:
+            keep = np.zeros(128, bool)
+            for c in (0, 40, 96)[:4 - t % 4]:
+                keep[c:c + 8] = True
+            b[:, :128][:, ~keep] = 0.0
+            if t % 4 == 3:
+                b[:, 128:] = 0.0
+        b[:, 5] *= np.float32(ratio)
+    out = run(gpu, orc, dtype, rows, cols, xs, w, f"gemm.zgroup.{dtype}.{ratio}")
+    for t in (0, 1, 2, 3, n - 1):
+        e = orc.rel_l2(out[t], orc.matvec_f64(dtype, w, rows, cols, xs[t]))
+        assert e < TOL, (t, e)
